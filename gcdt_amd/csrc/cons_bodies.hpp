@@ -176,9 +176,10 @@ __host__ __device__ inline unsigned long long cav_key(unsigned epoch, int piece)
 // Walk piece (a,b) from its wedge at a; calls f(tri) for each crossed
 // triangle.  Returns the crossed count, 0 if (a,b) already is an edge (marked
 // here when mark is set), -1 on error, -2 when it meets a constrained edge
-// and crossings are deferred (c.steiner).
+// and crossings are deferred (c.steiner), -3 when it crosses more than `most`
+// triangles (f has been called for the first `most`).
 template <class F>
-__host__ __device__ inline int cav_walk(const Cons& c, int a, int b, bool mark, int* t0out, F&& f)
+__host__ __device__ inline int cav_walk(const Cons& c, int a, int b, bool mark, int* t0out, F&& f, int most = 1 << 30)
 {
     const Mesh& m = c.m;
     int2 PA = m.pts[a], PB = m.pts[b];
@@ -206,6 +207,7 @@ __host__ __device__ inline int cav_walk(const Cons& c, int a, int b, bool mark, 
             return -1;
         }
         if (n < 0) return -1;
+        if (cnt >= most) return -3;
         f(n);
         cnt++;
         if (q == b) return cnt;
@@ -226,6 +228,26 @@ struct Win {
     int K;
     int off;  // scratch offset (ints)
 };
+
+// Cavities of more crossed triangles than this are walked, claimed and
+// retriangulated by a wave or a workgroup; shorter ones by one thread each.
+// One thread's walk is a chain of two dependent loads per triangle and its
+// Delaunay-vertex scans are quadratic; below about a dozen triangles a wave
+// per piece costs more than it saves (100,000 ring segments over 10M points
+// cross 2-6 triangles each).
+#ifndef GCDT_CAV_WAVE_K
+#define GCDT_CAV_WAVE_K 12
+#endif
+constexpr int CAV_WAVE_K = GCDT_CAV_WAVE_K;
+
+// Scratch of a cavity above CAV_WAVE_K: its crossed slots (K), the new owner of
+// each boundary edge (K + 2), and the arrays of cav_block_retri.
+__host__ __device__ inline long long cav_block_ints(int K) { return 9LL * K + 16; }
+
+// owner[] of a triangle of such a cavity once it is rewritten: above every key
+// of a later round (keys fall with the epoch), the low word the place of one
+// of its boundary edges, for cav_fix_block.
+__host__ __device__ inline unsigned long long cav_place(int p) { return 0xFFFFFFFF00000000ull | (unsigned)p; }
 
 // The Delaunay vertex of base (A, B) among the polygon vertices lo..hi-1
 // (coordinates in PX/PY): the one whose circle with A and B holds no other
@@ -251,15 +273,16 @@ struct DvScan {
 // R3 body: collect winner wi's cavity and retriangulate it in place.
 // Returns false (and flags MERR_CAVITY) on an inconsistent cavity.  DV finds
 // each Delaunay vertex (DvScan, or a wave-wide search whose lanes all run this
-// body for the same cavity).
+// body for the same cavity).  own: scratch of the caller's in place of
+// scr + w.off.
 template <class DV = DvScan>
 __host__ __device__ inline bool cav_retri_one(const Cons& c, const int2* pieces, const Win* wins, int wi, int* scr,
-                                              unsigned epoch)
+                                              unsigned epoch, int* own = nullptr)
 {
     const Mesh& m = c.m;
         Win w = wins[wi];
         int K = w.K;
-        int* slots = scr + w.off;         // K
+        int* slots = own ? own : scr + w.off;  // K
         int* Lv = slots + K;              // K (left chain, walk order)
         int* Rv = Lv + K;                 // K (right chain, walk order)
         int* Lb = Rv + K;                 // K+1 outer ids, left edges
@@ -417,8 +440,24 @@ __host__ __device__ inline bool cav_retri_one(const Cons& c, const int2* pieces,
     return true;
 }
 
-// R4 body: resolve the marked outer adjacency of rewritten triangle t.
-__host__ __device__ inline void cav_fix_one(const Cons& c, const Win* wins, const int* scr, int t, unsigned epoch)
+// Boundary edges of a cavity above CAV_WAVE_K in polygon order: left edge i at
+// place i (0..nl), right edge i at nl + 1 + i.  The first crossed triangle has
+// places 0 and K + 1, the last nl and nl + 1, any other one.  Finds the new
+// triangle with edge (u, v) from the place recorded for the old one.
+__host__ __device__ inline int cav_new_owner(const Mesh& m, const int* scr, const Win& w, int place, int u, int v)
+{
+    const int* newown = scr + w.off + w.K;
+    int T = newown[place];
+    if (!has2(m.tri[T], u, v)) T = newown[place == 0 ? w.K + 1 : place + 1];
+    return has2(m.tri[T], u, v) ? T : -1;
+}
+
+// R4 body: resolve the marked outer adjacency of rewritten triangle t.  A
+// neighbour rewritten in the same round is found among its cavity's slots, or
+// (byplace: cavities above CAV_WAVE_K recorded their boundary) by the place of
+// the old triangle's boundary edge.
+__host__ __device__ inline void cav_fix_one(const Cons& c, const Win* wins, const int* scr, int t, unsigned epoch,
+                                            bool byplace = false)
 {
     const Mesh& m = c.m;
         int3 tv = m.tri[t];
@@ -432,11 +471,13 @@ __host__ __device__ inline void cav_fix_one(const Cons& c, const Win* wins, cons
                 Win w = wins[c.cavof[nb]];
                 const int* sl = scr + w.off;
                 int found = -1;
-                for (int j = 0; j < w.K; j++)
-                    if (sl[j] != t && has2(m.tri[sl[j]], u, v)) {
-                        found = sl[j];
-                        break;
-                    }
+                if (byplace && w.K > CAV_WAVE_K) found = cav_new_owner(m, scr, w, (int)(unsigned)c.owner[nb], u, v);
+                else
+                    for (int j = 0; j < w.K; j++)
+                        if (sl[j] != t && has2(m.tri[sl[j]], u, v)) {
+                            found = sl[j];
+                            break;
+                        }
                 if (found < 0) at_or(c.err, MERR_ADJ);
                 set3(ta, k, found);
             } else {

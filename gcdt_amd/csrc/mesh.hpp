@@ -127,6 +127,10 @@ enum : int {
     C_HUGE = 26,      // count passes: cells of more elements than one workgroup sorts
     C_VAL = 27,       // mesh check: failed checks (VAL_* bits)
     C_VAL_FIRST = 28, // mesh check: first failing triangle
+    C_NLONG = 29,  // constraint rounds: pieces that cross many triangles
+    C_PATH = 30,   // constraint rounds: their crossed triangles
+    C_NMID = 31,   // constraint rounds: winners among them, by size
+    C_NBIGW = 6,   // (the flip rounds' C_NACT2: not in use at the same time)
     C_NUM = 32
 };
 
@@ -341,7 +345,6 @@ void mark_constraint_edges(Ctx& c, const int3* tri, const int3* adj, int T, int 
 struct ConsResult {
     int rounds = 0;
     long long pieces = 0;
-    long long rewritten = 0;
 };
 // nmax: constraint endpoints must be vertex ids in [0, nmax)
 // cell_end (optional): the Morton cell ends of m.pts (morton_order), so the
