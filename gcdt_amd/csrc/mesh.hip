@@ -1733,6 +1733,12 @@ constexpr int LCL_MAX_LIST = 512;  // rounds of at most this many items use it (
 struct LdsClaims {
     int* tag;
     unsigned long long* key;
+    static constexpr bool kMeta = true;
+    __device__ void propose(const FlipP& f, int t, int n, unsigned long long k) const
+    {
+        max(f, t, k);
+        max(f, n, k);
+    }
     __device__ void max(const FlipP& f, int t, unsigned long long k) const
     {
         unsigned h = hash32((uint32_t)t) & (LCL_CAP - 1);
@@ -1779,6 +1785,13 @@ struct EngSoA {
     Flip f;
     __device__ bool test(int t, unsigned ep, bool all, bool single) const { return flip_test(f, t, ep, all, single); }
     __device__ bool fixtest(int t, unsigned ep, bool all, bool single) const { return test(t, ep, all, single); }
+    // multi-launch rounds: the proposal list holds triangles
+    __device__ int propose(int t, unsigned ep, bool all, bool single) const { return test(t, ep, all, single) ? t : -1; }
+    __device__ int apply_round(int q, unsigned ep, int* t, int* nn) const
+    {
+        *t = q;
+        return apply<false>(q, ep, nn);
+    }
     // no LDS claims for this layout (the persistent tail never asks for them)
     __device__ bool fixtest_l(int t, unsigned ep, const LdsClaims&) const { return test(t, ep, false, false); }
     __device__ int apply_l(int t, unsigned ep, int* nn, const LdsClaims&) const { return apply<true>(t, ep, nn); }
@@ -1800,6 +1813,18 @@ struct EngPacked {
     // the test launch also settles the previous round's flips (flip_fixtest_p)
     static constexpr bool kFused = true;
     FlipP f;
+    PeerClaims pc;  // of the multi-launch rounds
+    // multi-launch rounds: the proposal list holds 3 t + edge
+    __device__ int propose(int t, unsigned ep, bool all, bool single) const
+    {
+        int k;
+        return flip_fixtest_p(f, t, ep, all, single, pc, &k) ? 3 * t + k : -1;
+    }
+    __device__ int apply_round(int q, unsigned ep, int* t, int* nn) const
+    {
+        *t = (int)((unsigned)q / 3u);
+        return flip_apply_peer(f, q, ep, nn, pc);
+    }
     __device__ bool test(int t, unsigned ep, bool all, bool single) const
     {
         return flip_test_p(f, t, ep, all, single);
@@ -1846,10 +1871,7 @@ __global__ __launch_bounds__(kBlock) void k_flip_test(E e, const int* list, cons
             q[j] = -1;
             long long i = base + (long long)j * kBlock + threadIdx.x;
             if (i < n) {
-                int t = list ? list[i] : (int)i;
-                if (E::kFused ? e.fixtest(t, epoch, list == nullptr, single != 0)
-                              : e.test(t, epoch, list == nullptr, single != 0))
-                    q[j] = t;
+                q[j] = e.propose(list ? list[i] : (int)i, epoch, list == nullptr, single != 0);
             }
             nq += q[j] >= 0;
         }
@@ -1883,9 +1905,8 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
             qb[j] = -1;
             long long i = base + (long long)j * kBlock + threadIdx.x;
             if (i < n) {
-                int t = list[i];
-                int nn = -1;
-                int res = e.template apply<false>(t, epoch, &nn);
+                int t, nn = -1;
+                int res = e.apply_round(list[i], epoch, &t, &nn);
                 if (res == 1) e.set_mark(t, (int)epoch + 1);
                 if (res == 1 || res == 2) qa[j] = t;
                 if (res == 2) qb[j] = nn;
@@ -2074,9 +2095,14 @@ namespace {
 // r is queued, and lists at or below the tail threshold finish in one
 // persistent workgroup.
 template <class E>
-long long flip_driver(Ctx& c, const E& e, int T, const int* init, int ninit, int* rounds)
+long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* rounds)
 {
     DBuf<int> la(T), lb(T), lf(T), lp(T);
+    DBuf<int> prop;  // PeerClaims: a byte per triangle
+    if constexpr (E::kFused) {
+        prop.alloc((size_t)T / 4 + 1);
+        e.pc.prop = (unsigned char*)prop.p;
+    }
     const int* act = init;
     int* nxt = la.p;
     int* other = lb.p;
@@ -2113,6 +2139,11 @@ long long flip_driver(Ctx& c, const E& e, int T, const int* init, int ninit, int
         unsigned seq = r > 1 ? c.snap_begin((r - 1) & 1) : 0u;
         k_flip_begin<<<1, C_NUM, 0, c.st>>>(c.dcnt.p, r > 1, snap, seq);
         GCDT_LAUNCH_CHECK();
+        if constexpr (E::kFused) {
+            // tags 1..250 in turn; all bytes are cleared before a tag comes again
+            if ((r - 1) % 250 == 0) fill_i32(c, prop.p, 0, (long long)prop.n);
+            e.pc.tag = (unsigned char)(1 + (r - 1) % 250);
+        }
         with_items(c.flip_items, [&](auto it) {
             constexpr int IT = decltype(it)::value;
             {

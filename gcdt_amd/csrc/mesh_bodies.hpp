@@ -538,7 +538,12 @@ __host__ __device__ inline bool flip_test_p(const FlipP& f, int t, unsigned epoc
 // workgroup (mesh.hip).  get<COH> returns t's claim; `loaded` is the word
 // already read with t's record, used when no re-read is needed.
 struct RecClaims {
-    __host__ __device__ void max(const FlipP& f, int t, unsigned long long key) const { at_max(&f.r[t].claim, key); }
+    static constexpr bool kMeta = true;  // proposals are kept in the records' meta words
+    __host__ __device__ void propose(const FlipP& f, int t, int n, unsigned long long key) const
+    {
+        at_max(&f.r[t].claim, key);
+        at_max(&f.r[n].claim, key);
+    }
     template <bool COH>
     __host__ __device__ unsigned long long get(const FlipP& f, int t, unsigned long long loaded) const
     {
@@ -549,6 +554,27 @@ struct RecClaims {
     __host__ __device__ unsigned long long load(const FlipP& f, int t) const
     {
         return ld_claim<COH>(&f.r[t].claim);
+    }
+};
+
+// Claims of the multi-launch rounds: a proposal claims only the triangle across
+// its edge.  That t proposes is itself t's claim on t: a byte per triangle says
+// so (the tag of the round; the bytes are cleared before a tag comes again),
+// and the proposed edge travels in the proposal list, so that a test writes
+// nothing into its own record.
+//
+// Device-scope atomics and partial writes are memory-side requests here, and
+// they bound the test: 55 ps an atomic whatever its address (10M random ones
+// take 580 us), about 20 ps a partial write.  Two atomics and a meta word per
+// proposal made 27.7M such requests in the second round over 20M triangles.
+struct PeerClaims {
+    static constexpr bool kMeta = false;
+    unsigned char* prop;
+    unsigned char tag;
+    __host__ __device__ void propose(const FlipP& f, int t, int n, unsigned long long key) const
+    {
+        at_max(&f.r[n].claim, key);
+        prop[t] = tag;
     }
 };
 
@@ -567,9 +593,10 @@ struct RecClaims {
 //   vertices is resolved to its partner of that flip.
 // By the end of the launch every entry and back-pointer is settled, as after
 // a separate fix launch; the last round's flips are settled by flip_fix_p.
+// *edge (optional) receives the proposed edge, 3 for none.
 template <class CL = RecClaims>
 __host__ __device__ inline bool flip_fixtest_p(const FlipP& f, int t, unsigned epoch, bool all_active,
-                                               bool single = true, const CL& cl = CL())
+                                               bool single = true, const CL& cl = CL(), int* edge = nullptr)
 {
     const FRec r = rec_load(&f.r[t]);
     const int prev = (int)epoch - 1;
@@ -628,15 +655,69 @@ __host__ __device__ inline bool flip_fixtest_p(const FlipP& f, int t, unsigned e
         if (incircle(r.p[0], r.p[1], r.p[2], rec_pt(rn, j)) > 0) {
             cand = k;
             const unsigned long long key = ((unsigned long long)epoch << 32) | (unsigned)(3 * t + k);
-            cl.max(f, t, key);
-            cl.max(f, n, key);
+            cl.propose(f, t, n, key);
         }
     }
     // most tested triangles propose nothing and already say so: a store would
     // only dirty the line
-    const int meta = (r.meta & ~(3 << 3)) | (cand << 3);
-    if (meta != r.meta) f.r[t].meta = meta;
+    if (CL::kMeta) {
+        const int meta = (r.meta & ~(3 << 3)) | (cand << 3);
+        if (meta != r.meta) f.r[t].meta = meta;
+    }
+    if (edge) *edge = cand;
     return cand != 3;
+}
+
+// Flips edge k of t (record r) with its neighbour n (record rn): both records
+// are written whole, the claim word as given.
+// t = (p,u,v), n = (o,v,u)  ->  t = (p,u,o) [partner in slot 1], n = (p,o,v) [partner in slot 2]
+__host__ __device__ inline void flip_records(const FlipP& f, int t, const FRec& r, int k, int n, const FRec& rn,
+                                             unsigned epoch, unsigned long long key)
+{
+    const int kn = nx3(k), kp = pv3(k);
+    const int p = get3(r.v, k), u = get3(r.v, kn), v = get3(r.v, kp);
+    const int j = slot_other(rn.v, u, v);
+    const int jn = nx3(j), jp = pv3(j);
+    const int o = get3(rn.v, j);
+    const int cft = r.meta & 7, cfn = rn.meta & 7;
+    const int2 pp = rec_pt(r, k), pu = rec_pt(r, kn), pv = rec_pt(r, kp), po = rec_pt(rn, j);
+    const int mk = (int)epoch + 1;
+    rec_store(&f.r[t], make_int3(p, u, o), make_int3(get3(rn.a, jn), n, get3(r.a, kp)), pp, pu, po,
+              rec_with_mark(((cfn >> jn) & 1) | (((cft >> kp) & 1) << 2) | FREC_NOCAND | (1 << 5), mk), (int)epoch,
+              key);
+    rec_store(&f.r[n], make_int3(p, o, v), make_int3(get3(rn.a, jp), get3(r.a, kn), t), pp, po, pv,
+              rec_with_mark(((cfn >> jp) & 1) | (((cft >> kn) & 1) << 1) | FREC_NOCAND | (2 << 5), mk), (int)epoch,
+              key);
+}
+
+// flip_apply of proposal e = 3 t + edge under PeerClaims (return codes of
+// flip_apply).  t's own proposal and the claims on it by others are compared
+// here: t loses to a claim on t above its own key, and to a claim on n, or a
+// proposal of n itself, above it.
+//
+// Records are read while winners rewrite them, 16 bytes at a time, but only
+// stable words decide: a triangle flipped by another proposal holds that
+// proposal's key in its claim word before, during and after the rewrite, so
+// nothing else of t's record is used unless its claim word is below t's key
+// (then no one else flips t); n's other fields are used only by the winner;
+// the prop bytes do not change in this pass.  A flip leaves its own key in
+// both claim words, which a proposer that lost to it may read in either state.
+__host__ __device__ inline int flip_apply_peer(const FlipP& f, int e, unsigned epoch, int* nout, const PeerClaims& cl)
+{
+    const int t = (int)((unsigned)e / 3u), k = e - 3 * t;
+    const unsigned long long key = ((unsigned long long)epoch << 32) | (unsigned)e;
+    const FRec r = rec_load(&f.r[t]);
+    if (r.claim > key) {
+        // r.claim is t2's; it wins (and flips t) unless t2 is claimed above it
+        const int t2 = (int)((r.claim & 0xffffffffu) / 3);
+        return ld_claim<false>(&f.r[t2].claim) <= r.claim ? 3 : 1;
+    }
+    const int n = get3(r.a, k);
+    const FRec rn = rec_load(&f.r[n]);
+    if (rn.claim != key || (n > t && cl.prop[n] == cl.tag)) return 1;
+    flip_records(f, t, r, k, n, rn, epoch, key);
+    *nout = n;
+    return 2;
 }
 
 // flip_apply over records: same claims protocol and return codes.  A flip
@@ -672,21 +753,7 @@ __host__ __device__ inline int flip_apply_p(const FlipP& f, int t, unsigned epoc
     const FRec rn = rec_load(&f.r[n]);
     const unsigned long long cn = cl.template get<COH>(f, n, rn.claim);
     if (cn != key) return 1;
-    const int kn = nx3(k), kp = pv3(k);
-    const int p = get3(r.v, k), u = get3(r.v, kn), v = get3(r.v, kp);
-    const int j = slot_other(rn.v, u, v);
-    const int jn = nx3(j), jp = pv3(j);
-    const int o = get3(rn.v, j);
-    const int cft = r.meta & 7, cfn = rn.meta & 7;
-    const int2 pp = rec_pt(r, k), pu = rec_pt(r, kn), pv = rec_pt(r, kp), po = rec_pt(rn, j);
-    const int mk = (int)epoch + 1;
-    // t = (p,u,v), n = (o,v,u)  ->  t = (p,u,o) [partner in slot 1], n = (p,o,v) [partner in slot 2]
-    rec_store(&f.r[t], make_int3(p, u, o), make_int3(get3(rn.a, jn), n, get3(r.a, kp)), pp, pu, po,
-              rec_with_mark(((cfn >> jn) & 1) | (((cft >> kp) & 1) << 2) | FREC_NOCAND | (1 << 5), mk), (int)epoch,
-              key);
-    rec_store(&f.r[n], make_int3(p, o, v), make_int3(get3(rn.a, jp), get3(r.a, kn), t), pp, po, pv,
-              rec_with_mark(((cfn >> jp) & 1) | (((cft >> kn) & 1) << 1) | FREC_NOCAND | (2 << 5), mk), (int)epoch,
-              key);
+    flip_records(f, t, r, k, n, rn, epoch, key);
     *nout = n;
     return 2;
 }
