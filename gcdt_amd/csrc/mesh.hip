@@ -188,6 +188,23 @@ __device__ inline void snap_store(unsigned long long* dst, unsigned seq, int v)
                        __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+__device__ inline void round_snap_store(const RoundSnap& s)
+{
+    if (s.dst && blockIdx.x == 0 && threadIdx.x < C_NUM) {
+        const int j = threadIdx.x;
+        snap_store(&s.dst[j], s.seq, j == S_ERR ? *s.err : (j < ROUND_WORDS ? s.set[j * ROUND_LINE] : 0));
+    }
+}
+
+__global__ void k_round_snap(RoundSnap s) { round_snap_store(s); }
+
+__global__ __launch_bounds__(kBlock) void k_rounds_start(int* ring, int next, int base)
+{
+    static_assert(ROUND_INTS == kBlock, "a workgroup per set");
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    ring[i] = i == R_NEXT ? next : (i == ROUND_INTS + R_BASE ? base : 0);
+}
+
 // the counters straight into the mapped pinned ring (a kernel costs less
 // than a copy-engine transfer)
 __global__ void k_snap(const int* cnt, unsigned long long* dst, unsigned seq)
@@ -242,6 +259,38 @@ const int* Ctx::wait_snapshot(int slot)
             if (e != hipErrorNotReady) GCDT_HIP(e);
         }
     }
+}
+
+void Ctx::rounds_start(int next, int base)
+{
+    ring.ensure(ROUND_SETS * ROUND_INTS);
+    k_rounds_start<<<ROUND_SETS, kBlock, 0, st>>>(ring.p, next, base);
+    GCDT_LAUNCH_CHECK();
+}
+
+void Ctx::rounds_turn(int r)
+{
+    // half way through one half of the ring the other half is cleared: its
+    // rounds are done and read, and it comes into use half a half later
+    constexpr int half = ROUND_SETS / 2;
+    if (r % half == half / 2 && r > half)
+        fill_i32(*this, ring.p + (r / half % 2 ? 0 : half * ROUND_INTS), 0, half * ROUND_INTS);
+}
+
+RoundSnap Ctx::round_snap(int r)
+{
+    RoundSnap s;
+    s.seq = snap_begin(r & 1);
+    s.dst = snap_dst(r & 1);
+    s.set = round_set(r);
+    s.err = dcnt.p + C_ERR;
+    return s;
+}
+
+void Ctx::round_snapshot(int r)
+{
+    k_round_snap<<<1, C_NUM, 0, st>>>(round_snap(r));
+    GCDT_LAUNCH_CHECK();
 }
 
 void Ctx::read(int i, int k)
@@ -1353,22 +1402,6 @@ int locate_bitmap_batch(Ctx& c, const int2* pts, const int* vinst, long long NP,
 
 // ================================================================== insertion rounds
 
-// Round prologue on the device: the previous round's output list becomes the
-// input (count C_NPEND2 -> C_NPEND) and the slot base is recorded.
-// With snap set, it first copies the previous round's counters to the host
-// ring (one launch instead of a begin kernel plus a copy).  C_NUM threads.
-__global__ void k_round_begin(int* cnt, int move, unsigned long long* snap, unsigned seq)
-{
-    if (snap) snap_store(&snap[threadIdx.x], seq, cnt[threadIdx.x]);
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    if (move) cnt[C_NPEND] = cnt[C_NPEND2];
-    cnt[C_NPEND2] = 0;
-    cnt[C_TBASE] = cnt[C_NTRI];
-    cnt[C_NW] = cnt[C_NW2];
-    cnt[C_NW2] = 0;
-}
-
 // The claimed-triangle list of a round: the claim whose atomicMax finds a key
 // of an older epoch is the triangle's first this round and appends it, so
 // every claimed triangle is listed once and the split step walks these
@@ -1460,9 +1493,11 @@ void with_items(int v, F&& f)
 // from the second one it claimed.
 template <int INS_ITEMS>
 __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, const int* cnt, int lcap, unsigned epoch,
-                                                      int* ntri)
+                                                      int* set, RoundSnap snap)
 {
+    round_snap_store(snap);
     int n = min(*cnt, lcap);  // an overfull list has flagged MERR_CAPACITY
+    const int first = set[R_BASE];
     TILE_LOOP(base, n, kBlock * INS_ITEMS)
     {
         int pp[INS_ITEMS], need[INS_ITEMS];
@@ -1483,7 +1518,7 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
             }
             tot += need[j];
         }
-        int b = block_alloc<kBlock>(tot, ntri);
+        int b = first + block_alloc<kBlock>(tot, &set[R_NEW]);
 #pragma unroll
         for (int j = 0; j < INS_ITEMS; j++) {
             if (need[j]) {
@@ -1495,22 +1530,25 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_ins_fix(Ins s, const int* cnt)
-{
-    int b = cnt[C_TBASE], e = min(cnt[C_NTRI], s.cap);
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x + b; i < e; i += (long long)gridDim.x * blockDim.x)
-        ins_fix(s, (int)i);
-}
-
-// Relocation of the pending points after the splits, fused with the next
-// round's claims (epoch next_ep) and its claimed-triangle list.
+// Outer adjacency of the round's new triangles (their slots follow from the
+// round's counters), then the relocation of the pending points, fused with the
+// next round's claims (epoch next_ep) and its claimed-triangle list.  Only the
+// claims of on-edge points read adjacency, and they resolve entries that this
+// launch has not settled yet (ins_edge_neighbour).  The slots of the next round
+// begin where this round's end.
 template <int INS_ITEMS>
-__global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, const int* cnt, int* list2, int* cnt2,
-                                                      unsigned next_ep, int* wl, int* nw, int wcap)
+__global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, const int* cnt, int* list2,
+                                                      unsigned next_ep, int* wl, int wcap, int* set, int* next_set)
 {
     __shared__ int s_buf[STAGE_CAP], s_buf2[STAGE_CAP];
     __shared__ int s_base, s_base2;
-    Staged<STAGE_CAP> sl(s_buf, &s_base, list2, cnt2), sw(s_buf2, &s_base2, wl, nw, wcap, s.err, MERR_CAPACITY);
+    Staged<STAGE_CAP> sl(s_buf, &s_base, list2, &set[R_NEXT]),
+        sw(s_buf2, &s_base2, wl, &set[R_NW], wcap, s.err, MERR_CAPACITY);
+    const int tb = set[R_BASE], te = tb + set[R_NEW];
+    if (blockIdx.x == 0 && threadIdx.x == 0) next_set[R_BASE] = te;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x + tb; i < min(te, s.cap);
+         i += (long long)gridDim.x * blockDim.x)
+        ins_fix(s, (int)i);
     int n = *cnt;
     TILE_LOOP(base, n, kBlock * INS_ITEMS)
     {
@@ -1540,14 +1578,24 @@ __global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, co
 // launch (block barriers between the phases, LDS counters for the lists)
 constexpr int TAIL_BS = 1024;
 
-__global__ __launch_bounds__(TAIL_BS) void k_ins_tail(Ins s, int* P, int* P2, int* cnt, int cp, unsigned epoch0,
-                                                      int max_rounds)
+// What a persistent tail hands to the host ring in place of the counters: one
+// word per thread, the others 0.
+__device__ inline void tail_snap(const RoundSnap& snap, int n, int r, int err, int ntri, int flips)
+{
+    const int j = threadIdx.x;
+    if (j >= C_NUM) return;
+    int v = j == C_TAIL_N ? n : j == C_TAIL_R ? r : j == C_TAIL_ERR ? err : j == C_NTRI ? ntri : j == C_TAIL_F ? flips : 0;
+    if (j == C_ERR) v = __hip_atomic_load(snap.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    snap_store(&snap.dst[j], snap.seq, v);
+}
+
+__global__ __launch_bounds__(TAIL_BS) void k_ins_tail(Ins s, int* P, int* P2, int n, int ntri, unsigned epoch0,
+                                                      int max_rounds, RoundSnap snap)
 {
     __shared__ int s_np, s_nt, s_tb;
-    int n = cnt[cp];
     unsigned ep = epoch0;
     int r = 0, err = 0;
-    if (threadIdx.x == 0) s_nt = __hip_atomic_load(&cnt[C_NTRI], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) s_nt = ntri;
     __syncthreads();
     while (n > 0 && r < max_rounds) {
         for (int i = threadIdx.x; i < n; i += TAIL_BS) ins_claim(s, P[i], ep);
@@ -1591,36 +1639,37 @@ __global__ __launch_bounds__(TAIL_BS) void k_ins_tail(Ins s, int* P, int* P2, in
         r++;
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        cnt[C_NTRI] = s_nt;
-        cnt[C_TAIL_N] = n;
-        cnt[C_TAIL_R] = r;
-        cnt[C_TAIL_ERR] = err;
-        cnt[C_TAIL_PAR] = r & 1;
-    }
+    __syncthreads();
+    tail_snap(snap, n, r, err, s_nt, 0);
 }
 
 int insert_rounds(Ctx& c, const Ins& s_in, DBuf<int>& pend, DBuf<int>& pend2, int npend, int ntri, int* rounds)
 {
     Ins s = s_in;
     s.pivot = c.pivot;
-    c.set(C_NPEND, npend);
-    c.set(C_NTRI, ntri);
     int* P = pend.p;   // input list of the next round to launch
     int* P2 = pend2.p;
     int r = 0;
     int est = npend;  // estimate of the next round's input size (exact for the first)
+    int nt = ntri;
     bool done = npend == 0;
     // Rounds are launched one ahead of the host's knowledge of their input
     // size: each round's counters are snapshot asynchronously and read after
     // the next round is queued, so the GPU does not wait for the host.
+    int n_in = npend;  // input of the round whose counters are read next
+    int nw_in = 0;     // and the triangles claimed for it (0: not known)
     auto check_round = [&](const int* h) {
-        if (h[C_ERR]) c.check_err();
-        if (h[C_NPEND] > 0 && h[C_NPEND2] >= h[C_NPEND] && h[C_NTRI] == h[C_TBASE])
+        if (h[S_ERR]) c.check_err();
+        if (n_in > 0 && h[S_NEXT] >= n_in && h[S_NEW] == 0)
             throw Error(GCDT_ERR_INTERNAL, "insertion round without progress");
         // exact list lengths of the round, for per-item bytes of the timed kernels
-        prof_add_items("ins_split", h[C_NW]);
-        prof_add_items("ins_reloc", h[C_NPEND]);
+        prof_add_items("ins_split", nw_in);
+        prof_add_items("ins_reloc", n_in);
+        n_in = h[S_NEXT];
+        nw_in = h[S_NW];
+        nt = h[S_BASE] + h[S_NEW];
+        if (n_in == 0) done = true;
+        est = n_in;
     };
     // Claimed-triangle lists: every pending point claims at most two
     // triangles, and each claimed triangle is listed once per round.
@@ -1633,94 +1682,65 @@ int insert_rounds(Ctx& c, const Ins& s_in, DBuf<int>& pend, DBuf<int>& pend2, in
         wb.ensure((size_t)wcap);
         W = wa.p;
         W2 = wb.p;
+        c.rounds_start(npend, ntri);
         // the first round's claims; later rounds claim inside the relocation
-        c.set(C_NW2, 0);
         ProfScope ps("ins_claim", c.st, est);
-        k_ins_claim_w<<<grid_for(est), kBlock, 0, c.st>>>(s, P, c.dcnt.p + C_NPEND, c.epoch + 1, W2,
-                                                          c.dcnt.p + C_NW2, (int)wcap);
+        k_ins_claim_w<<<grid_for(est), kBlock, 0, c.st>>>(s, P, c.round_set(0) + R_NEXT, c.epoch + 1, W2,
+                                                          c.round_set(0) + R_NW, (int)wcap);
         GCDT_LAUNCH_CHECK();
     }
     while (!done && est > c.tail_threshold) {
         if (++r > 100000) throw Error(GCDT_ERR_NOT_CONVERGED, "insertion rounds did not converge");
         unsigned ep = c.next_epoch();
-        // begins round r and snapshots round r-1 for the host
-        unsigned long long* snap = r > 1 ? c.snap_dst((r - 1) & 1) : nullptr;
-        unsigned seq = r > 1 ? c.snap_begin((r - 1) & 1) : 0u;
-        k_round_begin<<<1, C_NUM, 0, c.st>>>(c.dcnt.p, r > 1, snap, seq);
-        GCDT_LAUNCH_CHECK();
+        c.rounds_turn(r);
+        int *in = c.round_set(r - 1), *set = c.round_set(r);
+        // round r - 1 goes to the host with round r's first kernel
+        const RoundSnap snap = r > 1 ? c.round_snap(r - 1) : RoundSnap{};
         std::swap(W, W2);
         with_items(c.ins_items, [&](auto it) {
             constexpr int IT = decltype(it)::value;
             ProfScope ps("ins_split", c.st, 0);
-            k_ins_split<IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(s, W, c.dcnt.p + C_NW, (int)wcap,
-                                                                                 ep, c.dcnt.p + C_NTRI);
+            k_ins_split<IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(s, W, in + R_NW, (int)wcap, ep, set,
+                                                                                 snap);
             GCDT_LAUNCH_CHECK();
         });
-        {
-            ProfScope ps("ins_fix", c.st, 0);
-            k_ins_fix<<<grid_for(4LL * est), kBlock, 0, c.st>>>(s, c.dcnt.p);
-            GCDT_LAUNCH_CHECK();
-        }
         with_items(c.ins_items, [&](auto it) {
             constexpr int IT = decltype(it)::value;
             ProfScope ps("ins_reloc", c.st, 0);
             k_ins_reloc<IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
-                s, P, c.dcnt.p + C_NPEND, P2, c.dcnt.p + C_NPEND2, ep + 1, W2, c.dcnt.p + C_NW2, (int)wcap);
+                s, P, in + R_NEXT, P2, ep + 1, W2, (int)wcap, set, c.round_set(r + 1));
             GCDT_LAUNCH_CHECK();
         });
         std::swap(P, P2);
-        if (r >= 2) {
-            const int* h = c.wait_snapshot((r - 1) & 1);  // round r-1 (round r is queued)
-            check_round(h);
-            if (h[C_NPEND2] == 0) done = true;  // round r had no input
-            est = h[C_NPEND2];
-        }
+        if (r >= 2) check_round(c.round_wait(r - 1));  // round r is queued
     }
     if (r >= 1) {
-        c.snapshot(r & 1);
-        const int* h = c.wait_snapshot(r & 1);
-        check_round(h);
-        if (h[C_NPEND2] == 0) done = true;
-        est = h[C_NPEND2];
+        c.round_snapshot(r);
+        check_round(c.round_wait(r));
     }
     if (!done) {
-        // finish in one persistent workgroup; its input is P with the count moved
-        k_round_begin<<<1, C_NUM, 0, c.st>>>(c.dcnt.p, r > 0, nullptr, 0u);
-        GCDT_LAUNCH_CHECK();
+        // finish in one persistent workgroup
         unsigned ep0 = c.epoch + 1;
+        RoundSnap snap = c.round_snap(0);
         {
             ProfScope ps("ins_tail", c.st, est);
-            k_ins_tail<<<1, TAIL_BS, 0, c.st>>>(s, P, P2, c.dcnt.p, C_NPEND, ep0, 1 << 20);
+            k_ins_tail<<<1, TAIL_BS, 0, c.st>>>(s, P, P2, est, nt, ep0, 1 << 20, snap);
             GCDT_LAUNCH_CHECK();
         }
-        c.read(0, C_NUM);
-        if (c.hcnt[C_ERR]) c.check_err();
-        if (c.hcnt[C_TAIL_ERR]) throw Error(GCDT_ERR_INTERNAL, "insertion round without progress (tail)");
-        r += c.hcnt[C_TAIL_R];
-        c.epoch += (unsigned)c.hcnt[C_TAIL_R];
-        if (c.hcnt[C_TAIL_N] != 0) throw Error(GCDT_ERR_NOT_CONVERGED, "insertion tail did not converge");
+        const int* h = c.round_wait(0);
+        if (h[C_ERR]) c.check_err();
+        if (h[C_TAIL_ERR]) throw Error(GCDT_ERR_INTERNAL, "insertion round without progress (tail)");
+        r += h[C_TAIL_R];
+        c.epoch += (unsigned)h[C_TAIL_R];
+        if (h[C_TAIL_N] != 0) throw Error(GCDT_ERR_NOT_CONVERGED, "insertion tail did not converge");
+        nt = h[C_NTRI];
     }
     if (rounds) *rounds = r;
-    int nt = c.get(C_NTRI);
     if (nt > s.cap) throw Error(GCDT_ERR_CAPACITY, "triangle capacity exceeded");
     return nt;
 }
 
 // ================================================================== flip rounds
-
-// Flip round prologue: the previous round's output list becomes the input.
-// With snap set, it first copies the previous round's counters to the host
-// ring.  C_NUM threads.
-__global__ void k_flip_begin(int* cnt, int move, unsigned long long* snap, unsigned seq)
-{
-    if (snap) snap_store(&snap[threadIdx.x], seq, cnt[threadIdx.x]);
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    if (move) cnt[C_NACT] = cnt[C_NACT2];
-    cnt[C_NACT2] = 0;
-    cnt[C_NFLIP] = 0;
-    cnt[C_NPROP] = 0;
-}
 
 // Claims of the short rounds of one persistent workgroup, in an LDS hash
 // table instead of the records' claim words (device-scope atomics and
@@ -1854,8 +1874,10 @@ struct EngPacked {
 // `prop`, the only list the apply step reads.
 template <class E, int FT_ITEMS>
 __global__ __launch_bounds__(kBlock) void k_flip_test(E e, const int* list, const int* cnt, int lcap, unsigned epoch,
-                                                      int single, int* prop, int* nprop, int cap, int* eflag)
+                                                      int single, int* prop, int* nprop, int cap, int* eflag,
+                                                      RoundSnap snap)
 {
+    round_snap_store(snap);
     __shared__ int s_buf[STAGE_CAP];
     __shared__ int s_base;
     // a triangle proposes at most once per round, so `prop` (cap entries)
@@ -1940,8 +1962,8 @@ __global__ __launch_bounds__(kBlock) void k_flip_fix(E e, const int* list, const
 
 // Persistent single-workgroup tail of the flip rounds.
 template <class E>
-__global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int* lf, int* cnt, int cap,
-                                                       unsigned epoch0, int max_rounds)
+__global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int* lf, int n, int cap, unsigned epoch0,
+                                                       int max_rounds, int* eflag, RoundSnap snap)
 {
     // round counters double-buffered by round parity: a round's pair is reset
     // after the round's first barrier, which every thread passes only after
@@ -1951,8 +1973,7 @@ __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int*
     // table per round parity: the other one is cleared while a round applies
     __shared__ int s_tag[2][LCL_CAP];
     __shared__ unsigned long long s_key[2][LCL_CAP];
-    int n = min(cnt[C_NACT], cap);  // A, B and lf hold cap entries each
-    unsigned ep = epoch0;
+    unsigned ep = epoch0;  // A, B and lf hold cap entries each, n <= cap
     int r = 0, err = 0, flips = 0;
     int nf = 0;
     if (threadIdx.x == 0) {
@@ -2013,7 +2034,7 @@ __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int*
         int n2 = s_n2[q];
         nf = s_nf[q];
         if (n2 > cap || nf > cap) {  // cannot happen (one entry per triangle): flagged, not written
-            if (threadIdx.x == 0) atomicOr(&cnt[C_ERR], MERR_CAPACITY);
+            if (threadIdx.x == 0) atomicOr(eflag, MERR_CAPACITY);
             n = 0;
             break;
         }
@@ -2038,12 +2059,8 @@ __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int*
         for (int i = threadIdx.x; i < nf; i += TAIL_BS) e.fix(lf[i], ep - 1);
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        cnt[C_TAIL_N] = n;
-        cnt[C_TAIL_R] = r;
-        cnt[C_TAIL_ERR] = err;
-        cnt[C_TAIL_F] = flips;
-    }
+    __syncthreads();
+    tail_snap(snap, n, r, err, 0, flips);
 }
 
 template <class E>
@@ -2088,12 +2105,26 @@ __global__ __launch_bounds__(kBlock) void k_unpack_faces(const FRec* __restrict_
 
 namespace {
 
+// The two-tester rounds of at most this many triangles run in one persistent
+// workgroup; larger ones as launches of their own.  A workgroup takes about
+// 50 us for a round of 2,000 to 4,000 triangles (its one CU has 16 of them per
+// lane to work through) and 10 us for 700; a launched round takes 20 us at
+// either size.
+#ifndef GCDT_FLIP_WG_LIST
+#define GCDT_FLIP_WG_LIST 1024
+#endif
+constexpr int FLIP_WG_LIST = GCDT_FLIP_WG_LIST;
+
 // Rounds of test / apply / fix over a triangle list until no edge needs a
-// flip.  Round 1 reads `init` (or the implicit list of all T triangles,
-// counted in C_CONST); later rounds alternate between two device lists whose
-// lengths stay on the device (C_NACT); the host checks round r-1 while round
-// r is queued, and lists at or below the tail threshold finish in one
-// persistent workgroup.
+// flip.  Round 1 reads `init` (or the implicit list of all T triangles); later
+// rounds alternate between two device lists whose lengths stay on the device
+// (the rounds' counter ring); the host checks round r-1 while round r is
+// queued.  Lists above the tail threshold are tested by the lower of an edge's
+// two active triangles (single tester); from there on every listed triangle
+// tests, in launched rounds down to FLIP_WG_LIST triangles and then in one
+// persistent workgroup.  Where the rounds change over decides which flips
+// meet in a round, and with them the slots of the result, so the threshold is
+// the tunable's alone; FLIP_WG_LIST changes nothing but the time.
 template <class E>
 long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* rounds)
 {
@@ -2106,88 +2137,83 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
     const int* act = init;
     int* nxt = la.p;
     int* other = lb.p;
+    int est = init ? ninit : T;
+    if (est > std::min(c.tail_threshold, FLIP_WG_LIST)) c.rounds_start(est, 0);
     if (init) {
-        c.set(C_NACT, ninit);
         k_mark_list<E><<<grid_for(ninit), kBlock, 0, c.st>>>(e, init, ninit, (int)c.epoch + 1);
         GCDT_LAUNCH_CHECK();
-    } else {
-        c.set(C_CONST, T);
     }
     long long flips = 0;
     long long settled = 0;  // fused engines: flipped triangles settled inside test launches
     int r = 0;
-    int est = init ? ninit : T;
     bool done = est == 0;
-    int checked = 0;  // rounds whose snapshot has been read
+    int n_in = est;   // input of the round whose counters are read next
+    int n_flip = 0;   // flipped triangles of the last round read
     auto check_round = [&](const int* h) {
-        if (h[C_ERR]) c.check_err();
+        if (h[S_ERR]) c.check_err();
         // the highest-keyed proposal always wins both of its triangles
-        if (h[C_NACT2] > 0 && h[C_NFLIP] == 0) throw Error(GCDT_ERR_INTERNAL, "flip round without progress");
-        flips += h[C_NFLIP] / 2;
-        settled += h[C_NFLIP];
-        ++checked;
-        prof_add_items("flip_test", (checked == 1 && !init) ? h[C_CONST] : h[C_NACT]);
-        prof_add_items("flip_apply", h[C_NPROP]);
-        if (!E::kFused) prof_add_items("flip_fix", h[C_NFLIP]);  // else settled by the next test launch
+        if (h[S_NEXT] > 0 && h[S_FLIP] == 0) throw Error(GCDT_ERR_INTERNAL, "flip round without progress");
+        n_flip = h[S_FLIP];
+        flips += n_flip / 2;
+        settled += n_flip;
+        prof_add_items("flip_test", n_in);
+        prof_add_items("flip_apply", h[S_PROP]);
+        if (!E::kFused) prof_add_items("flip_fix", n_flip);  // else settled by the next test launch
+        n_in = h[S_NEXT];
+        if (n_in == 0) done = true;
+        est = n_in;
     };
-    while (!done && est > c.tail_threshold) {
-        if (++r > 1000000) throw Error(GCDT_ERR_NOT_CONVERGED, "flip rounds did not converge");
-        unsigned ep = c.next_epoch();
-        int cnt_idx = (r == 1 && !init) ? C_CONST : C_NACT;
-        // begins round r and snapshots round r-1 for the host
-        unsigned long long* snap = r > 1 ? c.snap_dst((r - 1) & 1) : nullptr;
-        unsigned seq = r > 1 ? c.snap_begin((r - 1) & 1) : 0u;
-        k_flip_begin<<<1, C_NUM, 0, c.st>>>(c.dcnt.p, r > 1, snap, seq);
-        GCDT_LAUNCH_CHECK();
-        if constexpr (E::kFused) {
-            // tags 1..250 in turn; all bytes are cleared before a tag comes again
-            if ((r - 1) % 250 == 0) fill_i32(c, prop.p, 0, (long long)prop.n);
-            e.pc.tag = (unsigned char)(1 + (r - 1) % 250);
-        }
-        with_items(c.flip_items, [&](auto it) {
-            constexpr int IT = decltype(it)::value;
-            {
-                ProfScope ps("flip_test", c.st, 0);
-                k_flip_test<E, IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
-                    e, act, c.dcnt.p + cnt_idx, (init && act == init) ? ninit : T, ep, c.single_tester, lp.p,
-                    c.dcnt.p + C_NPROP, T, c.dcnt.p + C_ERR);
+    auto launch_rounds = [&](int down_to, int single) {
+        while (!done && est > down_to) {
+            if (++r > 1000000) throw Error(GCDT_ERR_NOT_CONVERGED, "flip rounds did not converge");
+            unsigned ep = c.next_epoch();
+            c.rounds_turn(r);
+            int *in = c.round_set(r - 1), *set = c.round_set(r);
+            // round r - 1 goes to the host with round r's first kernel
+            const RoundSnap snap = r > 1 ? c.round_snap(r - 1) : RoundSnap{};
+            if constexpr (E::kFused) {
+                // tags 1..250 in turn; all bytes are cleared before a tag comes again
+                if ((r - 1) % 250 == 0) fill_i32(c, prop.p, 0, (long long)prop.n);
+                e.pc.tag = (unsigned char)(1 + (r - 1) % 250);
+            }
+            with_items(c.flip_items, [&](auto it) {
+                constexpr int IT = decltype(it)::value;
+                {
+                    ProfScope ps("flip_test", c.st, 0);
+                    k_flip_test<E, IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
+                        e, act, in + R_NEXT, (init && act == init) ? ninit : T, ep, single, lp.p, set + R_PROP, T,
+                        c.dcnt.p + C_ERR, snap);
+                    GCDT_LAUNCH_CHECK();
+                }
+                {
+                    ProfScope ps("flip_apply", c.st, 0);
+                    k_flip_apply<E, IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
+                        e, lp.p, set + R_PROP, ep, nxt, set + R_NEXT, lf.p, set + R_FLIP, T, c.dcnt.p + C_ERR);
+                    GCDT_LAUNCH_CHECK();
+                }
+            });
+            if (!E::kFused) {
+                ProfScope ps("flip_fix", c.st, 0);
+                k_flip_fix<E><<<grid_for(est), kBlock, 0, c.st>>>(e, lf.p, set + R_FLIP, T, ep);
                 GCDT_LAUNCH_CHECK();
             }
-            {
-                ProfScope ps("flip_apply", c.st, 0);
-                k_flip_apply<E, IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
-                    e, lp.p, c.dcnt.p + C_NPROP, ep, nxt, c.dcnt.p + C_NACT2, lf.p, c.dcnt.p + C_NFLIP, T,
-                    c.dcnt.p + C_ERR);
-                GCDT_LAUNCH_CHECK();
-            }
-        });
-        if (!E::kFused) {
-            ProfScope ps("flip_fix", c.st, 0);
-            k_flip_fix<E><<<grid_for(est), kBlock, 0, c.st>>>(e, lf.p, c.dcnt.p + C_NFLIP, T, ep);
-            GCDT_LAUNCH_CHECK();
+            act = nxt;
+            std::swap(nxt, other);
+            if (r >= 2) check_round(c.round_wait(r - 1));  // round r is queued
         }
-        act = nxt;
-        std::swap(nxt, other);
-        if (r >= 2) {
-            const int* h = c.wait_snapshot((r - 1) & 1);  // round r-1 (round r is queued)
-            check_round(h);
-            if (h[C_NACT2] == 0) done = true;
-            est = h[C_NACT2];
-        }
-    }
+    };
+    launch_rounds(c.tail_threshold, c.single_tester);
+    launch_rounds(FLIP_WG_LIST, 0);
     if (r >= 1) {
-        c.snapshot(r & 1);
-        const int* h = c.wait_snapshot(r & 1);
-        check_round(h);
-        if (h[C_NACT2] == 0) done = true;
-        est = h[C_NACT2];
+        c.round_snapshot(r);
+        check_round(c.round_wait(r));
         // the last round's flips are settled by the tail (or the fix below)
-        if (E::kFused) prof_add_items("flip_test_fix", settled - h[C_NFLIP]);
-        if (E::kFused && done && h[C_NFLIP] > 0) {
+        if (E::kFused) prof_add_items("flip_test_fix", settled - n_flip);
+        if (E::kFused && done && n_flip > 0) {
             // settle the last round's flips (no test follows; the tail's first
             // test settles them when the tail runs)
-            ProfScope ps("flip_fix", c.st, h[C_NFLIP]);
-            k_flip_fix<E><<<grid_for(h[C_NFLIP]), kBlock, 0, c.st>>>(e, lf.p, c.dcnt.p + C_NFLIP, T, c.epoch);
+            ProfScope ps("flip_fix", c.st, n_flip);
+            k_flip_fix<E><<<grid_for(n_flip), kBlock, 0, c.st>>>(e, lf.p, c.round_set(r) + R_FLIP, T, c.epoch);
             GCDT_LAUNCH_CHECK();
         }
     }
@@ -2197,33 +2223,29 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
         if (!act) {  // small mesh: materialise the implicit list
             k_iota<<<grid_for(est), kBlock, 0, c.st>>>(lb.p, est);
             GCDT_LAUNCH_CHECK();
-            k_mark_list<E><<<grid_for(est), kBlock, 0, c.st>>>(e, nullptr, est, (int)ep0);
-            GCDT_LAUNCH_CHECK();
             act = lb.p;
             nxt = la.p;
-            c.set(C_NACT, est);
         } else if (init && act == init) {
             // the tail alternates its two lists: work on a copy of the
-            // caller's list (C_NACT holds ninit already)
+            // caller's list
             GCDT_HIP(hipMemcpyAsync(lb.p, init, sizeof(int) * (size_t)ninit, hipMemcpyDeviceToDevice, c.st));
             act = lb.p;
             nxt = la.p;
-        } else if (r >= 1) {
-            k_flip_begin<<<1, C_NUM, 0, c.st>>>(c.dcnt.p, 1, nullptr, 0u);
-            GCDT_LAUNCH_CHECK();
         }
+        RoundSnap snap = c.round_snap(0);
         {
             ProfScope ps("flip_tail", c.st, est);
-            k_flip_tail<E><<<1, TAIL_BS, 0, c.st>>>(e, (int*)act, nxt, lf.p, c.dcnt.p, T, ep0, 1 << 20);
+            k_flip_tail<E><<<1, TAIL_BS, 0, c.st>>>(e, (int*)act, nxt, lf.p, est, T, ep0, 1 << 20, c.dcnt.p + C_ERR,
+                                                    snap);
             GCDT_LAUNCH_CHECK();
         }
-        c.read(0, C_NUM);
-        if (c.hcnt[C_ERR]) c.check_err();
-        if (c.hcnt[C_TAIL_ERR]) throw Error(GCDT_ERR_INTERNAL, "flip round without progress (tail)");
-        r += c.hcnt[C_TAIL_R];
-        c.epoch += (unsigned)c.hcnt[C_TAIL_R];
-        flips += c.hcnt[C_TAIL_F];
-        if (c.hcnt[C_TAIL_N] != 0) throw Error(GCDT_ERR_NOT_CONVERGED, "flip tail did not converge");
+        const int* h = c.round_wait(0);
+        if (h[C_ERR]) c.check_err();
+        if (h[C_TAIL_ERR]) throw Error(GCDT_ERR_INTERNAL, "flip round without progress (tail)");
+        r += h[C_TAIL_R];
+        c.epoch += (unsigned)h[C_TAIL_R];
+        flips += h[C_TAIL_F];
+        if (h[C_TAIL_N] != 0) throw Error(GCDT_ERR_NOT_CONVERGED, "flip tail did not converge");
     }
     if (rounds) *rounds = r;
     return flips;

@@ -98,16 +98,11 @@ struct DBuf {
 
 // device counters (indices into Ctx::dcnt)
 enum : int {
-    C_NPEND = 0,
-    C_NPEND2 = 1,
-    C_NTRI = 2,
-    C_TBASE = 3,
+    C_NPEND = 0,   // point location: pending points
+    C_NTRI = 2,    // insertion tail: triangles
     C_ERR = 4,
-    C_NACT = 5,
-    C_NACT2 = 6,
-    C_NFLIP = 7,
+    C_NBIGW = 6,   // constraint rounds: winners above CAV_MID_K
     C_TOTAL = 8,   // scan totals
-    C_CONST = 9,   // a constant count for implicit lists
     C_NPIECE = 10,
     C_NQ = 11,
     C_NQ2 = 12,
@@ -117,11 +112,7 @@ enum : int {
     C_TAIL_N = 16,    // persistent tail: remaining list length
     C_TAIL_R = 17,    // rounds done
     C_TAIL_ERR = 18,  // 1 = a round without progress
-    C_TAIL_PAR = 19,  // parity: the final list is the second buffer
     C_TAIL_F = 20,    // flips done
-    C_NPROP = 21,     // proposals of the current flip round
-    C_NW = 22,        // insertion: triangles claimed for the current round
-    C_NW2 = 23,       // insertion: triangles claimed for the next round
     C_STN_T = 24,     // crossing pass: triangles in use
     C_STN_S = 25,     // crossing pass: crossing vertices
     C_HUGE = 26,      // count passes: cells of more elements than one workgroup sorts
@@ -129,9 +120,39 @@ enum : int {
     C_VAL_FIRST = 28, // mesh check: first failing triangle
     C_NLONG = 29,  // constraint rounds: pieces that cross many triangles
     C_PATH = 30,   // constraint rounds: their crossed triangles
-    C_NMID = 31,   // constraint rounds: winners among them, by size
-    C_NBIGW = 6,   // (the flip rounds' C_NACT2: not in use at the same time)
+    C_NMID = 31,   // constraint rounds: the other long winners
     C_NUM = 32
+};
+
+// Counters of the insertion and flip rounds: a ring of ROUND_SETS sets, round r
+// in set r % ROUND_SETS.  A round reads the set of the round before it and
+// appends to its own, which was cleared many rounds ago, so no launch has to
+// move or clear counters between two rounds (a one-wave kernel for it cost
+// 2.5 us and two gaps per round).  Every counter has a 128-byte line to itself:
+// a word that all workgroups read beside one that they add to atomically is
+// read behind those additions, 11 ns each (10M insertion splits 1.0 -> 1.8 ms).
+enum : int {
+    ROUND_LINE = 32,          // ints
+    R_NEXT = 0 * ROUND_LINE,  // length of the list for the next round
+    R_NW = 1 * ROUND_LINE,    // insertion: triangles claimed for the next round
+    R_NEW = 2 * ROUND_LINE,   // insertion: triangles made this round
+    R_BASE = 3 * ROUND_LINE,  // insertion: the first of them
+    R_FLIP = 4 * ROUND_LINE,  // flips: flipped triangles
+    R_PROP = 5 * ROUND_LINE,  // flips: proposals
+    ROUND_WORDS = 6,
+    ROUND_INTS = 8 * ROUND_LINE,  // ints per set
+    ROUND_SETS = 32
+};
+// the same words in a snapshot
+enum : int { S_NEXT = 0, S_NW = 1, S_NEW = 2, S_BASE = 3, S_FLIP = 4, S_PROP = 5, S_ERR = C_NUM - 1 };
+
+// a round's counters on their way to the host ring, copied by the first
+// workgroup of the next round's first kernel (dst null: nothing to copy)
+struct RoundSnap {
+    const int* set = nullptr;
+    const int* err = nullptr;
+    unsigned long long* dst = nullptr;
+    unsigned seq = 0;
 };
 
 // Process-wide defaults of the round tunables (environment variables
@@ -212,6 +233,15 @@ struct Ctx {
     unsigned long long* snap_dst(int slot) const { return hring_dev + C_NUM * slot; }
     unsigned snap_begin(int slot);
     void zero_counters();
+    // the rounds' counter ring: cleared, with the first list's length in set 0
+    // and the first triangle slot in set 1
+    DBuf<int> ring;
+    int* round_set(int r) { return ring.p + ROUND_INTS * (r % ROUND_SETS); }
+    void rounds_start(int next, int base);
+    void rounds_turn(int r);  // before round r is queued: clears sets that come into use later
+    RoundSnap round_snap(int r);
+    const int* round_wait(int r) { return wait_snapshot(r & 1); }
+    void round_snapshot(int r);  // a launch of its own, after the last round
     void check_err();  // throws on a device error flag
     // deferred pool releases of a solve on a non-null stream
     std::vector<PendingFree> deferred;

@@ -130,6 +130,27 @@ __host__ __device__ inline unsigned long long ins_key_of(const Ins& s, int p, in
     return ins_key(p, k < 3, close, epoch);
 }
 
+// The triangle across edge k of t, also while the outer adjacency of a round's
+// splits is being settled (ins_fix, in the same launch): an entry may still
+// name a parent -- marked in a new triangle, plain in an old one -- and the edge
+// has then gone to the parent's child that holds both its vertices.
+__host__ __device__ inline int ins_edge_neighbour(const Ins& s, int t, int k)
+{
+    const Mesh& m = s.m;
+    const int a = A3(m, t, k);
+    if (a == -1) return -1;
+    const int nb = adj_is_mark(a) ? adj_unmark(a) : a;
+    const int sn = m.sons[nb];
+    if (sn == -1) return nb;
+    const int3 tv = m.tri[t];
+    const int u = get3(tv, nx3(k)), v = get3(tv, pv3(k));
+    const int c0 = sn > 0 ? sn : -sn, nc = sn > 0 ? 3 : 2;
+    for (int x = c0; x < c0 + nc; x++)
+        if (has2(m.tri[x], u, v)) return x;
+    at_or(s.err, MERR_ADJ);
+    return -1;
+}
+
 // Computes p's key for this round (cached in pkey) and returns its triangle
 // (the caller performs the claim so a wave can combine claims on one triangle);
 // -1 when p is not pending.  *t2 receives the second triangle of an on-edge
@@ -142,7 +163,7 @@ __host__ __device__ inline int ins_key_round(const Ins& s, int p, unsigned epoch
     int t = l >> 2, k = l & 3;
     *key = ins_key_of(s, p, t, k, epoch);
     s.pkey[p] = *key;
-    if (k < 3) *t2 = A3(s.m, t, k);
+    if (k < 3) *t2 = ins_edge_neighbour(s, t, k);
     return t;
 }
 
