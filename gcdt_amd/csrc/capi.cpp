@@ -66,6 +66,20 @@ struct Timer {
     }
 };
 
+// Host clock of the phases of a solve.  Every phase ends with the host waiting
+// for a counter of its last rounds, so the clock runs with the device but for
+// the launches after it; an event and a wait per phase cost a solve 100 us.
+struct PhaseClock {
+    std::chrono::steady_clock::time_point t = std::chrono::steady_clock::now();
+    double lap()
+    {
+        const auto now = std::chrono::steady_clock::now();
+        const double ms = std::chrono::duration<double, std::milli>(now - t).count();
+        t = now;
+        return ms;
+    }
+};
+
 extern "C" {
 
 const char* gcdt_last_error(void) { return g_last_error.c_str(); }
@@ -275,7 +289,6 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
 {
     gcdt_stats& st = out.st;
     Timer total(c.st);
-    check_points(c, pts_in, N);
     // work in Morton order for locality; ids are mapped back at the end
     DBuf<int2> pts_buf((size_t)N + 4);
     DBuf<int> perm(N > 0 ? N : 1), inv(N > 0 ? N : 1);
@@ -285,11 +298,10 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     morton_order(c, pts_in, N, pts, perm.p, inv.p, cell_end.p);
     relabel_pairs(c, cons_in, C, inv.p, N, cons_buf.p);
     const int2* cons = cons_buf.p;
-    write_corners(c, pts, N);
     // ---- 1. sample + sample mesh
-    Timer t1(c.st);
-    DBuf<int> sid(1 << 16);
-    int S = sample_points_morton(c, pts, cell_end.p, sid.p);
+    PhaseClock phase;
+    DBuf<int> sid(1 << 16), soff((1 << 16) + 1);
+    int S = sample_points_morton(c, pts, cell_end.p, sid.p, soff.p);
     // cell_end stays for the constraints' split pass
     DBuf<int> loc((size_t)N + 4), pend((size_t)(N > 1 ? N : 1)), pend2((size_t)(N > 1 ? N : 1));
     DBuf<unsigned long long> pkey((size_t)N + 4);
@@ -297,10 +309,12 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     DBuf<int3> tA(capA), aA(capA);
     DBuf<int> sA(capA);
     DBuf<unsigned long long> clA(capA);
-    init_square(c, nullptr, tA.p, aA.p, N);
-    fill_i32(c, sA.p, -1, capA);
-    fill_u64(c, clA.p, 0, capA);
-    locate_two_ids(c, pts, sid.p, S, loc.p, pend.p);
+    FillJobs fa;
+    fa.add(sA.p, -1, capA);
+    fa.add(clA.p, 0, 2 * capA);
+    fa.add(c.dcnt.p + C_NPEND, 0, 1);
+    fill_jobs(c, fa);
+    seed_square(c, pts, N, tA.p, aA.p, sid.p, S, loc.p, pend.p);
     Ins ia;
     ia.m = Mesh{pts, tA.p, aA.p, sA.p, nullptr};
     ia.loc = loc.p;
@@ -312,7 +326,7 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     int ntA = insert_rounds(c, ia, pend, pend2, S, 2, &rs);
     long long capB = 4LL * N + 8;
     DBuf<int3> tB(capB), aB(capB);
-    int Ts = filter_leaves_morton(c, pts, tA.p, aA.p, sA.p, ntA, tB.p, aB.p, capB);
+    int Ts = filter_leaves_morton(c, pts, tA.p, aA.p, sA.p, ntA, tB.p, aB.p, 2LL * S + 2);
     tA.release();
     aA.release();
     sA.release();
@@ -321,24 +335,18 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     int fr = 0;
     st.flips += flip_rounds(c, Mesh{pts, tB.p, aB.p, nullptr, nullptr}, Ts, nullptr, 0, &fr);
     validate_mesh(c, "the sample mesh's flips", Mesh{pts, tB.p, aB.p, nullptr, nullptr}, N + 4, Ts, true);
-    st.ms_sample = t1.ms();
-    // ---- 2. bitmap over the sample Delaunay mesh
-    Timer t2(c.st);
-    int *bo = nullptr, *bt = nullptr, nbt = 0;
-    build_bitmap(c, pts, tB.p, Ts, &bo, &bt, &nbt);
-    st.ms_bitmap = t2.ms();
-    // ---- 3. locate + insert the rest
-    Timer t3(c.st);
-    DBuf<int> isv(N > 0 ? N : 1);
-    fill_i32(c, isv.p, 0, N);
-    int np = locate_bitmap(c, pts, N, tB.p, Ts, bo, bt, loc.p, isv.p, pend.p);
-    dev_give(bo, sizeof(int) * ((1 << 20) + 1));
-    dev_give(bt, sizeof(int) * (size_t)(nbt > 0 ? nbt : 1));
-    isv.release();
+    st.ms_sample = phase.lap();
+    // ---- 2. locate the rest, each walking from its own cell's sample
+    int np = locate_walk(c, pts, N, tB.p, aB.p, Ts, sid.p, soff.p, loc.p, pend.p);
+    sid.release();
+    soff.release();
+    // ---- 3. insert them
     DBuf<int> sB(capB);
     DBuf<unsigned long long> clB(capB);
-    fill_i32(c, sB.p, -1, capB);
-    fill_u64(c, clB.p, 0, capB);
+    FillJobs fb;
+    fb.add(sB.p, -1, capB);
+    fb.add(clB.p, 0, 2 * capB);
+    fill_jobs(c, fb);
     Ins ib;
     ib.m = Mesh{pts, tB.p, aB.p, sB.p, nullptr};
     ib.loc = loc.p;
@@ -360,18 +368,15 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     tB.release();
     aB.release();
     sB.release();
-    if (T != 2 * N + 2) throw Error(GCDT_ERR_INTERNAL, "leaf count " + std::to_string(T) + " != 2N+2");
-    st.ms_insert = t3.ms();
+    st.ms_insert = phase.lap();
     // ---- 4. Delaunay flips (unpacked into tris_out / adj_out)
-    Timer t4(c.st);
     int f2 = 0;
     st.flips += flip_rounds_records(c, rec.p, Mesh{pts, tris_out, adj_out, nullptr, nullptr}, T, &f2);
     validate_mesh(c, "the flips", Mesh{pts, tris_out, adj_out, nullptr, nullptr}, N + 4, T, true);
     rec.release();
     st.flip_rounds = fr + f2;
-    st.ms_flip = t4.ms();
+    st.ms_flip = phase.lap();
     // ---- 5. constraints
-    Timer t5(c.st);
     if (cflag_out) fill_i32(c, cflag_out, 0, T);
     if (C > 0) {
         DBuf<int> cflag_buf, touched(T);
@@ -407,8 +412,8 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
         }
     }
     unmap_tris(c, tris_out, T, perm.p, N);
-    st.ms_constraints = t5.ms();
     st.ms_total = total.ms();
+    st.ms_constraints = phase.lap();
     st.num_triangles = T;
     out.T = T;
 }
@@ -845,16 +850,18 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     batch_order(c, (const int2*)points, vinst.p, d_cbase.p, d_lvl.p, NP, ncells, pts.p, perm.p, inv.p, cell_end.p);
     // ---- 1. sample meshes: one point per (instance, 16x16 cell), inserted from
     //         every instance's two seed triangles, then made Delaunay
-    Timer t1(c.st);
+    PhaseClock phase;
     long long capA = 2LL * K + 4LL * std::min<long long>(NP, (long long)K << 8) + 8;
     DBuf<int> sid(std::max<long long>(1, std::min<long long>(NP, (long long)K << 8)));
     int S = batch_sample_sorted(c, d_cbase.p, d_lvl.p, cell_end.p, K, sid.p);
-    cell_end.release();
     DBuf<int3> tA(capA), aA(capA);
     DBuf<int> sA(capA), loc(nv), pend(NP > 0 ? NP : 1), pend2(NP > 0 ? NP : 1);
     DBuf<unsigned long long> clA(capA), pkey(nv);
-    fill_i32(c, sA.p, -1, capA);
-    fill_u64(c, clA.p, 0, capA);
+    FillJobs fa;
+    fa.add(sA.p, -1, capA);
+    fa.add(clA.p, 0, 2 * capA);
+    fa.add(c.dcnt.p + C_NPEND, 0, 1);
+    fill_jobs(c, fa);
     batch_init(c, pts.p, tA.p, aA.p, K, NP);
     batch_locate_ids(c, pts.p, vinst.p, sid.p, S, loc.p, pend.p);
     sid.release();
@@ -871,7 +878,7 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     if (capB > (1LL << 31) - 1) throw Error(GCDT_ERR_INVALID, "batch too large");
     DBuf<int3> tB(capB), aB(capB);
     int Ts = filter_leaves_inst(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, ncells, NP, tA.p, aA.p, sA.p, ntA, tB.p,
-                                aB.p, capB);
+                                aB.p, 2LL * S + 2LL * K);
     tA.release();
     aA.release();
     sA.release();
@@ -880,20 +887,16 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     int fr = 0;
     bs.flips += flip_rounds(c, Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, Ts, nullptr, 0, &fr);
     validate_mesh(c, "the sample meshes' flips", Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, nv, Ts, true);
-    // ---- 2. locate the other points through a per-instance bitmap of the
-    //         sample meshes, then insert them
-    int *bo = nullptr, *bt = nullptr, nbt = 0;
-    build_bitmap_batch(c, pts.p, vinst.p, NP, K, tB.p, Ts, &bo, &bt, &nbt);
-    DBuf<int> isv(NP > 0 ? NP : 1);
-    fill_i32(c, isv.p, 0, NP);
-    int np = locate_bitmap_batch(c, pts.p, vinst.p, NP, tB.p, Ts, bo, bt, loc.p, isv.p, pend.p);
-    dev_give(bo, sizeof(int) * (size_t)(((long long)K << 8) + 1));
-    dev_give(bt, sizeof(int) * (size_t)(nbt > 0 ? nbt : 1));
-    isv.release();
+    // ---- 2. locate the other points, each walking from its own cell's sample,
+    //         then insert them
+    int np = locate_walk_batch(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, cell_end.p, NP, K, tB.p, aB.p, Ts, loc.p, pend.p);
+    cell_end.release();
     DBuf<int> sB(capB);
     DBuf<unsigned long long> clB(capB);
-    fill_i32(c, sB.p, -1, capB);
-    fill_u64(c, clB.p, 0, capB);
+    FillJobs fb;
+    fb.add(sB.p, -1, capB);
+    fb.add(clB.p, 0, 2 * capB);
+    fill_jobs(c, fb);
     Ins s2;
     s2.m = Mesh{pts.p, tB.p, aB.p, sB.p, nullptr};
     s2.loc = loc.p;
@@ -916,19 +919,16 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     aB.release();
     sB.release();
     DBuf<int3> tri(Tn), adj(Tn);  // after the insertion DAG is gone: a lower peak
-    if (T != Tn) throw Error(GCDT_ERR_INTERNAL, "batch leaf count mismatch");
-    bs.ms_insert = t1.ms();
+    bs.ms_insert = phase.lap();
     bs.insert_rounds = ri + ri2;
     // ---- Delaunay flips of all instances together (unpacked into tri / adj)
-    Timer t2(c.st);
     int fr2 = 0;
     bs.flips += flip_rounds_records(c, rec.p, Mesh{pts.p, tri.p, adj.p, nullptr, nullptr}, T, &fr2);
     validate_mesh(c, "the flips", Mesh{pts.p, tri.p, adj.p, nullptr, nullptr}, nv, T, true);
     rec.release();
     bs.flip_rounds = fr + fr2;
-    bs.ms_flip = t2.ms();
+    bs.ms_flip = phase.lap();
     // ---- constraints
-    Timer t3(c.st);
     if (NC > 0) {
         DBuf<int2> cg(NC);
         batch_cons(c, (const int2*)cons, d_coff.p, d_poff.p, K, NC, cg.p);
@@ -948,7 +948,7 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
         }
         validate_mesh(c, "the constraints", m, nv, T, true);
     }
-    bs.ms_constraints = t3.ms();
+    bs.ms_constraints = phase.lap();
     batch_out(c, tri.p, T, vinst.p, perm.p, d_poff.p, d_toff.p, NP, K, (int3*)tris_out);
     bs.ms_total = total.ms();
     bs.num_instances = K;

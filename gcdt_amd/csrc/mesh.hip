@@ -293,10 +293,13 @@ void Ctx::round_snapshot(int r)
     GCDT_LAUNCH_CHECK();
 }
 
+// through the mapped ring and a poll: a copy and a stream synchronisation cost
+// the host 15-20 us, this 8
 void Ctx::read(int i, int k)
 {
-    GCDT_HIP(hipMemcpyAsync(hcnt + i, dcnt.p + i, sizeof(int) * k, hipMemcpyDeviceToHost, st));
-    GCDT_HIP(hipStreamSynchronize(st));
+    snapshot(0);
+    const int* h = wait_snapshot(0);
+    for (int j = i; j < i + k; j++) hcnt[j] = h[j];
 }
 
 __global__ void k_set1(int* p, int v) { *p = v; }
@@ -486,6 +489,29 @@ void fill_u64(Ctx& c, unsigned long long* p, unsigned long long v, long long n)
     GCDT_LAUNCH_CHECK();
 }
 
+__global__ __launch_bounds__(kBlock) void k_fill_jobs(FillJobs f)
+{
+    const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
+    for (int j = 0; j < f.njobs; j++) {
+        int* p = f.job[j].p;
+        const long long n = f.job[j].n;
+        const int v = f.job[j].v;
+        const bool wide = ((unsigned long long)p & 15) == 0;  // buffers start 256-byte aligned, counters need not
+        const long long n4 = wide ? n / 4 : 0;
+        for (long long i = i0; i < n4; i += step) ((int4*)p)[i] = make_int4(v, v, v, v);
+        for (long long i = 4 * n4 + i0; i < n; i += step) p[i] = v;
+    }
+}
+
+void fill_jobs(Ctx& c, const FillJobs& f)
+{
+    long long most = 0;
+    for (int j = 0; j < f.njobs; j++) most = std::max(most, f.job[j].n);
+    if (most == 0) return;
+    k_fill_jobs<<<grid_for((most + 3) / 4), kBlock, 0, c.st>>>(f);
+    GCDT_LAUNCH_CHECK();
+}
+
 constexpr int SCAN_ITEMS = 16;
 constexpr int SCAN_TILE = kBlock * SCAN_ITEMS;
 constexpr int SCAN_PAD(int i) { return i + (i >> 4); }
@@ -555,11 +581,30 @@ __global__ __launch_bounds__(1024) void k_scan_sums(int* sums, int nt, int* tota
     }
 }
 
-template <bool INCL>
-__global__ __launch_bounds__(kBlock) void k_scan_apply(const int* in, int* out, long long n, const int* sums)
+// OWN: sums[] holds the tiles' own totals and each workgroup adds up those
+// before it (and the last one writes the grand total); else sums[] is scanned.
+template <bool INCL, bool OWN>
+__global__ __launch_bounds__(kBlock) void k_scan_apply(const int* in, int* out, long long n, const int* sums, int* total,
+                                                       int* total2)
 {
     __shared__ int tile[SCAN_PAD(SCAN_TILE)];
+    __shared__ int s_pre;
     long long base = (long long)blockIdx.x * SCAN_TILE;
+    if (OWN) {
+        int v = 0, tot;
+        for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlock) v += sums[i];
+        block_excl_scan(v, tot);
+        if (threadIdx.x == 0) {
+            s_pre = tot;
+            if (blockIdx.x == gridDim.x - 1) {
+                if (total) *total = tot + sums[blockIdx.x];
+                if (total2) *total2 = tot + sums[blockIdx.x];
+            }
+        }
+        __syncthreads();
+    } else if (threadIdx.x == 0) {
+        s_pre = sums[blockIdx.x];
+    }
 #pragma unroll
     for (int j = 0; j < SCAN_ITEMS; j++) {
         int li = j * kBlock + threadIdx.x;
@@ -575,7 +620,8 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(const int* in, int* out, 
         s += v[j];
     }
     int tot;
-    int run = sums[blockIdx.x] + block_excl_scan(s, tot);
+    const int pre = block_excl_scan(s, tot);  // its barriers order s_pre too
+    int run = s_pre + pre;
 #pragma unroll
     for (int j = 0; j < SCAN_ITEMS; j++) {
         run += INCL ? v[j] : 0;
@@ -588,6 +634,45 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(const int* in, int* out, 
         int li = j * kBlock + threadIdx.x;
         long long i = base + li;
         if (i < n) out[i] = tile[SCAN_PAD(li)];
+    }
+}
+
+// A whole scan of up to SCAN_ONE ints in one workgroup.
+constexpr int SCAN_ONE = 16384;
+
+template <bool INCL>
+__global__ __launch_bounds__(1024) void k_scan_one(const int* in, int* out, int n, int* total, int* total2)
+{
+    __shared__ int wsum[16];
+    int carry = 0;
+    for (int base = 0; base < n; base += 4096) {
+        const int i = base + 4 * (int)threadIdx.x;
+        int v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = i + j < n ? in[i + j] : 0;
+        int wt;
+        const int sum = v[0] + v[1] + v[2] + v[3];
+        const int ex = wave_excl_scan(sum, wt);
+        if (__lane_id() == 0) wsum[threadIdx.x >> 6] = wt;
+        __syncthreads();
+        int pre = 0, tot = 0;
+        for (int q = 0; q < 16; q++) {
+            if (q < (int)(threadIdx.x >> 6)) pre += wsum[q];
+            tot += wsum[q];
+        }
+        int run = carry + pre + ex;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            run += INCL ? v[j] : 0;
+            if (i + j < n) out[i + j] = run;
+            run += INCL ? 0 : v[j];
+        }
+        carry += tot;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        if (total) *total = carry;
+        if (total2) *total2 = carry;
     }
 }
 
@@ -606,6 +691,7 @@ static void scan_impl(Ctx& c, const int* in, int* out, long long n, bool total_a
         }
         return;
     }
+    int *total = c.dcnt.p + C_TOTAL, *total2 = total_at_end ? out + n : nullptr;
     long long nt = (n + SCAN_TILE - 1) / SCAN_TILE;
     int* sums;
     if (c.ext_scratch) {
@@ -616,14 +702,32 @@ static void scan_impl(Ctx& c, const int* in, int* out, long long n, bool total_a
         c.scan_sums.ensure((size_t)nt + 1);
         sums = c.scan_sums.p;
     }
+    // one launch up to SCAN_ONE ints; two up to 4,096 tiles, whose totals every
+    // workgroup can add up itself; else a launch between them for the totals
+    if (n <= SCAN_ONE) {
+        if (incl)
+            k_scan_one<true><<<1, 1024, 0, c.st>>>(in, out, (int)n, total, total2);
+        else
+            k_scan_one<false><<<1, 1024, 0, c.st>>>(in, out, (int)n, total, total2);
+        GCDT_LAUNCH_CHECK();
+        return;
+    }
     k_scan_tile_sums<<<(unsigned)nt, kBlock, 0, c.st>>>(in, n, sums);
     GCDT_LAUNCH_CHECK();
-    k_scan_sums<<<1, 1024, 0, c.st>>>(sums, (int)nt, c.dcnt.p + C_TOTAL, total_at_end ? out + n : nullptr);
+    if (nt <= 4096) {
+        if (incl)
+            k_scan_apply<true, true><<<(unsigned)nt, kBlock, 0, c.st>>>(in, out, n, sums, total, total2);
+        else
+            k_scan_apply<false, true><<<(unsigned)nt, kBlock, 0, c.st>>>(in, out, n, sums, total, total2);
+        GCDT_LAUNCH_CHECK();
+        return;
+    }
+    k_scan_sums<<<1, 1024, 0, c.st>>>(sums, (int)nt, total, total2);
     GCDT_LAUNCH_CHECK();
     if (incl)
-        k_scan_apply<true><<<(unsigned)nt, kBlock, 0, c.st>>>(in, out, n, sums);
+        k_scan_apply<true, false><<<(unsigned)nt, kBlock, 0, c.st>>>(in, out, n, sums, nullptr, nullptr);
     else
-        k_scan_apply<false><<<(unsigned)nt, kBlock, 0, c.st>>>(in, out, n, sums);
+        k_scan_apply<false, false><<<(unsigned)nt, kBlock, 0, c.st>>>(in, out, n, sums, nullptr, nullptr);
     GCDT_LAUNCH_CHECK();
 }
 
@@ -635,31 +739,35 @@ void scan_excl_total(Ctx& c, const int* in, int* out, long long n) { scan_impl(c
 
 constexpr int GRID_R = (1 << 30) - 1;
 
+__device__ inline void square_corners(int2* pts, int n)
+{
+    pts[n] = make_int2(0, 0);
+    pts[n + 1] = make_int2(GRID_R, 0);
+    pts[n + 2] = make_int2(GRID_R, GRID_R);
+    pts[n + 3] = make_int2(0, GRID_R);
+}
+
+// rawMesh.cu:16-21: (N,N+1,N+3) and (N+1,N+2,N+3) split along the anti-diagonal
+__device__ inline void square_seeds(int3* tri, int3* adj, int n)
+{
+    tri[0] = make_int3(n, n + 1, n + 3);
+    tri[1] = make_int3(n + 1, n + 2, n + 3);
+    adj[0] = make_int3(1, -1, -1);
+    adj[1] = make_int3(-1, 0, -1);
+}
+
 __global__ void k_init_square(int2* pts, int3* tri, int3* adj, int n)
 {
-    if (pts) {
-        pts[n] = make_int2(0, 0);
-        pts[n + 1] = make_int2(GRID_R, 0);
-        pts[n + 2] = make_int2(GRID_R, GRID_R);
-        pts[n + 3] = make_int2(0, GRID_R);
-    }
-    // rawMesh.cu:16-21: (N,N+1,N+3) and (N+1,N+2,N+3) split along the anti-diagonal
-    if (tri) {
-        tri[0] = make_int3(n, n + 1, n + 3);
-        tri[1] = make_int3(n + 1, n + 2, n + 3);
-    }
-    if (adj) {
-        adj[0] = make_int3(1, -1, -1);
-        adj[1] = make_int3(-1, 0, -1);
-    }
+    square_corners(pts, n);
+    square_seeds(tri, adj, n);
 }
+
+__device__ inline bool point_inside(int2 p) { return p.x > 0 && p.y > 0 && p.x < GRID_R && p.y < GRID_R; }
 
 __global__ __launch_bounds__(kBlock) void k_check_points(const int2* pts, int n, int* err)
 {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-        int2 p = pts[i];
-        if (p.x <= 0 || p.y <= 0 || p.x >= GRID_R || p.y >= GRID_R) atomicOr(err, MERR_INVALID);
-    }
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+        if (!point_inside(pts[i])) atomicOr(err, MERR_INVALID);
 }
 
 void check_points(Ctx& c, const int2* pts, int n)
@@ -676,13 +784,7 @@ void init_square(Ctx& c, int2* pts, int3* tri, int3* adj, int n)
     GCDT_LAUNCH_CHECK();
 }
 
-__global__ void k_write_corners(int2* pts, int n)
-{
-    pts[n] = make_int2(0, 0);
-    pts[n + 1] = make_int2(GRID_R, 0);
-    pts[n + 2] = make_int2(GRID_R, GRID_R);
-    pts[n + 3] = make_int2(0, GRID_R);
-}
+__global__ void k_write_corners(int2* pts, int n) { square_corners(pts, n); }
 
 void write_corners(Ctx& c, int2* pts, int n)
 {
@@ -695,23 +797,13 @@ constexpr int LOG_BITMAP = 10;  // math_base.cuh:25 logBitmap
 constexpr int SAMPLE_CELLS = 1 << (2 * LOG_SAMPLE);
 constexpr int BITMAP_CELLS = 1 << (2 * LOG_BITMAP);
 
-// Cell grids of the point-location bitmap ("boostmap").  GridOne: one mesh,
-// 1024x1024 cells over the square (math_base.cuh:25 logBitmap).  GridInst:
-// a batch of instances that all span the square, each with its own 16x16
-// cells; a cell id is instance * 256 + local cell.
+// Cell grid of the point-location bitmap ("boostmap") that the reference's entry
+// points build and read: 1024x1024 cells over the square (math_base.cuh:25
+// logBitmap).
 struct GridOne {
     static constexpr int LOG = LOG_BITMAP;
     __device__ long long tri_base(const int3&) const { return 0; }
     __device__ long long pt_base(int) const { return 0; }
-};
-
-struct GridInst {
-    static constexpr int LOG = 4;
-    const int* vinst;
-    long long NP;  // corners of instance i are NP + 4i .. NP + 4i + 3
-    __device__ int inst_of(int v) const { return v < NP ? vinst[v] : (int)((v - NP) >> 2); }
-    __device__ long long tri_base(const int3& t) const { return (long long)inst_of(t.x) << (2 * LOG); }
-    __device__ long long pt_base(int p) const { return (long long)vinst[p] << (2 * LOG); }
 };
 
 template <class G>
@@ -1110,20 +1202,32 @@ static void cell_reorder_huge(Ctx& c, const KF& kf, const int* end, const typena
     GCDT_LAUNCH_CHECK();
 }
 
+// What the count passes leave in C_HUGE: buckets of more than CELL_RANK_MAX
+// elements, plus CELL_HUGE for each of more than CELL_BLOCK_MAX (so many of the
+// former that they reach CELL_HUGE only cost the larger path an empty scan).
+constexpr int CELL_HUGE = 1 << 20;
+__device__ inline void count_large(int r, int* huge)
+{
+    if (r == CELL_RANK_MAX) atomicAdd(huge, 1);
+    if (r == CELL_BLOCK_MAX) atomicAdd(huge, CELL_HUGE);
+}
+
 // eb[0..n): (element, bucket, ...), grouped by bucket.  Each element is
-// placed (KF::put) at its position in the reordered order.  huge: some bucket
-// holds more than CELL_BLOCK_MAX elements.
+// placed (KF::put) at its position in the reordered order.  large: C_HUGE of
+// the count pass; C_NQ was cleared before it.
 template <class KF>
-static void cell_reorder(Ctx& c, const KF& kf, const int* end, const typename KF::Slot* eb, long long n, bool huge)
+static void cell_reorder(Ctx& c, const KF& kf, const int* end, const typename KF::Slot* eb, long long n, int large)
 {
     if (n <= 0) return;
+    const bool huge = large >= CELL_HUGE;
     // a list entry per bucket above the rank cap: at most n / (cap + 1)
     DBuf<int> big((size_t)(n / (CELL_RANK_MAX + 1) + 1));
-    c.set(C_NQ, 0);
     k_cell_rank<KF><<<grid_for(n), kBlock, 0, c.st>>>(kf, end, eb, n, big.p, c.dcnt.p + C_NQ);
     GCDT_LAUNCH_CHECK();
-    k_cell_sort_block<KF><<<1024, kBlock, 0, c.st>>>(kf, end, big.p, c.dcnt.p + C_NQ, eb);
-    GCDT_LAUNCH_CHECK();
+    if (large) {
+        k_cell_sort_block<KF><<<1024, kBlock, 0, c.st>>>(kf, end, big.p, c.dcnt.p + C_NQ, eb);
+        GCDT_LAUNCH_CHECK();
+    }
     if (huge) cell_reorder_huge(c, kf, end, eb, n);
 }
 
@@ -1132,12 +1236,18 @@ static void cell_reorder(Ctx& c, const KF& kf, const int* end, const typename KF
 // inv[], the scatter writes (index, cell, x, y) at the cell's start plus that
 // rank, and the per-cell reorder places each point by input index, writing
 // the sorted points, perm and the inverse map.
-__global__ __launch_bounds__(kBlock) void k_morton_count(const int2* pts, int n, int* cnt, int* rank, int* huge)
+// Points outside the square are flagged here and land in some cell (the caller
+// fails before they are used).
+__device__ inline int morton_cell_any(int2 p) { return (int)(morton_cell(p) & (BITMAP_CELLS - 1)); }
+
+__global__ __launch_bounds__(kBlock) void k_morton_count(const int2* pts, int n, int* cnt, int* rank, int* huge, int* err)
 {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-        const int r = atomicAdd(&cnt[morton_cell(pts[i])], 1);
+        const int2 p = pts[i];
+        if (!point_inside(p)) atomicOr(err, MERR_INVALID);
+        const int r = atomicAdd(&cnt[morton_cell_any(p)], 1);
         rank[i] = r;
-        if (r == CELL_BLOCK_MAX) atomicAdd(huge, 1);
+        count_large(r, huge);
     }
 }
 
@@ -1148,7 +1258,7 @@ __global__ __launch_bounds__(kBlock) void k_morton_scatter(const int2* pts, int 
 {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         const int2 p = pts[i];
-        const int cell = (int)morton_cell(p);
+        const int cell = morton_cell_any(p);
         const int pos = (cell ? cell_end[cell - 1] : 0) + rank[i];
         eb[pos] = make_int4((int)i, cell, p.x, p.y);
     }
@@ -1156,17 +1266,22 @@ __global__ __launch_bounds__(kBlock) void k_morton_scatter(const int2* pts, int 
 
 void morton_order(Ctx& c, const int2* pts, int n, int2* out, int* perm, int* inv, int* cell_end)
 {
-    fill_i32(c, cell_end, 0, BITMAP_CELLS + 1);
+    FillJobs f;
+    f.add(cell_end, 0, BITMAP_CELLS + 1);
+    f.add(c.dcnt.p + C_HUGE, 0, 1);
+    f.add(c.dcnt.p + C_NQ, 0, 1);
+    fill_jobs(c, f);
     if (n <= 0) return;
-    c.set(C_HUGE, 0);
-    k_morton_count<<<grid_for(n), kBlock, 0, c.st>>>(pts, n, cell_end, inv, c.dcnt.p + C_HUGE);
+    k_morton_count<<<grid_for(n), kBlock, 0, c.st>>>(pts, n, cell_end, inv, c.dcnt.p + C_HUGE, c.dcnt.p + C_ERR);
     GCDT_LAUNCH_CHECK();
     scan_incl(c, cell_end, cell_end, BITMAP_CELLS);
     DBuf<int4> eb((size_t)n);
     k_morton_scatter<<<grid_for(n), kBlock, 0, c.st>>>(pts, n, cell_end, inv, eb.p);
     GCDT_LAUNCH_CHECK();
+    c.read(0, C_NUM);
+    if (c.hcnt[C_ERR]) c.check_err();
     // inv held the arrival ranks; placing rewrites it as the inverse map
-    cell_reorder(c, CellKeyPoint{pts, perm, out, inv}, cell_end, eb.p, n, c.get(C_HUGE) > 0);
+    cell_reorder(c, CellKeyPoint{pts, perm, out, inv}, cell_end, eb.p, n, c.hcnt[C_HUGE]);
 }
 
 // Sample of Morton-ordered points: the 256x256 sample cell with Morton index
@@ -1230,14 +1345,13 @@ __global__ __launch_bounds__(kBlock) void k_sample_morton_emit(const int2* pts, 
     }
 }
 
-int sample_points_morton(Ctx& c, const int2* pts, const int* cell_end, int* sample_ids)
+int sample_points_morton(Ctx& c, const int2* pts, const int* cell_end, int* sample_ids, int* offs)
 {
-    DBuf<int> offs(SAMPLE_CELLS + 1);
-    k_sample_morton_flags<<<grid_for(SAMPLE_CELLS), kBlock, 0, c.st>>>(cell_end, offs.p);
+    k_sample_morton_flags<<<grid_for(SAMPLE_CELLS), kBlock, 0, c.st>>>(cell_end, offs);
     GCDT_LAUNCH_CHECK();
-    scan_excl(c, offs.p, offs.p, SAMPLE_CELLS);
+    scan_excl(c, offs, offs, SAMPLE_CELLS);
     // one wave per sample cell
-    k_sample_morton_emit<<<grid_for(64LL * SAMPLE_CELLS), kBlock, 0, c.st>>>(pts, cell_end, offs.p, sample_ids);
+    k_sample_morton_emit<<<grid_for(64LL * SAMPLE_CELLS), kBlock, 0, c.st>>>(pts, cell_end, offs, sample_ids);
     GCDT_LAUNCH_CHECK();
     return c.get(C_TOTAL);
 }
@@ -1290,9 +1404,14 @@ __global__ __launch_bounds__(kBlock) void k_locate_two(const int2* pts, int n, i
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_locate_two_ids(const int2* pts, const int* ids, int n, int* loc, int* pend)
+__global__ __launch_bounds__(kBlock) void k_seed_square(int2* pts, int n, int3* tri, int3* adj, const int* ids, int nids,
+                                                        int* loc, int* pend)
 {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        square_corners(pts, n);
+        square_seeds(tri, adj, n);
+    }
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nids; i += (long long)gridDim.x * blockDim.x) {
         int p = ids[i];
         int o = orient2d(make_int2(GRID_R, 0), make_int2(0, GRID_R), pts[p]);
         loc[p] = o > 0 ? 3 : (o < 0 ? 4 + 3 : 0);
@@ -1300,13 +1419,10 @@ __global__ __launch_bounds__(kBlock) void k_locate_two_ids(const int2* pts, cons
     }
 }
 
-int locate_two_ids(Ctx& c, const int2* pts, const int* ids, int n, int* loc, int* pend)
+void seed_square(Ctx& c, int2* pts, int n, int3* tri, int3* adj, const int* ids, int nids, int* loc, int* pend)
 {
-    if (n > 0) {
-        k_locate_two_ids<<<grid_for(n), kBlock, 0, c.st>>>(pts, ids, n, loc, pend);
-        GCDT_LAUNCH_CHECK();
-    }
-    return n;
+    k_seed_square<<<grid_for(nids), kBlock, 0, c.st>>>(pts, n, tri, adj, ids, nids, loc, pend);
+    GCDT_LAUNCH_CHECK();
 }
 
 int locate_two(Ctx& c, const int2* pts, int n, int* loc, int* pend)
@@ -1384,8 +1500,9 @@ static int locate_bitmap_g(Ctx& c, const G& g, const int2* pts, int n, const int
                                                              c.dcnt.p + C_NPEND, c.dcnt.p + C_ERR);
         GCDT_LAUNCH_CHECK();
     }
-    c.check_err();
-    return c.get(C_NPEND);
+    c.read(0, C_NUM);
+    if (c.hcnt[C_ERR]) c.check_err();
+    return c.hcnt[C_NPEND];
 }
 
 int locate_bitmap(Ctx& c, const int2* pts, int n, const int3* tri, int T, const int* bm_off, const int* bm_tri,
@@ -1394,10 +1511,109 @@ int locate_bitmap(Ctx& c, const int2* pts, int n, const int3* tri, int T, const 
     return locate_bitmap_g(c, GridOne{}, pts, n, tri, T, bm_off, bm_tri, loc, isv, pend);
 }
 
-int locate_bitmap_batch(Ctx& c, const int2* pts, const int* vinst, long long NP, const int3* tri, int T,
-                        const int* bm_off, const int* bm_tri, int* loc, int* isv, int* pend)
+// vertex -> a triangle of the mesh that has it (set for the mesh's vertices only)
+__global__ __launch_bounds__(kBlock) void k_vertex_tri(const int3* tri, int T, int* vt)
 {
-    return locate_bitmap_g(c, GridInst{vinst, NP}, pts, (int)NP, tri, T, bm_off, bm_tri, loc, isv, pend);
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < T; i += (long long)gridDim.x * blockDim.x) {
+        const int3 t = tri[i];
+        vt[t.x] = (int)i;
+        vt[t.y] = (int)i;
+        vt[t.z] = (int)i;
+    }
+}
+
+// The sample of a point's own cell: of the whole square (sample_points_morton),
+// or the first point of the instance's 16x16 cell (batch_sample_sorted).
+struct CellSampleOne {
+    const int *ids, *offs;
+    __device__ int of(int, int2 P) const { return ids[offs[morton_cell(P) >> (2 * (LOG_BITMAP - LOG_SAMPLE))]]; }
+};
+
+struct CellSampleInst {
+    const int *vinst, *cbase, *lvl, *cell_end;
+    __device__ int of(int p, int2 P) const
+    {
+        const int inst = vinst[p], sh = 2 * (lvl[inst] - 4);
+        const int f0 = cbase[inst] + ((int)(morton_cell(P) >> 12) << sh);  // 4 of 10 levels
+        return f0 ? cell_end[f0 - 1] : 0;
+    }
+};
+
+// A thread per point: from its cell's sample, across any edge that has the
+// point strictly outside, to the triangle whose closed region holds it (on a
+// Delaunay mesh such a walk ends).  Which of an edge's two triangles a point
+// on it is recorded in does not matter (closeness_rank_edge).  Bound by the
+// chain of loads: two per triangle, mostly in L2 (the sample mesh has at most
+// 131k triangles).
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_locate_walk(S smp, const int2* pts, int n, const int3* tri, const int3* adj,
+                                                        int T, const int* vt, int* loc, int* pend, int* npend, int* err)
+{
+    __shared__ int s_buf[STAGE_CAP];
+    __shared__ int s_base;
+    Staged<STAGE_CAP> sp(s_buf, &s_base, pend, npend);
+    TILE_LOOP(base, n, kBlock)
+    {
+        const long long i = base + threadIdx.x;
+        bool want = false;
+        if (i < n) {
+            const int p = (int)i;
+            const int2 P = pts[p];
+            const int v = smp.of(p, P);
+            int r = -1, t = vt[v];
+            if (v != p) {
+                for (int g = 0; g < T && t >= 0; g++) {
+                    const int3 tv = tri[t], ta = adj[t];
+                    const int2 A = pts[tv.x], B = pts[tv.y], C = pts[tv.z];
+                    const int o0 = orient2d(B, C, P), o1 = orient2d(C, A, P), o2 = orient2d(A, B, P);
+                    if (o0 >= 0 && o1 >= 0 && o2 >= 0) {
+                        const int z = (o0 == 0) + (o1 == 0) + (o2 == 0);
+                        r = z == 0 ? 3 : (z > 1 ? -2 : (o0 == 0 ? 0 : (o1 == 0 ? 1 : 2)));
+                        break;
+                    }
+                    t = o0 < 0 ? ta.x : (o1 < 0 ? ta.y : ta.z);
+                }
+                want = r >= 0;
+                if (!want) atomicOr(err, r == -2 ? MERR_DUPLICATE : MERR_LOCATE);
+            }
+            loc[p] = want ? t * 4 + r : -1;
+        }
+        const int slot = sp.reserve(want ? 1 : 0);
+        if (want) s_buf[slot] = (int)i;
+    }
+    sp.flush();
+}
+
+template <class S>
+static int locate_walk_s(Ctx& c, const S& smp, const int2* pts, int n, long long nv, const int3* tri, const int3* adj,
+                         int T, int* loc, int* pend)
+{
+    if (n <= 0) return 0;
+    DBuf<int> vt((size_t)nv);
+    k_vertex_tri<<<grid_for(T), kBlock, 0, c.st>>>(tri, T, vt.p);
+    GCDT_LAUNCH_CHECK();
+    {
+        ProfScope ps("locate_walk", c.st, n);
+        k_locate_walk<S><<<grid_for(n), kBlock, 0, c.st>>>(smp, pts, n, tri, adj, T, vt.p, loc, pend, c.dcnt.p + C_NPEND,
+                                                           c.dcnt.p + C_ERR);
+        GCDT_LAUNCH_CHECK();
+    }
+    c.read(0, C_NUM);
+    if (c.hcnt[C_ERR]) c.check_err();
+    return c.hcnt[C_NPEND];
+}
+
+int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const int3* adj, int T, const int* ids,
+                const int* offs, int* loc, int* pend)
+{
+    return locate_walk_s(c, CellSampleOne{ids, offs}, pts, n, (long long)n + 4, tri, adj, T, loc, pend);
+}
+
+int locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
+                      long long NP, int K, const int3* tri, const int3* adj, int T, int* loc, int* pend)
+{
+    return locate_walk_s(c, CellSampleInst{vinst, cbase, lvl, cell_end}, pts, (int)NP, NP + 4LL * K, tri, adj, T, loc,
+                         pend);
 }
 
 // ================================================================== insertion rounds
@@ -2287,10 +2503,12 @@ long long flip_rounds(Ctx& c, const Mesh& m, int T, const int* init, int ninit, 
         return flip_rounds_records(c, rec.p, m, T, rounds);
     }
     DBuf<unsigned long long> claim(T);
-    fill_u64(c, claim.p, 0, T);
     DBuf<int> stamp(T), partner(T), cand(T), mark(T);
-    fill_i32(c, stamp.p, 0, T);
-    fill_i32(c, mark.p, 0, T);
+    FillJobs f;
+    f.add(claim.p, 0, 2LL * T);
+    f.add(stamp.p, 0, T);
+    f.add(mark.p, 0, T);
+    fill_jobs(c, f);
     EngSoA e;
     e.f.m = m;
     e.f.claim = claim.p;
@@ -2430,7 +2648,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_cell_count(BatchCells b, const
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < NP; i += (long long)gridDim.x * blockDim.x) {
         const int r = atomicAdd(&cnt[b.cell((int)i, pts[i])], 1);
         rank[i] = r;
-        if (r == CELL_BLOCK_MAX) atomicAdd(huge, 1);
+        count_large(r, huge);
     }
 }
 
@@ -2448,17 +2666,20 @@ __global__ __launch_bounds__(kBlock) void k_batch_cell_scatter(BatchCells b, con
 void batch_order(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, long long NP,
                  long long ncells, int2* out, int* perm, int* inv, int* cell_end)
 {
-    fill_i32(c, cell_end, 0, ncells + 1);
+    FillJobs f;
+    f.add(cell_end, 0, ncells + 1);
+    f.add(c.dcnt.p + C_HUGE, 0, 1);
+    f.add(c.dcnt.p + C_NQ, 0, 1);
+    fill_jobs(c, f);
     if (NP <= 0) return;
     BatchCells b{vinst, cbase, lvl};
-    c.set(C_HUGE, 0);
     k_batch_cell_count<<<grid_for(NP), kBlock, 0, c.st>>>(b, pts, NP, cell_end, inv, c.dcnt.p + C_HUGE);
     GCDT_LAUNCH_CHECK();
     scan_incl(c, cell_end, cell_end, ncells);
     DBuf<int4> eb((size_t)NP);
     k_batch_cell_scatter<<<grid_for(NP), kBlock, 0, c.st>>>(b, pts, NP, cell_end, inv, eb.p);
     GCDT_LAUNCH_CHECK();
-    cell_reorder(c, CellKeyPoint{pts, perm, out, inv}, cell_end, eb.p, NP, c.get(C_HUGE) > 0);
+    cell_reorder(c, CellKeyPoint{pts, perm, out, inv}, cell_end, eb.p, NP, c.get(C_HUGE));
 }
 
 // Sorted range of 16x16 cell c (Morton index) of instance i: the fine cells
@@ -2694,8 +2915,51 @@ __device__ inline unsigned morton_cell_leaf(int2 p)
     for (int b = 0; b < LEAF_CELL_BITS; b++) r |= (((x >> b) & 1u) << (2 * b)) | (((y >> b) & 1u) << (2 * b + 1));
     return r;
 }
+// Small meshes sort by a coarser grid of about one cell per leaf (4^bits
+// cells, so that clearing and scanning the counts costs no more than the
+// leaves do) and order each coarse cell by fine cell first: the same order.
 struct LeafKeyOne {
-    __device__ int key(const int3&, int2 g) const { return (int)morton_cell_leaf(g); }
+    int shift;  // 2 * (LEAF_CELL_BITS - bits)
+    __device__ int key(const int3&, int2 g) const { return (int)(morton_cell_leaf(g) >> shift); }
+};
+static int leaf_bits(long long nleaf)
+{
+    int b = 5;
+    while (b < LEAF_CELL_BITS && (1LL << (2 * b)) < nleaf) b++;
+    return b;
+}
+__device__ inline int2 centroid(const int2* pts, const int3& t)
+{
+    const int2 a = pts[t.x], b = pts[t.y], c = pts[t.z];
+    return make_int2((int)(((long long)a.x + b.x + c.x) / 3), (int)(((long long)a.y + b.y + c.y) / 3));
+}
+
+// CellKeyTri with the leaf's fine cell before its vertex ids
+struct CellKeyTriFine {
+    const int3* tri;
+    const int2* pts;
+    int* src;
+    int* dest;
+    using Key = int4;
+    using Slot = int2;
+    __device__ void put(long long pos, const Slot& e) const { put_elem(pos, e.x); }
+    __device__ void put_elem(long long pos, int el) const
+    {
+        src[pos] = el;
+        dest[el] = (int)pos;
+    }
+    __device__ Key of(int e) const
+    {
+        const int3 t = tri[e];
+        const int a = min(t.x, min(t.y, t.z)), c = max(t.x, max(t.y, t.z));
+        return make_int4((int)morton_cell_leaf(centroid(pts, t)), a, t.x + t.y + t.z - a - c, c);
+    }
+    __device__ static Key max_key() { return make_int4(INT_MAX, INT_MAX, INT_MAX, INT_MAX); }
+    __device__ static bool less(const Key& x, const Key& y)
+    {
+        if (x.x != y.x) return x.x < y.x;
+        return x.y < y.y || (x.y == y.y && (x.z < y.z || (x.z == y.z && x.w < y.w)));
+    }
 };
 
 // The count pass keeps each leaf's rank within its cell in rank[]; the dest
@@ -2708,17 +2972,15 @@ __global__ __launch_bounds__(kBlock) void k_leaf_cells(KEY kf, const int2* pts, 
     {
         int cell = -1;
         if (i < T && sons[i] == -1) {
-            int3 t = tri[i];
-            int2 a = pts[t.x], b = pts[t.y], c = pts[t.z];
-            int2 g = make_int2((int)(((long long)a.x + b.x + c.x) / 3), (int)(((long long)a.y + b.y + c.y) / 3));
-            cell = kf.key(t, g);
+            const int3 t = tri[i];
+            cell = kf.key(t, centroid(pts, t));
         }
         // consecutive leaves were allocated together and mostly share a cell
         int r = wave_run_add(cnt, cell);
         if (cell >= 0) {
             cellof[i] = cell;
             rank[i] = r;
-            if (r == CELL_BLOCK_MAX) atomicAdd(huge, 1);
+            count_large(r, huge);
         }
     }
 }
@@ -2774,30 +3036,37 @@ __global__ __launch_bounds__(kBlock) void k_leaf_move(const int3* tri, const int
     }
 }
 
-template <class KEY, class OUT>
-static int filter_leaves_sorted(Ctx& c, const KEY& kf, long long ncells, const int2* pts, const int3* tri,
-                                const int3* adj, const int* sons, int T, const OUT& out, long long cap)
+// CK: the order inside a cell
+template <class CK, class KEY, class OUT>
+static int filter_leaves_sorted(Ctx& c, CK ck, const KEY& kf, long long ncells, const int2* pts, const int3* tri,
+                                const int3* adj, const int* sons, int T, const OUT& out, long long nleaf)
 {
     DBuf<int> cnt((size_t)ncells + 1), cellof(T > 0 ? T : 1), dest(T > 0 ? T : 1);
-    fill_i32(c, cnt.p, 0, ncells + 1);
-    c.set(C_HUGE, 0);
+    FillJobs f;
+    f.add(cnt.p, 0, ncells + 1);
+    f.add(c.dcnt.p + C_HUGE, 0, 1);
+    f.add(c.dcnt.p + C_NQ, 0, 1);
+    fill_jobs(c, f);
     k_leaf_cells<KEY><<<grid_for(T), kBlock, 0, c.st>>>(kf, pts, tri, sons, T, cnt.p, cellof.p, dest.p,
                                                         c.dcnt.p + C_HUGE);
     GCDT_LAUNCH_CHECK();
     scan_excl_total(c, cnt.p, cnt.p, ncells);
-    c.read(C_TOTAL, C_HUGE - C_TOTAL + 1);
-    const int n = c.hcnt[C_TOTAL];
-    const bool huge = c.hcnt[C_HUGE] > 0;
-    if (n > cap) throw Error(GCDT_ERR_CAPACITY, "more leaves than the output holds");
+    c.read(0, C_NUM);
+    const int n = c.hcnt[C_TOTAL], large = c.hcnt[C_HUGE];
+    if (n != nleaf)
+        throw Error(GCDT_ERR_INTERNAL, "leaf count " + std::to_string(n) + " != " + std::to_string(nleaf));
     DBuf<int> src(n > 0 ? n : 1);
     {
         DBuf<int2> eb(n > 0 ? n : 1);
-        k_leaf_dest<<<grid_for(T), kBlock, 0, c.st>>>(sons, cellof.p, T, cnt.p, dest.p, eb.p, cap);
+        k_leaf_dest<<<grid_for(T), kBlock, 0, c.st>>>(sons, cellof.p, T, cnt.p, dest.p, eb.p, nleaf);
         GCDT_LAUNCH_CHECK();
         cellof.release();
         // each cell's leaves by their vertex ids (the count pass placed them
         // in arrival order); cnt holds the cells' starts, cnt[c + 1] their ends
-        cell_reorder(c, CellKeyTri{tri, src.p, dest.p}, cnt.p + 1, eb.p, n, huge);
+        ck.tri = tri;
+        ck.src = src.p;
+        ck.dest = dest.p;
+        cell_reorder(c, ck, cnt.p + 1, eb.p, n, large);
     }
     if (n > 0) {
         ProfScope ps("leaf_move", c.st, n);
@@ -2807,16 +3076,29 @@ static int filter_leaves_sorted(Ctx& c, const KEY& kf, long long ncells, const i
     return n;
 }
 
-int filter_leaves_morton(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2,
-                         int3* adj2, long long cap)
+template <class OUT>
+static int filter_leaves_one(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
+                             const OUT& out, long long nleaf)
 {
-    return filter_leaves_sorted(c, LeafKeyOne{}, LEAF_CELLS, pts, tri, adj, sons, T, LeafToArrays{tri2, adj2}, cap);
+    const int b = leaf_bits(nleaf);
+    const LeafKeyOne key{2 * (LEAF_CELL_BITS - b)};
+    if (b == LEAF_CELL_BITS)
+        return filter_leaves_sorted(c, CellKeyTri{}, key, LEAF_CELLS, pts, tri, adj, sons, T, out, nleaf);
+    CellKeyTriFine ck{};
+    ck.pts = pts;
+    return filter_leaves_sorted(c, ck, key, 1LL << (2 * b), pts, tri, adj, sons, T, out, nleaf);
+}
+
+int filter_leaves_morton(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2,
+                         int3* adj2, long long nleaf)
+{
+    return filter_leaves_one(c, pts, tri, adj, sons, T, LeafToArrays{tri2, adj2}, nleaf);
 }
 
 int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
-                             FRec* rec, long long cap)
+                             FRec* rec, long long nleaf)
 {
-    return filter_leaves_sorted(c, LeafKeyOne{}, LEAF_CELLS, pts, tri, adj, sons, T, LeafToRecords{rec, pts}, cap);
+    return filter_leaves_one(c, pts, tri, adj, sons, T, LeafToRecords{rec, pts}, nleaf);
 }
 
 // Batch meshes: instance-major, then the Morton order of the centroid's cell
@@ -2836,18 +3118,18 @@ struct LeafKeyInst {
 
 int filter_leaves_inst(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, long long ncells,
                        long long NP, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2, int3* adj2,
-                       long long cap)
+                       long long nleaf)
 {
-    return filter_leaves_sorted(c, LeafKeyInst{vinst, cbase, lvl, NP}, ncells, pts, tri, adj, sons, T,
-                                LeafToArrays{tri2, adj2}, cap);
+    return filter_leaves_sorted(c, CellKeyTri{}, LeafKeyInst{vinst, cbase, lvl, NP}, ncells, pts, tri, adj, sons, T,
+                                LeafToArrays{tri2, adj2}, nleaf);
 }
 
 int filter_leaves_inst_rec(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl,
                            long long ncells, long long NP, const int3* tri, const int3* adj, const int* sons, int T,
-                           FRec* rec, long long cap)
+                           FRec* rec, long long nleaf)
 {
-    return filter_leaves_sorted(c, LeafKeyInst{vinst, cbase, lvl, NP}, ncells, pts, tri, adj, sons, T,
-                                LeafToRecords{rec, pts}, cap);
+    return filter_leaves_sorted(c, CellKeyTri{}, LeafKeyInst{vinst, cbase, lvl, NP}, ncells, pts, tri, adj, sons, T,
+                                LeafToRecords{rec, pts}, nleaf);
 }
 
 int filter_leaves(Ctx& c, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2, int3* adj2,
@@ -2984,12 +3266,6 @@ static void build_bitmap_g(Ctx& c, const G& g, long long ncells, const int2* pts
 void build_bitmap(Ctx& c, const int2* pts, const int3* tri, int T, int** offsets, int** tris, int* ntris)
 {
     build_bitmap_g(c, GridOne{}, BITMAP_CELLS, pts, tri, T, offsets, tris, ntris);
-}
-
-void build_bitmap_batch(Ctx& c, const int2* pts, const int* vinst, long long NP, int K, const int3* tri, int T,
-                        int** offsets, int** tris, int* ntris)
-{
-    build_bitmap_g(c, GridInst{vinst, NP}, (long long)K << (2 * GridInst::LOG), pts, tri, T, offsets, tris, ntris);
 }
 
 // ================================================================== adjacency from a triangle list

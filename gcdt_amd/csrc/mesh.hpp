@@ -270,6 +270,21 @@ int prof_names(char* buf, int cap);
 // primitives
 void fill_i32(Ctx& c, int* p, int v, long long n);
 void fill_u64(Ctx& c, unsigned long long* p, unsigned long long v, long long n);
+// several fills in one launch; each repeats a 32-bit word
+struct FillJobs {
+    static constexpr int kMax = 6;
+    struct Job {
+        int* p;
+        long long n;
+        int v;
+    } job[kMax];
+    int njobs = 0;
+    void add(void* p, int v, long long n)
+    {
+        if (n > 0) job[njobs++] = Job{(int*)p, n, v};
+    }
+};
+void fill_jobs(Ctx& c, const FillJobs& f);
 // exclusive scan of n ints (out may alias in); total also to dcnt[C_TOTAL]
 void scan_excl(Ctx& c, const int* in, int* out, long long n);
 // inclusive scan: out[i] = in[0] + ... + in[i]
@@ -282,6 +297,9 @@ long long scan_scratch_ints(long long n);
 void init_square(Ctx& c, int2* pts, int3* tri, int3* adj, int n);
 // flags GCDT_ERR_INVALID unless every point is strictly inside the square
 void check_points(Ctx& c, const int2* pts, int n);
+// corners and seed triangles of the square, and the listed points in the two
+// seeds (loc, pend)
+void seed_square(Ctx& c, int2* pts, int n, int3* tri, int3* adj, const int* ids, int nids, int* loc, int* pend);
 // sample: one point per occupied 256x256 cell (smallest id); returns count
 int sample_points(Ctx& c, const int2* pts, int n, int* sample_ids, int2* sample_pts);
 // insertion rounds; pend holds npend point ids with loc[] set; tri/adj/sons
@@ -305,12 +323,14 @@ long long flip_rounds_records(Ctx& c, FRec* rec, const Mesh& m, int T, int* roun
 // spatial order: points sorted by the Morton code of their 1024^2 cell
 // (out[k] = pts[perm[k]], inv = perm^-1)
 // Counting sort of points by 20-bit Morton cell; cell_end[BITMAP_CELLS + 1]
-// receives each cell's end offset in the sorted order.
+// receives each cell's end offset in the sorted order.  Fails with
+// GCDT_ERR_INVALID unless every point is strictly inside the square.
 void morton_order(Ctx& c, const int2* pts, int n, int2* out, int* perm, int* inv, int* cell_end);
 // One sample point per occupied 256x256 cell of Morton-ordered points (the
 // cell's extreme point towards the nearer edges of the square), from
-// morton_order's cell_end; returns the count.
-int sample_points_morton(Ctx& c, const int2* pts, const int* cell_end, int* sample_ids);
+// morton_order's cell_end; returns the count.  offs (65537 ints) receives the
+// index of each 256x256 cell's sample, by the cell's Morton index.
+int sample_points_morton(Ctx& c, const int2* pts, const int* cell_end, int* sample_ids, int* offs);
 void relabel_pairs(Ctx& c, const int2* in, int C, const int* inv, int n, int2* out);
 void unmap_tris(Ctx& c, int3* tri, int T, const int* perm, int n);
 // batches: instance map, per-instance corners/seed triangles/location, local
@@ -326,12 +346,6 @@ void batch_order(Ctx& c, const int2* pts, const int* vinst, const int* cbase, co
 int batch_sample_sorted(Ctx& c, const int* cbase, const int* lvl, const int* cell_end, int K, int* ids);
 // listed points into their instance's seed triangles
 void batch_locate_ids(Ctx& c, const int2* pts, const int* vinst, const int* ids, int n, int* loc, int* pend);
-// bitmap of a batch's sample meshes: 16x16 cells per instance; offsets has
-// (K*256 + 1) ints
-void build_bitmap_batch(Ctx& c, const int2* pts, const int* vinst, long long NP, int K, const int3* tri, int T,
-                        int** offsets, int** tris, int* ntris);
-int locate_bitmap_batch(Ctx& c, const int2* pts, const int* vinst, long long NP, const int3* tri, int T,
-                        const int* bm_off, const int* bm_tri, int* loc, int* isv, int* pend);
 void batch_cons(Ctx& c, const int2* in, const long long* coff, const long long* poff, int K, long long NC, int2* out);
 // per-instance triangle lists with local vertex ids; perm (nullable) maps the
 // batch's internal point order back to the caller's
@@ -344,27 +358,37 @@ int filter_leaves(Ctx& c, const int3* tri, const int3* adj, const int* sons, int
                   long long cap);
 // same, with the leaves placed in Morton order of their centroid cell
 int filter_leaves_morton(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2,
-                         int3* adj2, long long cap);
+                         int3* adj2, long long nleaf);
 // batch meshes: leaves sorted by (instance, centroid cell in the instance's
 // grid of 4^L cells: cbase/lvl/ncells as for the batched point order)
 int filter_leaves_inst(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, long long ncells,
                        long long NP, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2, int3* adj2,
-                       long long cap);
+                       long long nleaf);
 // the same two orders, written straight into packed flip records
+// (filter_leaves_morton, _inst and these fail with GCDT_ERR_INTERNAL unless the
+// mesh has nleaf leaves)
 int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
-                             FRec* rec, long long cap);
+                             FRec* rec, long long nleaf);
 int filter_leaves_inst_rec(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl,
                            long long ncells, long long NP, const int3* tri, const int3* adj, const int* sons, int T,
-                           FRec* rec, long long cap);
+                           FRec* rec, long long nleaf);
 // bitmap CSR over 1024^2 cells; allocates offsets/tris from the pool
 void build_bitmap(Ctx& c, const int2* pts, const int3* tri, int T, int** offsets, int** tris, int* ntris);
 // mark vertices of tri[0..T) in isv (must be zeroed), then locate the other
 // points of [0,n) through the bitmap; fills loc and pend; returns npend
 int locate_bitmap(Ctx& c, const int2* pts, int n, const int3* tri, int T, const int* bm_off, const int* bm_tri,
                   int* loc, int* isv, int* pend);
+// Location without a bitmap: every point of [0,n) that is no sample walks through
+// the sample Delaunay mesh from its own cell's sample; fills loc and pend,
+// returns npend.  ids / offs as sample_points_morton gives them.  (The bitmap's
+// build alone costs 190 us with its launches and waits; the walk also wins at
+// 10M points, 27.68 -> 27.48 ms of kernels.)
+int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const int3* adj, int T, const int* ids,
+                const int* offs, int* loc, int* pend);
+int locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
+                      long long NP, int K, const int3* tri, const int3* adj, int T, int* loc, int* pend);
 // locate all points of [0,n) in the two corner triangles 0/1
 int locate_two(Ctx& c, const int2* pts, int n, int* loc, int* pend);
-int locate_two_ids(Ctx& c, const int2* pts, const int* ids, int n, int* loc, int* pend);
 // adjacency of a plain triangle list (edges matched through vertex buckets)
 void build_adjacency(Ctx& c, const int3* tri, int T, int nv, int3* adj);
 // constrained flags: bit k of cflag[t] set when edge k of t equals a constraint
