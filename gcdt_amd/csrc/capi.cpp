@@ -377,7 +377,7 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     st.flip_rounds = fr + f2;
     st.ms_flip = phase.lap();
     // ---- 5. constraints
-    if (cflag_out) fill_i32(c, cflag_out, 0, T);
+    if (cflag_out && C <= 0) fill_i32(c, cflag_out, 0, T);
     if (C > 0) {
         DBuf<int> cflag_buf, touched(T);
         int* cflag = cflag_out;
@@ -386,22 +386,19 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
         if (!cflag) {
             cflag_buf.alloc((size_t)tcap);
             cflag = cflag_buf.p;
-            fill_i32(c, cflag, 0, T);
         }
-        fill_i32(c, touched.p, 0, T);
         Mesh m{pts, tris_out, adj_out, nullptr, cflag};
         ConsDefer defer;
-        ConsResult cr = insert_constraints(c, m, T, N + 4, N, cons, C, touched.p, cell_end.p,
+        DBuf<int> tl(T);
+        ConsResult cr = insert_constraints(c, m, T, N + 4, N, cons, C, touched.p, tl.p, cell_end.p,
                                            steiner ? &defer : nullptr);
         st.constraint_rounds = cr.rounds;
         st.segments = cr.pieces;
         st.splits = cr.pieces - C;
         // only edges of rewritten triangles can be non-Delaunay now
-        DBuf<int> tl(T);
-        int nt = flags_to_list(c, touched.p, T, tl.p);
-        if (nt > 0) {
+        if (cr.rewritten > 0) {
             int f3 = 0;
-            st.flips += flip_rounds(c, m, T, tl.p, nt, &f3);
+            st.flips += flip_rounds(c, m, T, tl.p, cr.rewritten, &f3);
             st.flip_rounds += f3;
         }
         validate_mesh(c, "the constraints", m, N + 4, T, true);
@@ -785,10 +782,9 @@ int gcdt_add_constraints(void* tmp, size_t tmpBytes, const gcdt_int2* points, gc
     filter_leaves(c, (const int3*)tris, (const int3*)adjTris, sons, Tall, tri.p, adj.p, T);
     k_leaf_slots<<<grid_for(Tall), kBlock, 0, c.st>>>(sons, off.p, Tall, slot.p);
     GCDT_LAUNCH_CHECK();
-    fill_i32(c, cflag.p, 0, T);
-    fill_i32(c, touched.p, 0, T);
     Mesh m{(const int2*)points, tri.p, adj.p, nullptr, cflag.p};
-    insert_constraints(c, m, T, numPoints + 4, numPoints, (const int2*)cons, numCons, touched.p, nullptr);
+    if (numCons <= 0) fill_i32(c, touched.p, 0, T);
+    insert_constraints(c, m, T, numPoints + 4, numPoints, (const int2*)cons, numCons, touched.p, nullptr, nullptr);
     // crossed triangles are retired in the DAG; their replacements go out
     k_retire<<<grid_for(T), kBlock, 0, c.st>>>(touched.p, slot.p, T, sons);
     GCDT_LAUNCH_CHECK();
@@ -934,16 +930,13 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
         batch_cons(c, (const int2*)cons, d_coff.p, d_poff.p, K, NC, cg.p);
         relabel_pairs(c, cg.p, (int)NC, inv.p, (int)NP, cg.p);
         DBuf<int> cflag(T), touched(T), tl(T);
-        fill_i32(c, cflag.p, 0, T);
-        fill_i32(c, touched.p, 0, T);
         Mesh m{pts.p, tri.p, adj.p, nullptr, cflag.p};
-        ConsResult cr = insert_constraints(c, m, T, (int)nv, (int)NP, cg.p, (int)NC, touched.p, nullptr);
+        ConsResult cr = insert_constraints(c, m, T, (int)nv, (int)NP, cg.p, (int)NC, touched.p, tl.p, nullptr);
         bs.constraint_rounds = cr.rounds;
         bs.segments = cr.pieces;
-        int ntl = flags_to_list(c, touched.p, T, tl.p);
-        if (ntl > 0) {
+        if (cr.rewritten > 0) {
             int f3 = 0;
-            bs.flips += flip_rounds(c, m, T, tl.p, ntl, &f3);
+            bs.flips += flip_rounds(c, m, T, tl.p, cr.rewritten, &f3);
             bs.flip_rounds += f3;
         }
         validate_mesh(c, "the constraints", m, nv, T, true);

@@ -780,22 +780,48 @@ __global__ __launch_bounds__(BS) void k_cav_retri_block(Cons c, const int2* piec
 constexpr int FIX_LANES = 16;
 static_assert(CAV_WAVE_K <= FIX_LANES, "lanes per short cavity");
 
+// (touched != nullptr: every rewritten triangle is flagged there, and listed
+// the first time)
 __global__ __launch_bounds__(kBlock) void k_cav_fix(Cons c, const Win* wins, const int* nwin, const int* scr,
-                                                    const int* rew, const int* nrew, unsigned epoch)
+                                                    const int* rew, const int* nrew, unsigned epoch, int* touched,
+                                                    int* tlist, int* ntlist, int tcap)
 {
-    const long long nw = *nwin;
+    __shared__ int s_buf[STAGE_CAP];
+    __shared__ int s_base;
+    Staged<STAGE_CAP> sl(s_buf, &s_base, tlist, ntlist, tcap, c.err, MERR_CAPACITY);
+    const long long nw = *nwin, ns = nw * FIX_LANES;
     const int n = *nrew;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nw * FIX_LANES; i += (long long)gridDim.x * blockDim.x) {
-        const Win w = wins[i / FIX_LANES];
-        const int j = (int)(i % FIX_LANES);
-        if (w.K <= CAV_WAVE_K && j < w.K) cav_fix_one(c, wins, scr, scr[w.off + j], epoch, true);
+    // short cavities first, then the listed triangles, in whole tiles
+    const long long s0 = (ns + kBlock - 1) / kBlock * kBlock;
+    TILE_LOOP(base, s0 + n, kBlock)
+    {
+        const long long i = base + threadIdx.x;
+        int t = -1;
+        if (i < ns) {
+            const Win w = wins[i / FIX_LANES];
+            const int j = (int)(i % FIX_LANES);
+            if (w.K <= CAV_WAVE_K && j < w.K) t = scr[w.off + j];
+        } else if (i >= s0 && i < s0 + n) {
+            t = rew[i - s0];
+        }
+        bool first = false;
+        if (t >= 0) {
+            cav_fix_one(c, wins, scr, t, epoch, true);
+            if (touched && !touched[t]) {
+                touched[t] = 1;
+                first = true;
+            }
+        }
+        const int at = sl.reserve(first ? 1 : 0);
+        if (first) s_buf[at] = t;
     }
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        cav_fix_one(c, wins, scr, rew[i], epoch, true);
+    sl.flush();
 }
 
-__global__ void k_cav_begin(int* cnt)
+// move: the pieces left by the round before are the queue
+__global__ void k_cav_begin(int* cnt, int move)
 {
+    if (move) cnt[C_NQ] = cnt[C_NQ2];
     cnt[C_NQ2] = 0;
     cnt[C_NWIN] = 0;
     cnt[C_SCR] = 0;
@@ -863,175 +889,101 @@ struct SegStrips {
     }
 };
 
-// lanes that share one segment's strips: a segment across the square has 1,024
-// of them, most have one or two
-constexpr int SEG_LANES = 16;
-
 __device__ inline bool seg_valid(int2 e, int nmax) { return e.x >= 0 && e.y >= 0 && e.x < nmax && e.y < nmax && e.x != e.y; }
 
-// SEG_LANES lanes per segment take its strips in turn.  Bound by the latency of
-// a strip's arithmetic: with one thread per segment (and 64-bit divisions per
-// column) both passes lasted as long as the longest segment's column loop,
-// 155 + 186 us of 12 segments over 300 points and 864 + 1,024 us of 1,000 rows
-// over 100,000 points.
-__global__ __launch_bounds__(kBlock) void k_seg_ncells(const int2* pts, const int2* cons, int C, int nmax, int* cnt,
-                                                       int* err)
-{
-    const int sub = threadIdx.x % SEG_LANES;
-    for (long long i0 = (long long)blockIdx.x * (kBlock / SEG_LANES); i0 < C;
-         i0 += (long long)gridDim.x * (kBlock / SEG_LANES)) {
-        const long long i = i0 + threadIdx.x / SEG_LANES;
-        int k = 0;
-        if (i < C) {
-            const int2 e = cons[i];
-            if (!seg_valid(e, nmax)) {
-                if (sub == 0) atomicOr(err, MERR_INVALID);
-            } else {
-                const SegStrips g(pts[e.x], pts[e.y]);
-                for (int s = g.first() + sub; s <= g.last(); s += SEG_LANES) {
-                    int lo, hi;
-                    g.cells(s, lo, hi);
-                    k += hi - lo + 1;
-                }
-            }
-        }
-        for (int d = SEG_LANES / 2; d > 0; d >>= 1) {
-            const int t = __shfl_down(k, d, 64);
-            if (sub + d < SEG_LANES) k += t;
-        }
-        if (i < C && sub == 0) cnt[i] = k;
-    }
-}
-
-// one (segment, Morton cell) pair per entry
-__global__ __launch_bounds__(kBlock) void k_seg_cells(const int2* pts, const int2* cons, int C, int nmax, const int* off,
-                                                      int* pair_seg, int* pair_cell)
-{
-    const int sub = threadIdx.x % SEG_LANES;
-    for (long long i0 = (long long)blockIdx.x * (kBlock / SEG_LANES); i0 < C;
-         i0 += (long long)gridDim.x * (kBlock / SEG_LANES)) {
-        const long long i = i0 + threadIdx.x / SEG_LANES;
-        int2 e = make_int2(-1, -1);
-        if (i < C) e = cons[i];
-        // a segment's pairs start at off[i]; its lanes take consecutive places,
-        // in any order (hits are sorted along the segment later)
-        const bool ok = i < C && seg_valid(e, nmax);
-        const SegStrips g(ok ? pts[e.x] : make_int2(0, 0), ok ? pts[e.y] : make_int2(0, 0));
-        const int last = ok ? g.last() : -1;
-        int base = ok ? off[i] : 0;
-        for (int s0 = g.first();; s0 += SEG_LANES) {
-            // wave-uniform trip count: the shuffles below need every lane
-            if (__ballot(s0 <= last) == 0) break;
-            const int s = s0 + sub;
-            int lo = 0, hi = -1;
-            if (s <= last) g.cells(s, lo, hi);
-            const int k = hi - lo + 1;
-            int inc = k;
-            for (int d = 1; d < SEG_LANES; d <<= 1) {
-                const int t = __shfl_up(inc, d, 64);
-                if (sub >= d) inc += t;
-            }
-            int o = base + inc - k;
-            for (int v = lo; v <= hi; v++, o++) {
-                pair_seg[o] = (int)i;
-                pair_cell[o] = (int)(g.rows ? cell_morton((unsigned)v, (unsigned)s) : cell_morton((unsigned)s, (unsigned)v));
-            }
-            base += __shfl(inc, (int)(threadIdx.x & 63) - sub + SEG_LANES - 1, 64);
-        }
-    }
-}
-
-// The points of each pair's cell that lie strictly inside its segment: counted
-// per segment (pos == nullptr), or written to hits[hoff[seg] + ...].
-__global__ __launch_bounds__(kBlock) void k_seg_hits(const int2* pts, const int* cell_end, const int2* cons,
-                                                     const int* pair_seg, const int* pair_cell, long long npairs,
-                                                     int* hcnt, const int* hoff, int* hits)
-{
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < npairs; i += (long long)gridDim.x * blockDim.x) {
-        int sg = pair_seg[i], cell = pair_cell[i];
-        int2 e = cons[sg];
-        int2 A = pts[e.x], B = pts[e.y];
-        int p0 = cell ? cell_end[cell - 1] : 0, p1 = cell_end[cell];
-        for (int p = p0; p < p1; p++) {
-            if (p == e.x || p == e.y) continue;
-            int2 P = pts[p];
-            if (orient2d(A, B, P) != 0 || !strictly_between(A, B, P)) continue;
-            int k = atomicAdd(&hcnt[sg], 1);
-            if (hits) hits[hoff[sg] + k] = p;
-        }
-    }
-}
-
-// pieces per segment: h + 1 for a sorted segment; a segment with more than
-// SEG_SORT_MAX vertices on it goes to the walk list (its count comes later)
-__global__ __launch_bounds__(kBlock) void k_seg_npieces(const int2* cons, int C, int nmax, const int* hcnt, int* np,
-                                                        int* sort_list, int* nsort, int* walk_list, int* nwalk)
-{
-    WAVE_LOOP(i, C)
-    {
-        int h = 0;
-        bool valid = false;
-        if (i < C) {
-            valid = seg_valid(cons[i], nmax);
-            h = hcnt[i];
-            np[i] = valid ? (h <= SEG_SORT_MAX ? h + 1 : 0) : 0;
-        }
-        bool srt = valid && h >= 2 && h <= SEG_SORT_MAX, wlk = valid && h > SEG_SORT_MAX;
-        int a = wave_alloc(srt ? 1 : 0, nsort);
-        if (srt) sort_list[a] = (int)i;
-        int b = wave_alloc(wlk ? 1 : 0, nwalk);
-        if (wlk) walk_list[b] = (int)i;
-    }
-}
-
-// one workgroup per listed segment: its vertices sorted along it (bitonic
-// sort in LDS of (position along the segment, vertex) pairs)
-__global__ __launch_bounds__(kBlock) void k_seg_sort(const int2* pts, const int2* cons, const int* list, const int* nlist,
-                                                     const int* hcnt, const int* hoff, int* hits)
+// Vertices strictly inside each segment, one wave per segment: its lanes take
+// strips in turn, test the points of every cell and collect the vertices on
+// the segment in LDS, where they are sorted along it.  They leave at hpos[i]
+// of hits[] (room permitting: the cursor counts on and the caller repeats the
+// launch with more), np[i] = pieces of the segment.  A segment with more than
+// SEG_SORT_MAX vertices on it goes to the walk list (its count comes later).
+// Bound by the latency of a strip's chain (cell ends, points); the passes of
+// one thread per segment and strip that this replaces took 155 + 186 us for
+// 12 segments over 300 points and 864 + 1,024 us for 1,000 rows over 100,000.
+__global__ __launch_bounds__(64) void k_seg_find(const int2* pts, const int* cell_end, const int2* cons, int C, int nmax,
+                                                 int* np, int* hcnt, int* hpos, int* hits, int hcap, int* hcur,
+                                                 int* walk_list, int* nwalk, int* err)
 {
     __shared__ long long s_key[SEG_SORT_MAX];
     __shared__ int s_val[SEG_SORT_MAX];
-    int n = *nlist;
-    for (int w = blockIdx.x; w < n; w += gridDim.x) {
-        int sg = list[w];
-        int h = hcnt[sg], o = hoff[sg];
-        int2 e = cons[sg];
-        int2 A = pts[e.x], B = pts[e.y];
-        long long dx = (long long)B.x - A.x, dy = (long long)B.y - A.y;
-        int m = 1;
-        while (m < h) m <<= 1;
-        for (int k = threadIdx.x; k < m; k += blockDim.x) {
-            if (k < h) {
-                int p = hits[o + k];
-                int2 P = pts[p];
-                s_key[k] = ((long long)P.x - A.x) * dx + ((long long)P.y - A.y) * dy;
-                s_val[k] = p;
-            } else {
-                s_key[k] = LLONG_MAX;
-                s_val[k] = -1;
+    __shared__ int s_n, s_at;
+    const int lane = threadIdx.x;
+    for (int i = blockIdx.x; i < C; i += gridDim.x) {
+        const int2 e = cons[i];
+        if (!seg_valid(e, nmax)) {  // block-uniform
+            if (lane == 0) {
+                atomicOr(err, MERR_INVALID);
+                np[i] = 0;
+                hcnt[i] = 0;
+            }
+            continue;
+        }
+        if (lane == 0) s_n = 0;
+        __syncthreads();
+        const int2 A = pts[e.x], B = pts[e.y];
+        const long long dx = (long long)B.x - A.x, dy = (long long)B.y - A.y;
+        const SegStrips g(A, B);
+        for (int st = g.first() + lane; st <= g.last(); st += 64) {
+            int lo, hi;
+            g.cells(st, lo, hi);
+            for (int v = lo; v <= hi; v++) {
+                const unsigned cell = g.rows ? cell_morton((unsigned)v, (unsigned)st) : cell_morton((unsigned)st, (unsigned)v);
+                const int p1 = cell_end[cell];
+                for (int p = cell ? cell_end[cell - 1] : 0; p < p1; p++) {
+                    if (p == e.x || p == e.y) continue;
+                    const int2 P = pts[p];
+                    if (orient2d(A, B, P) != 0 || !strictly_between(A, B, P)) continue;
+                    const int k = atomicAdd(&s_n, 1);
+                    if (k < SEG_SORT_MAX) {
+                        s_key[k] = ((long long)P.x - A.x) * dx + ((long long)P.y - A.y) * dy;
+                        s_val[k] = p;
+                    }
+                }
             }
         }
         __syncthreads();
-        for (int size = 2; size <= m; size <<= 1) {
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                for (int k = threadIdx.x; k < m; k += blockDim.x) {
-                    int j = k ^ stride;
-                    if (j > k) {
-                        bool up = (k & size) == 0;
-                        long long a = s_key[k], b = s_key[j];
-                        if ((a > b) == up) {
-                            s_key[k] = b;
-                            s_key[j] = a;
-                            int t = s_val[k];
-                            s_val[k] = s_val[j];
-                            s_val[j] = t;
+        const int h = s_n;
+        if (h > 1 && h <= SEG_SORT_MAX) {
+            int m = 2;
+            while (m < h) m <<= 1;
+            for (int k = h + lane; k < m; k += 64) {
+                s_key[k] = LLONG_MAX;
+                s_val[k] = -1;
+            }
+            __syncthreads();
+            for (int size = 2; size <= m; size <<= 1) {
+                for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                    for (int k = lane; k < (m >> 1); k += 64) {
+                        const int a = 2 * k - (k & (stride - 1)), b = a + stride;
+                        const bool up = (a & size) == 0;
+                        const long long ka = s_key[a], kb = s_key[b];
+                        if ((ka > kb) == up) {
+                            s_key[a] = kb;
+                            s_key[b] = ka;
+                            const int t = s_val[a];
+                            s_val[a] = s_val[b];
+                            s_val[b] = t;
                         }
                     }
+                    __syncthreads();
                 }
-                __syncthreads();
             }
         }
-        for (int k = threadIdx.x; k < h; k += blockDim.x) hits[o + k] = s_val[k];
+        if (lane == 0) {
+            hcnt[i] = h;
+            np[i] = h <= SEG_SORT_MAX ? h + 1 : 0;
+            s_at = -1;
+            if (h > SEG_SORT_MAX) {
+                walk_list[atomicAdd(nwalk, 1)] = i;
+            } else if (h > 0) {
+                const int at = atomicAdd(hcur, h);
+                hpos[i] = at;
+                if (at >= 0 && h <= hcap - at) s_at = at;
+            }
+        }
+        __syncthreads();
+        if (s_at >= 0)
+            for (int k = lane; k < h; k += 64) hits[s_at + k] = s_val[k];
         __syncthreads();
     }
 }
@@ -1049,39 +1001,47 @@ __device__ inline int upper_bound_seg(const int* a, int n, long long x)
 
 // one thread per piece of the sorted segments: (previous vertex, next vertex)
 // along the segment; an existing edge is marked constrained and stored with
-// a negative first vertex
+// a negative first vertex, any other piece is queued for the rounds
 __global__ __launch_bounds__(kBlock) void k_seg_pieces(Cons c, const int2* cons, int C, const int* poff,
-                                                       const int* hcnt, const int* hoff, const int* hits,
-                                                       long long total, int2* pieces)
+                                                       const int* hcnt, const int* hpos, const int* hits,
+                                                       long long total, int2* pieces, int* queue, int* nq)
 {
     const Mesh& m = c.m;
-    for (long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x; j < total; j += (long long)gridDim.x * blockDim.x) {
-        int sg = upper_bound_seg(poff, C + 1, j) - 1;
-        int h = hcnt[sg];
-        if (h > SEG_SORT_MAX) continue;  // the walk writes this segment's pieces
-        int k = (int)(j - poff[sg]);
-        int2 e = cons[sg];
-        // the q-th vertex from e.x (hits are sorted from e.x towards e.y)
-        auto vtx = [&](int q) { return q == 0 ? e.x : (q == h + 1 ? e.y : hits[hoff[sg] + q - 1]); };
-        int u = vtx(k), v = vtx(k + 1);
-        int t, s;
-        int r = find_wedge(c, u, v, t, s);
-        if (r < 0) {
-            at_or(c.err, MERR_WALK);
-            pieces[j] = make_int2(u, v);
-            continue;
+    WAVE_LOOP(j, total)
+    {
+        bool want = false;
+        const int sg = j < total ? upper_bound_seg(poff, C + 1, j) - 1 : 0;
+        const int h = j < total ? hcnt[sg] : 0;
+        if (j < total && h <= SEG_SORT_MAX) {  // else the walk writes this segment's pieces
+            const int k = (int)(j - poff[sg]);
+            const int2 e = cons[sg];
+            // the q-th vertex from e.x (hits are sorted from e.x towards e.y)
+            auto vtx = [&](int q) { return q == 0 ? e.x : (q == h + 1 ? e.y : hits[hpos[sg] + q - 1]); };
+            const int u = vtx(k), v = vtx(k + 1);
+            int t, s;
+            const int r = find_wedge(c, u, v, t, s);
+            if (r < 0) at_or(c.err, MERR_WALK);
+            if (r == 1 && get3(m.tri[t], nx3(s)) == v) {
+                mark_pair(c, t, pv3(s));
+                pieces[j] = make_int2(-(u + 1), v);
+            } else {
+                pieces[j] = make_int2(u, v);
+                want = true;
+            }
         }
-        if (r == 1 && get3(m.tri[t], nx3(s)) == v) {
-            mark_pair(c, t, pv3(s));
-            pieces[j] = make_int2(-(u + 1), v);
-        } else {
-            pieces[j] = make_int2(u, v);
-        }
+        const int at = wave_alloc(want ? 1 : 0, nq);
+        if (want) queue[at] = (int)j;
     }
 }
 
 // the walk's pieces for the listed (long) segments: counted into np, then
 // written at their offsets
+__global__ __launch_bounds__(kBlock) void k_seg_counts(const int2* cons, int C, int nmax, const int* hcnt, int* np)
+{
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < C; i += (long long)gridDim.x * blockDim.x)
+        np[i] = seg_valid(cons[i], nmax) && hcnt[i] <= SEG_SORT_MAX ? hcnt[i] + 1 : 0;
+}
+
 __global__ __launch_bounds__(kBlock) void k_seg_walk(Cons c, const int2* cons, const int* list, const int* nlist,
                                                      int* np, const int* poff, int2* pieces)
 {
@@ -1094,65 +1054,58 @@ __global__ __launch_bounds__(kBlock) void k_seg_walk(Cons c, const int2* cons, c
     }
 }
 
+// *nq: true when the pieces that need a cavity have been queued (C_NQ was
+// cleared by the caller, and C_NREW, C_NQ2 as cursors)
 static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const int2* cons, int C, int nmax,
-                              DBuf<int2>& pieces)
+                              DBuf<int2>& pieces, DBuf<int>& queue, bool* queued)
 {
     const int2* pts = c.m.pts;
-    DBuf<int> off((size_t)C + 1);
-    k_seg_ncells<<<grid_for((long long)C * SEG_LANES), kBlock, 0, cx.st>>>(pts, cons, C, nmax, off.p, c.err);
-    GCDT_LAUNCH_CHECK();
-    cx.check_err();
-    scan_excl_total(cx, off.p, off.p, C);
-    long long npairs = cx.get(C_TOTAL);
-    DBuf<int> pseg(npairs > 0 ? npairs : 1), pcell(npairs > 0 ? npairs : 1);
-    k_seg_cells<<<grid_for((long long)C * SEG_LANES), kBlock, 0, cx.st>>>(pts, cons, C, nmax, off.p, pseg.p, pcell.p);
-    GCDT_LAUNCH_CHECK();
-    off.release();
-    // vertices strictly inside each segment: count, offsets, positions
-    DBuf<int> hcnt((size_t)C + 1), hoff((size_t)C + 1);
-    fill_i32(cx, hcnt.p, 0, C);
-    k_seg_hits<<<grid_for(npairs), kBlock, 0, cx.st>>>(pts, cell_end, cons, pseg.p, pcell.p, npairs, hcnt.p, nullptr,
-                                                       nullptr);
-    GCDT_LAUNCH_CHECK();
-    scan_excl_total(cx, hcnt.p, hoff.p, C);
-    long long nh = cx.get(C_TOTAL);
-    DBuf<int> hits(nh > 0 ? nh : 1);
-    fill_i32(cx, hcnt.p, 0, C);
-    k_seg_hits<<<grid_for(npairs), kBlock, 0, cx.st>>>(pts, cell_end, cons, pseg.p, pcell.p, npairs, hcnt.p, hoff.p,
-                                                       hits.p);
-    GCDT_LAUNCH_CHECK();
-    pseg.release();
-    pcell.release();
-    // pieces per segment; segments with many vertices keep the walk
-    DBuf<int> np((size_t)C + 1), slist(C > 0 ? C : 1), wlist(C > 0 ? C : 1);
-    cx.set(C_NQ, 0);
-    cx.set(C_NQ2, 0);
-    k_seg_npieces<<<grid_for(C), kBlock, 0, cx.st>>>(cons, C, nmax, hcnt.p, np.p, slist.p, cx.dcnt.p + C_NQ, wlist.p,
-                                                     cx.dcnt.p + C_NQ2);
-    GCDT_LAUNCH_CHECK();
-    k_seg_sort<<<std::min(std::max(C, 1), 65536), kBlock, 0, cx.st>>>(pts, cons, slist.p, cx.dcnt.p + C_NQ, hcnt.p,
-                                                                      hoff.p, hits.p);
-    GCDT_LAUNCH_CHECK();
-    cx.read(C_NQ, 2);
-    int nwalk = cx.hcnt[C_NQ2];
+    int* cnt = cx.dcnt.p;
+    DBuf<int> np((size_t)C + 1), hcnt(C), hpos(C), wlist(C), hits((size_t)2 * C + 1024);
+    for (int tries = 0;; tries++) {
+        const int hcap = (int)std::min<size_t>(hits.n, 1u << 30);
+        k_seg_find<<<std::min(C, 16384), 64, 0, cx.st>>>(pts, cell_end, cons, C, nmax, np.p, hcnt.p, hpos.p, hits.p, hcap,
+                                                         cnt + C_NREW, wlist.p, cnt + C_NQ2, c.err);
+        GCDT_LAUNCH_CHECK();
+        scan_excl_total(cx, np.p, np.p, C);
+        cx.read(0, C_NUM);
+        if (cx.hcnt[C_ERR]) cx.check_err();
+        const long long nh = cx.hcnt[C_NREW];
+        if (nh < 0 || nh > (1LL << 30)) throw Error(GCDT_ERR_SCRATCH, "too many vertices on the constraints");
+        if (nh <= (long long)hits.n) break;
+        if (tries) throw Error(GCDT_ERR_INTERNAL, "constraint split changed between two passes");
+        hits.ensure((size_t)nh);
+        cx.set(C_NREW, 0);
+        cx.set(C_NQ2, 0);
+    }
+    int total = cx.hcnt[C_TOTAL];
+    const int nwalk = cx.hcnt[C_NQ2];
     if (nwalk > 0) {
-        k_seg_walk<<<grid_for(nwalk), kBlock, 0, cx.st>>>(c, cons, wlist.p, cx.dcnt.p + C_NQ2, np.p, nullptr, nullptr);
+        // segments with many vertices keep the walk: their counts, and the
+        // offsets again (from the counts of the others)
+        DBuf<int> cnts((size_t)C + 1);
+        k_seg_counts<<<grid_for(C), kBlock, 0, cx.st>>>(cons, C, nmax, hcnt.p, cnts.p);
+        GCDT_LAUNCH_CHECK();
+        k_seg_walk<<<grid_for(nwalk), kBlock, 0, cx.st>>>(c, cons, wlist.p, cnt + C_NQ2, cnts.p, nullptr, nullptr);
+        GCDT_LAUNCH_CHECK();
+        scan_excl_total(cx, cnts.p, np.p, C);
+        cx.read(0, C_NUM);
+        if (cx.hcnt[C_ERR]) cx.check_err();
+        total = cx.hcnt[C_TOTAL];
+    }
+    pieces.alloc(total > 0 ? total : 1);
+    queue.alloc(total > 0 ? total : 1);
+    if (total > 0) {
+        k_seg_pieces<<<grid_for(total), kBlock, 0, cx.st>>>(c, cons, C, np.p, hcnt.p, hpos.p, hits.p, total, pieces.p,
+                                                            queue.p, cnt + C_NQ);
+        GCDT_LAUNCH_CHECK();
+    }
+    *queued = nwalk == 0;
+    if (nwalk > 0) {
+        k_seg_walk<<<grid_for(nwalk), kBlock, 0, cx.st>>>(c, cons, wlist.p, cnt + C_NQ2, nullptr, np.p, pieces.p);
         GCDT_LAUNCH_CHECK();
         cx.check_err();
     }
-    scan_excl_total(cx, np.p, np.p, C);
-    int total = cx.get(C_TOTAL);
-    pieces.alloc(total > 0 ? total : 1);
-    if (total > 0) {
-        k_seg_pieces<<<grid_for(total), kBlock, 0, cx.st>>>(c, cons, C, np.p, hcnt.p, hoff.p, hits.p, total, pieces.p);
-        GCDT_LAUNCH_CHECK();
-    }
-    if (nwalk > 0) {
-        k_seg_walk<<<grid_for(nwalk), kBlock, 0, cx.st>>>(c, cons, wlist.p, cx.dcnt.p + C_NQ2, nullptr, np.p,
-                                                          pieces.p);
-        GCDT_LAUNCH_CHECK();
-    }
-    cx.check_err();
     return total;
 }
 
@@ -1163,9 +1116,10 @@ static int split_pieces(Ctx& cx, const Cons& c, const int2* cons, int C, int nma
     DBuf<int> cnt((size_t)C + 1);
     k_split_count<<<grid_for(C), kBlock, 0, cx.st>>>(c, cons, C, nmax, cnt.p);
     GCDT_LAUNCH_CHECK();
-    cx.check_err();
     scan_excl_total(cx, cnt.p, cnt.p, C);
-    int np = cx.get(C_TOTAL);
+    cx.read(0, C_NUM);
+    if (cx.hcnt[C_ERR]) cx.check_err();
+    int np = cx.hcnt[C_TOTAL];
     pieces.alloc(np > 0 ? np : 1);
     k_split_emit<<<grid_for(C), kBlock, 0, cx.st>>>(c, cons, C, cnt.p, pieces.p);
     GCDT_LAUNCH_CHECK();
@@ -1191,23 +1145,22 @@ long long mark_constraint_chains(Ctx& cx, const Mesh& m, int T, int nv, int nmax
     return split_pieces(cx, c, cons, C, nmax, pieces);
 }
 
-__global__ __launch_bounds__(kBlock) void k_touched(const int* stamp, int T, int* touched)
-{
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < T; i += (long long)gridDim.x * blockDim.x)
-        touched[i] = stamp[i] != 0;
-}
-
 ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, const int2* cons, int C,
-                              int* touched, const int* cell_end, ConsDefer* defer)
+                              int* touched, int* tlist, const int* cell_end, ConsDefer* defer)
 {
     ConsResult res;
     if (C <= 0) return res;
     DBuf<int> vt(nv);
     DBuf<unsigned long long> owner(T);
     DBuf<int> stamp(T), cavof(T);
-    fill_i32(cx, vt.p, -1, nv);
-    fill_u64(cx, owner.p, ~0ull, T);
-    fill_i32(cx, stamp.p, 0, T);
+    FillJobs f;
+    f.add(vt.p, -1, nv);
+    f.add(owner.p, -1, 2LL * T);
+    f.add(stamp.p, 0, T);
+    f.add(m.cflag, 0, T);
+    f.add(touched, 0, T);
+    f.add(cx.dcnt.p + C_NPIECE, 0, C_NWIN - C_NPIECE + 1);
+    fill_jobs(cx, f);
     k_build_vt<<<grid_for(T), kBlock, 0, cx.st>>>(m.tri, T, vt.p);
     GCDT_LAUNCH_CHECK();
     Cons c;
@@ -1220,7 +1173,9 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
     c.steiner = defer != nullptr;
     // 1. split into pieces
     DBuf<int2> pieces;
-    int np = cell_end ? split_pieces_cells(cx, c, cell_end, cons, C, nmax, pieces)
+    DBuf<int> qa;
+    bool queued = false;
+    int np = cell_end ? split_pieces_cells(cx, c, cell_end, cons, C, nmax, pieces, qa, &queued)
                       : split_pieces(cx, c, cons, C, nmax, pieces);
     res.pieces = np;
     DBuf<int> dflag;
@@ -1230,12 +1185,15 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
         c.defer = dflag.p;
     }
     // 2. rounds over pieces that need a cavity
-    DBuf<int> qa(np > 0 ? np : 1), qb(np > 0 ? np : 1), ncross(np > 0 ? np : 1);
+    DBuf<int> qb(np > 0 ? np : 1), ncross(np > 0 ? np : 1);
     DBuf<Win> wins(np > 0 ? np : 1);
-    cx.set(C_NQ, 0);
-    k_piece_queue<<<grid_for(np), kBlock, 0, cx.st>>>(pieces.p, np, qa.p, cx.dcnt.p + C_NQ);
-    GCDT_LAUNCH_CHECK();
-    int nq = cx.get(C_NQ);
+    if (!queued) {
+        qa.ensure(np > 0 ? np : 1);
+        cx.set(C_NQ, 0);
+        k_piece_queue<<<grid_for(np), kBlock, 0, cx.st>>>(pieces.p, np, qa.p, cx.dcnt.p + C_NQ);
+        GCDT_LAUNCH_CHECK();
+    }
+    int nq = np;  // at most; the first round's counters tell
     int* Q = qa.p;
     int* Q2 = qb.p;
     DBuf<int> scr, rew;
@@ -1253,7 +1211,7 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
         long long npath = 0;
         for (int tries = 0;; tries++) {
             const int pcap = (int)std::min<size_t>(paths.n, 1u << 30);
-            k_cav_begin<<<1, 1, 0, cx.st>>>(cnt);
+            k_cav_begin<<<1, 1, 0, cx.st>>>(cnt, r > 1 && tries == 0);
             GCDT_LAUNCH_CHECK();
             k_cav_claim<<<g, kBlock, 0, cx.st>>>(c, pieces.p, Q, cnt + C_NQ, ep, ncross.p, paths.p, pcap, cnt + C_PATH,
                                                  ppos.p, longq.p, cnt + C_NLONG);
@@ -1263,6 +1221,7 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
                                                                   ppos.p);
             GCDT_LAUNCH_CHECK();
             cx.read(0, C_NUM);
+            nq = cx.hcnt[C_NQ];
             npath = cx.hcnt[C_PATH];
             if (npath < 0 || npath > (1LL << 30)) throw Error(GCDT_ERR_SCRATCH, "constraints cross too many triangles");
             if (npath <= (long long)paths.n) break;
@@ -1270,6 +1229,11 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
             // claims are the same)
             if (tries) throw Error(GCDT_ERR_INTERNAL, "constraint paths changed between two walks");
             paths.ensure((size_t)npath);
+        }
+        if (nq == 0) {  // every piece was an edge already
+            if (cx.hcnt[C_ERR]) cx.check_err();
+            r--;
+            break;
         }
         const int nlong = cx.hcnt[C_NLONG];
         // scratch of every queued piece: cav_block_ints(K) (9 K + 16) for the
@@ -1309,20 +1273,16 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
             GCDT_LAUNCH_CHECK();
         }
         k_cav_fix<<<grid_for(std::max<long long>((long long)FIX_LANES * (nq - nlong), npl)), kBlock, 0, cx.st>>>(
-            c, wins.p, cnt + C_NWIN, scr.p, rew.p, cnt + C_NREW, ep);
+            c, wins.p, cnt + C_NWIN, scr.p, rew.p, cnt + C_NREW, ep, touched, tlist, cnt + C_NPIECE, tlist ? T : 0);
         GCDT_LAUNCH_CHECK();
         cx.read(0, C_NUM);
         if (cx.hcnt[C_ERR]) cx.check_err();
         nq = cx.hcnt[C_NQ2];
         if (nq > 0 && cx.hcnt[C_NWIN] == 0) throw Error(GCDT_ERR_INTERNAL, "constraint round without progress");
-        cx.set(C_NQ, nq);
+        res.rewritten = cx.hcnt[C_NPIECE];
         std::swap(Q, Q2);
     }
     res.rounds = r;
-    if (touched) {
-        k_touched<<<grid_for(T), kBlock, 0, cx.st>>>(stamp.p, T, touched);
-        GCDT_LAUNCH_CHECK();
-    }
     if (defer) {
         defer->pieces = std::move(pieces);
         defer->flag = std::move(dflag);

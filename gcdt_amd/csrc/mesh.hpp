@@ -103,7 +103,7 @@ enum : int {
     C_ERR = 4,
     C_NBIGW = 6,   // constraint rounds: winners above CAV_MID_K
     C_TOTAL = 8,   // scan totals
-    C_NPIECE = 10,
+    C_NPIECE = 10,  // constraint rounds: triangles rewritten so far
     C_NQ = 11,
     C_NQ2 = 12,
     C_SCR = 13,    // cavity scratch cursor
@@ -399,6 +399,7 @@ void mark_constraint_edges(Ctx& c, const int3* tri, const int3* adj, int T, int 
 struct ConsResult {
     int rounds = 0;
     long long pieces = 0;
+    int rewritten = 0;  // triangles in tlist
 };
 // nmax: constraint endpoints must be vertex ids in [0, nmax)
 // cell_end (optional): the Morton cell ends of m.pts (morton_order), so the
@@ -412,7 +413,7 @@ struct ConsDefer {
     int np = 0;
 };
 ConsResult insert_constraints(Ctx& c, const Mesh& m, int T, int nv, int nmax, const int2* cons, int C, int* touched,
-                              const int* cell_end, ConsDefer* defer = nullptr);
+                              int* tlist, const int* cell_end, ConsDefer* defer = nullptr);
 // Crossing pass (steiner.hip): inserts the deferred pieces into the CDT of the
 // others with a vertex at every crossing (ids nv0, nv0 + 1, ...); the mesh
 // arrays hold tcap triangles.  The crossing points are written to out with

@@ -23,10 +23,18 @@ SMALL = (("GCDT_CAV_WAVE_K=4", "GCDT_CAV_MID_K=8", "GCDT_CAV_LDS_K=20"),
 
 
 def segments(kind: str, n: int, c: int, seed: int = 5):
-    """n random points and c disjoint parallel segments of up to the square's
+    """"online": many vertices on each segment.  Else n random points and c disjoint parallel segments of up to the square's
     side: rows, columns, or lines of slope 3 or 1/3 (steep, flat)."""
     rng = np.random.default_rng(seed)
     side = 1 << 20
+    if kind == "online":
+        # n points on each of c rows, which the segments run along, and as many anywhere
+        at = (np.arange(c) * 2 + 1) * (side // (2 * c))
+        x = np.sort(rng.permutation(side - 2)[:n] + 1)
+        on = np.stack(np.meshgrid(x, at), 2).reshape(-1, 2)
+        segs = np.stack([np.stack([np.zeros(c, int), at], 1), np.stack([np.full(c, side - 1), at], 1)], 1)
+        xy, ids = gen.dedup(np.concatenate([rng.integers(0, side, (n, 2)), on, segs.reshape(-1, 2)]))
+        return gen.to_grid(xy), ids[n + len(on):].reshape(-1, 2).astype(np.int32)
     pts = rng.integers(0, side, (n, 2))
     at = (np.arange(c) * 2 + 1) * (side // (2 * c))
     lo = rng.integers(0, side // 3, c)
@@ -56,7 +64,9 @@ def check(g, cons, tris):
 
 
 CASES = [("rows", 400, 3), ("rows", 5000, 40), ("columns", 5000, 40), ("steep", 3000, 25), ("flat", 3001, 25),
-         ("columns", 60, 2)]
+         ("columns", 60, 2),
+         # more vertices on the segments than the first buffer holds; more than one wave sorts (1,024)
+         ("online", 900, 3), ("online", 1100, 1)]
 
 
 def emulated(lib, case, seed):
