@@ -11,7 +11,13 @@
 //   orient(p, q, r) = sign | Xp Yp Wp ; Xq Yq Wq ; Xr Yr Wr |         (< 2^248: 4 limbs)
 //   incircle(a, b, c, d) = sign | XW  YW  X^2+Y^2  W^2 |_{a,b,c,d}   (< 2^618: 10 limbs)
 // which equal orient2d / incircle of predicates.hpp on grid points (rows of
-// the second are scaled by W^2 > 0, which keeps the sign).  No floating point.
+// the second are scaled by W^2 > 0, which keeps the sign).
+//
+// The determinants cost thousands of 64-bit products (incircle_h about 100 us
+// on one lane), so callers ask the filters below first: the same determinant
+// in double on the rounded coordinates, with a bound on its error.  A filter
+// gives the exact sign or 0 for "not certain", never a wrong sign; zero
+// determinants always go to the exact form.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -207,6 +213,64 @@ __host__ __device__ inline int hpt_cmp_y(const HPt& u, const HPt& p)
 {
     typedef Big<4> B;
     return (B::of(u.Y) * B::of(p.W) - B::of(p.Y) * B::of(u.W)).sign();
+}
+
+// ---------------------------------------------------------------- filters
+
+// A point's coordinates rounded to double.  A grid point is exact.  For a
+// crossing, X is rounded twice (its words), W once and the quotient once: at
+// most 4.01 u relative (u = 2^-53), below 2^-20.9 absolute on the 2^30 grid.
+struct DPt {
+    double x, y;
+};
+
+__host__ __device__ inline double big2_double(const Big<2>& v)
+{
+    const bool neg = v.neg();
+    const Big<2> m = neg ? -v : v;
+    const double d = (double)m.w[1] * 18446744073709551616.0 + (double)m.w[0];
+    return neg ? -d : d;
+}
+
+__host__ __device__ inline DPt dpt(const HPt& h)
+{
+    const double w = (double)h.W;
+    return DPt{big2_double(h.X) / w, big2_double(h.Y) / w};
+}
+
+__host__ __device__ inline DPt dpt(int2 p) { return DPt{(double)p.x, (double)p.y}; }
+
+// A difference of two such coordinates is off by less than 2 * 2^-20.9 plus
+// its own rounding 2^-22.
+constexpr double FILTER_DELTA = 1.0 / (1 << 19);
+constexpr double FILTER_U = 1.0 / 9007199254740992.0;
+
+__host__ __device__ inline double dabs(double v) { return v < 0 ? -v : v; }
+__host__ __device__ inline double dmax(double a, double b) { return a > b ? a : b; }
+
+// With every difference at most M (the error included): the two products are
+// off by 4 M delta + 2 delta^2 from the inputs and 3 M^2 u from rounding.
+__host__ __device__ inline int orient_filter(const DPt& p, const DPt& q, const DPt& r)
+{
+    const double ax = p.x - r.x, ay = p.y - r.y, bx = q.x - r.x, by = q.y - r.y;
+    const double det = ax * by - ay * bx;
+    const double M = dmax(dmax(dabs(ax), dabs(ay)), dmax(dabs(bx), dabs(by))) + FILTER_DELTA;
+    const double e = 8.0 * FILTER_DELTA * M + 8.0 * FILTER_U * M * M;
+    return det > e ? 1 : (det < -e ? -1 : 0);
+}
+
+// A lifted length (at most 2 M^2) is off by 4 M delta + 2 delta^2, a cross
+// product likewise, so the three products by 48 M^3 delta + 72 M^2 delta^2
+// (below 64 delta (M + delta)^3), and by 84 u M^4 from rounding.
+__host__ __device__ inline int incircle_filter(const DPt& a, const DPt& b, const DPt& c, const DPt& d)
+{
+    const double ax = a.x - d.x, ay = a.y - d.y, bx = b.x - d.x, by = b.y - d.y, cx = c.x - d.x, cy = c.y - d.y;
+    const double det = (ax * ax + ay * ay) * (bx * cy - by * cx) + (bx * bx + by * by) * (cx * ay - cy * ax) +
+                       (cx * cx + cy * cy) * (ax * by - ay * bx);
+    const double M = dmax(dmax(dmax(dabs(ax), dabs(ay)), dmax(dabs(bx), dabs(by))), dmax(dabs(cx), dabs(cy))) +
+                     FILTER_DELTA;
+    const double e = M * M * M * (64.0 * FILTER_DELTA + 256.0 * FILTER_U * M);
+    return det > e ? 1 : (det < -e ? -1 : 0);
 }
 
 }  // namespace gcdt

@@ -56,15 +56,21 @@ struct Stn {
 
 __host__ __device__ inline HPt stn_pt(const Stn& s, int v) { return v < s.nv0 ? hpt_grid(s.pts[v]) : s.hp[v - s.nv0]; }
 
+__host__ __device__ inline DPt stn_dpt(const Stn& s, int v) { return v < s.nv0 ? dpt(s.pts[v]) : dpt(s.hp[v - s.nv0]); }
+
 __host__ __device__ inline int stn_orient(const Stn& s, int a, int b, int c)
 {
     if (a < s.nv0 && b < s.nv0 && c < s.nv0) return orient2d(s.pts[a], s.pts[b], s.pts[c]);
+    const int o = orient_filter(stn_dpt(s, a), stn_dpt(s, b), stn_dpt(s, c));
+    if (o) return o;
     return orient_h(stn_pt(s, a), stn_pt(s, b), stn_pt(s, c));
 }
 
 __host__ __device__ inline int stn_incircle(const Stn& s, int a, int b, int c, int d)
 {
     if (a < s.nv0 && b < s.nv0 && c < s.nv0 && d < s.nv0) return incircle(s.pts[a], s.pts[b], s.pts[c], s.pts[d]);
+    const int o = incircle_filter(stn_dpt(s, a), stn_dpt(s, b), stn_dpt(s, c), stn_dpt(s, d));
+    if (o) return o;
     return incircle_h(stn_pt(s, a), stn_pt(s, b), stn_pt(s, c), stn_pt(s, d));
 }
 
