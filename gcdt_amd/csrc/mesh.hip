@@ -2176,6 +2176,83 @@ __global__ __launch_bounds__(kBlock) void k_flip_fix(E e, const int* list, const
         e.fix(list[i], epoch);
 }
 
+// One flip round of at most SHORT_MAX triangles in one workgroup: its list and
+// the listed triangles' records stay in LDS from round to round (kept: the
+// records are there), four lanes share a triangle, one an edge, and whoever
+// tested the edge that wins flips it from the records it holds.  Only the
+// neighbour slots are read again for that: the test settles them, in records
+// of other lanes too.  Returns the length of the next list; lf receives the
+// flipped triangles, *nf their count.
+//
+// Such a round is a chain of waits: list, record, neighbours, up to three
+// in-circle tests in a row (0.4 us each for a lone wave), claims, and in the
+// apply list, record, neighbour and stores again.
+constexpr int SHORT_MAX = TAIL_BS / 4;
+
+__device__ inline int short_round(const FlipP& f, int* list, FRec* rec, bool kept, int n, unsigned ep,
+                                  const LdsClaims& cl, const LdsClaims& next, int* n2, int* nf, int q, int* lf)
+{
+    const int i = (int)threadIdx.x >> 2, k = (int)threadIdx.x & 3;
+    const int lane = (int)threadIdx.x & 63, lead = lane & ~3;
+    const bool on = ((int)(threadIdx.x & ~63u) >> 2) < n;  // the wave has a triangle
+    int t = -1, nn = -1, cand = 3;
+    FRec r, rn;
+    unsigned long long key = 0ull;
+    if (on) {
+        bool hit = false;
+        if (i < n && k < 3) {
+            t = list[i];
+            r = kept ? rec_load(&rec[i]) : rec_load(&f.r[t]);
+            hit = flip_fixtest_edge(f, t, r, k, ep, &nn, &rn);
+        }
+        const unsigned m = (unsigned)(__ballot(hit) >> lead) & 7u;
+        cand = m ? __ffsll((long long)m) - 1 : 3;
+        t = __shfl(t, lead, 64);
+        nn = __shfl(nn, lead + cand, 64);
+        key = ((unsigned long long)ep << 32) | (unsigned)(3 * t + cand);
+        if (cand != 3 && k < 2) cl.max(f, k == 0 ? t : nn, key);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        n2[q ^ 1] = 0;
+        nf[q ^ 1] = 0;
+    }
+    for (int j = threadIdx.x; j < LCL_CAP; j += TAIL_BS) {
+        next.tag[j] = -1;
+        next.key[j] = 0ull;
+    }
+    if (on) {
+        const unsigned long long own = cand != 3 && k < 2 ? cl.find(k == 0 ? t : nn) : 0ull;
+        const unsigned long long ct = __shfl(own, lead, 64), cn = __shfl(own, lead + 1, 64);
+        int res = 0;  // as flip_apply_p
+        if (cand != 3) {
+            if (ct == key) res = cn == key ? 2 : 1;
+            else res = (ct >> 32) == ep && cl.find((int)((ct & 0xffffffffu) / 3)) == ct ? 3 : 1;
+        }
+        int b = wave_alloc(k == 0 ? (res == 1 ? 1 : res == 2 ? 2 : 0) : 0, &n2[q]);
+        const int w = wave_alloc(k == 0 && res == 2 ? 2 : 0, &nf[q]);
+        b = __shfl(b, lead, 64);
+        if (k == 0 && res == 2) {
+            lf[w] = t;
+            lf[w + 1] = nn;
+        }
+        if (res == 1 && k == 0) {
+            list[b] = t;
+            r.a = f.r[t].a;
+            if (b < SHORT_MAX) rec_store(&rec[b], r.v, r.a, r.p[0], r.p[1], r.p[2], r.meta, r.stamp, 0ull);
+        } else if (res == 2 && k == cand) {
+            r.a = f.r[t].a;
+            rn.a = f.r[nn].a;
+            flip_records(&f.r[t], &f.r[nn], t, r, k, nn, rn, ep, key);
+            list[b] = t;
+            list[b + 1] = nn;
+            if (b + 1 < SHORT_MAX) flip_records(&rec[b], &rec[b + 1], t, r, k, nn, rn, ep, key);
+        }
+    }
+    __syncthreads();
+    return n2[q];
+}
+
 // Persistent single-workgroup tail of the flip rounds.
 template <class E>
 __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int* lf, int n, int cap, unsigned epoch0,
@@ -2189,6 +2266,9 @@ __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int*
     // table per round parity: the other one is cleared while a round applies
     __shared__ int s_tag[2][LCL_CAP];
     __shared__ unsigned long long s_key[2][LCL_CAP];
+    // list and records of the rounds of at most SHORT_MAX triangles
+    __shared__ int s_list[E::kFused ? 2 * SHORT_MAX : 1];
+    __shared__ int4 s_rec[E::kFused ? SHORT_MAX * (sizeof(FRec) / sizeof(int4)) : 1];
     unsigned ep = epoch0;  // A, B and lf hold cap entries each, n <= cap
     int r = 0, err = 0, flips = 0;
     int nf = 0;
@@ -2203,6 +2283,32 @@ __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int*
     }
     __syncthreads();
     while (n > 0 && r < max_rounds) {
+        if constexpr (E::kFused) {
+            if (n <= SHORT_MAX) {
+                for (int i = threadIdx.x; i < n; i += TAIL_BS) s_list[i] = A[i];
+                __syncthreads();
+                for (bool kept = false; n > 0 && n <= SHORT_MAX && r < max_rounds; kept = true) {
+                    const int q = r & 1;
+                    const int n2 = short_round(e.f, s_list, (FRec*)s_rec, kept, n, ep, LdsClaims{s_tag[q], s_key[q]},
+                                               LdsClaims{s_tag[q ^ 1], s_key[q ^ 1]}, s_n2, s_nf, q, lf);
+                    nf = s_nf[q];
+                    if (n2 > 0 && nf == 0) {
+                        err = 1;
+                        break;
+                    }
+                    flips += nf / 2;
+                    n = n2;
+                    ep++;
+                    r++;
+                }
+                if (err) break;
+                if (n > SHORT_MAX) {
+                    for (int i = threadIdx.x; i < n; i += TAIL_BS) A[i] = s_list[i];
+                    __syncthreads();
+                }
+                continue;
+            }
+        }
         const int q = r & 1;
         const bool lds = E::kFused && n <= LCL_MAX_LIST;
         const LdsClaims cl{s_tag[q], s_key[q]};

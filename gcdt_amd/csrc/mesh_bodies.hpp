@@ -689,10 +689,47 @@ __host__ __device__ inline bool flip_fixtest_p(const FlipP& f, int t, unsigned e
     return cand != 3;
 }
 
+// Edge k of triangle t (record r) in flip_fixtest_p, for rounds in which every
+// listed triangle tests: settles the slot if t flipped last round, and tests
+// the edge.  True if the edge needs a flip; *nout and *rn are then the
+// triangle across it and its record.
+__host__ __device__ inline bool flip_fixtest_edge(const FlipP& f, int t, const FRec& r, int k, unsigned epoch, int* nout,
+                                                  FRec* rn)
+{
+    const int prev = (int)epoch - 1;
+    const bool cons = (r.meta >> k) & 1;
+    const int ps = rec_pslot(r.meta);
+    const bool flipped = r.stamp == prev && ps < 3;
+    const int partner = flipped ? get3(r.a, ps) : -1;
+    const int av = get3(r.a, k);
+    const bool pend = flipped && k != ps;
+    if (av < 0 || (!pend && (cons || av == partner))) return false;
+    int n = av;
+    *rn = rec_load(&f.r[av]);
+    const int u = get3(r.v, nx3(k)), v = get3(r.v, pv3(k));
+    if (!has2(rn->v, u, v)) {
+        // av flipped last round and the edge went to its partner
+        if (rn->stamp != prev) {
+            at_or(f.err, MERR_ADJ);
+            return false;
+        }
+        n = get3(rn->a, rec_pslot(rn->meta));
+        *rn = rec_load(&f.r[n]);
+        if (pend) (&f.r[t].a.x)[k] = n;
+    } else if (pend && rn->stamp != prev) {
+        // the outer edge that kept its triangle already points here
+        const int j = slot_other(rn->v, u, v);
+        if (get3(rn->a, j) != t) (&f.r[av].a.x)[j] = t;
+    }
+    if (cons || n == partner) return false;
+    *nout = n;
+    return incircle(r.p[0], r.p[1], r.p[2], rec_pt(*rn, slot_other(rn->v, u, v))) > 0;
+}
+
 // Flips edge k of t (record r) with its neighbour n (record rn): both records
-// are written whole, the claim word as given.
+// are written whole, to *pt and *pn, the claim word as given.
 // t = (p,u,v), n = (o,v,u)  ->  t = (p,u,o) [partner in slot 1], n = (p,o,v) [partner in slot 2]
-__host__ __device__ inline void flip_records(const FlipP& f, int t, const FRec& r, int k, int n, const FRec& rn,
+__host__ __device__ inline void flip_records(FRec* pt, FRec* pn, int t, const FRec& r, int k, int n, const FRec& rn,
                                              unsigned epoch, unsigned long long key)
 {
     const int kn = nx3(k), kp = pv3(k);
@@ -703,10 +740,10 @@ __host__ __device__ inline void flip_records(const FlipP& f, int t, const FRec& 
     const int cft = r.meta & 7, cfn = rn.meta & 7;
     const int2 pp = rec_pt(r, k), pu = rec_pt(r, kn), pv = rec_pt(r, kp), po = rec_pt(rn, j);
     const int mk = (int)epoch + 1;
-    rec_store(&f.r[t], make_int3(p, u, o), make_int3(get3(rn.a, jn), n, get3(r.a, kp)), pp, pu, po,
+    rec_store(pt, make_int3(p, u, o), make_int3(get3(rn.a, jn), n, get3(r.a, kp)), pp, pu, po,
               rec_with_mark(((cfn >> jn) & 1) | (((cft >> kp) & 1) << 2) | FREC_NOCAND | (1 << 5), mk), (int)epoch,
               key);
-    rec_store(&f.r[n], make_int3(p, o, v), make_int3(get3(rn.a, jp), get3(r.a, kn), t), pp, po, pv,
+    rec_store(pn, make_int3(p, o, v), make_int3(get3(rn.a, jp), get3(r.a, kn), t), pp, po, pv,
               rec_with_mark(((cfn >> jp) & 1) | (((cft >> kn) & 1) << 1) | FREC_NOCAND | (2 << 5), mk), (int)epoch,
               key);
 }
@@ -736,7 +773,7 @@ __host__ __device__ inline int flip_apply_peer(const FlipP& f, int e, unsigned e
     const int n = get3(r.a, k);
     const FRec rn = rec_load(&f.r[n]);
     if (rn.claim != key || (n > t && cl.prop[n] == cl.tag)) return 1;
-    flip_records(f, t, r, k, n, rn, epoch, key);
+    flip_records(&f.r[t], &f.r[n], t, r, k, n, rn, epoch, key);
     *nout = n;
     return 2;
 }
@@ -774,7 +811,7 @@ __host__ __device__ inline int flip_apply_p(const FlipP& f, int t, unsigned epoc
     const FRec rn = rec_load(&f.r[n]);
     const unsigned long long cn = cl.template get<COH>(f, n, rn.claim);
     if (cn != key) return 1;
-    flip_records(f, t, r, k, n, rn, epoch, key);
+    flip_records(&f.r[t], &f.r[n], t, r, k, n, rn, epoch, key);
     *nout = n;
     return 2;
 }
