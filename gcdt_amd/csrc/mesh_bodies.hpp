@@ -36,6 +36,16 @@ __device__ inline unsigned long long ld_u64(const unsigned long long* p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// The same for words that only one workgroup touches while it runs: performed
+// in its own L2 (a device-scope atomic goes to memory and back).
+__device__ inline unsigned long long at_max_wg(unsigned long long* p, unsigned long long v)
+{
+    return __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline unsigned long long ld_u64_wg(const unsigned long long* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 // COH: inside a persistent workgroup (atomic load); otherwise a kernel
 // boundary separates the claims from this read and a plain load suffices.
 template <bool COH>
@@ -67,6 +77,12 @@ struct Mesh {
 };
 
 __host__ __device__ inline int& A3(const Mesh& m, int t, int k) { return ((int*)m.adj)[3 * (long long)t + k]; }
+
+// coordinate k of three by selects over values
+__host__ __device__ inline int2 sel_pt(int2 p0, int2 p1, int2 p2, int k)
+{
+    return make_int2(k == 0 ? p0.x : (k == 1 ? p1.x : p2.x), k == 0 ? p0.y : (k == 1 ? p1.y : p2.y));
+}
 
 // ------------------------------------------------------------------ insertion
 
@@ -117,13 +133,20 @@ __host__ __device__ inline unsigned closeness_rank_edge(int2 U, int2 V, int2 P, 
     return (cls << 9) | (hash32((uint32_t)p) & 511u);
 }
 
+// closeness of point p (at P) in triangle (A, B, C), or on its edge opposite slot k < 3
+__host__ __device__ inline unsigned ins_close(const Ins& s, int2 A, int2 B, int2 C, int2 P, int p, int k)
+{
+    if (s.pivot != 1) return hash32((uint32_t)p) & 2047u;
+    return k < 3 ? closeness_rank_edge(sel_pt(A, B, C, nx3(k)), sel_pt(A, B, C, pv3(k)), P, p)
+                 : closeness_rank(A, B, C, P, p);
+}
+
 __host__ __device__ inline unsigned long long ins_key_of(const Ins& s, int p, int t, int k, unsigned epoch)
 {
     unsigned close;
     if (s.pivot == 1) {
         int3 tv = s.m.tri[t];
-        close = k < 3 ? closeness_rank_edge(s.m.pts[get3(tv, nx3(k))], s.m.pts[get3(tv, pv3(k))], s.m.pts[p], p)
-                      : closeness_rank(s.m.pts[tv.x], s.m.pts[tv.y], s.m.pts[tv.z], s.m.pts[p], p);
+        close = ins_close(s, s.m.pts[tv.x], s.m.pts[tv.y], s.m.pts[tv.z], s.m.pts[p], p, k);
     } else {
         close = hash32((uint32_t)p) & 2047u;
     }
@@ -190,12 +213,12 @@ __host__ __device__ inline int ins_need(const Ins& s, int p, unsigned epoch)
     return ld_claim<COH>(&s.claim[A3(s.m, t, k)]) == key ? 4 : 0;
 }
 
-// Split the triangle(s) of winner p into new slots [base, base+need).
+// Split the triangle(s) of winner p (at l = loc[p]) into new slots
+// [base, base+need).
 // Reference: addNewTriangle_step2, rawMesh.cu:200-280 (same child layout).
-__host__ __device__ inline void ins_split(const Ins& s, int p, int base)
+__host__ __device__ inline void ins_split_at(const Ins& s, int p, int l, int base)
 {
     const Mesh& m = s.m;
-    int l = s.loc[p];
     int t = l >> 2, k = l & 3;
     int3 tv = m.tri[t];
     int3 ta = m.adj[t];
@@ -234,6 +257,8 @@ __host__ __device__ inline void ins_split(const Ins& s, int p, int base)
     }
     s.loc[p] = -1;
 }
+
+__host__ __device__ inline void ins_split(const Ins& s, int p, int base) { ins_split_at(s, p, s.loc[p], base); }
 
 // Resolve the outer adjacency of new slot c after all splits of the round:
 // a marked entry names the parent's old neighbour m; if m was split in the
@@ -312,6 +337,52 @@ __host__ __device__ inline int ins_relocate(const Ins& s, int p)
     at_or(s.err, MERR_LOCATE);
     s.loc[p] = -1;
     return 0;
+}
+
+// The same for the tail's short lists, where the claim words still name the
+// point that split a triangle: the children of an interior split follow from
+// the parent's vertices and that point, so the two reads of a level go out
+// together.  *l becomes the point's new place, *close its closeness there.
+// Returns 1 if p stays pending.
+__host__ __device__ inline int ins_relocate_at(const Ins& s, int p, int* l, unsigned* close)
+{
+    const Mesh& m = s.m;
+    const int t = *l >> 2;
+    const int sn = m.sons[t];
+    const int q = (int)(unsigned)s.claim[t];
+    const int3 tv = m.tri[t];
+    const int2 P = m.pts[p];
+    if (sn == -1) return 1;
+    const int c0 = sn > 0 ? sn : -sn, nc = sn > 0 ? 3 : 2;
+    int r = -1, c = c0;
+    int2 A, B, C;
+    if (sn > 0) {
+        const int2 Q = m.pts[q], X = m.pts[tv.x], Y = m.pts[tv.y], Z = m.pts[tv.z];
+        for (int j = 0; j < 3 && r == -1; j++) {
+            A = Q;
+            B = sel_pt(Y, Z, X, j);
+            C = sel_pt(Z, X, Y, j);
+            r = classify(A, B, C, P);
+            c = c0 + j;
+        }
+    } else {
+        for (int j = 0; j < nc && r == -1; j++) {
+            const int3 cv = m.tri[c0 + j];
+            A = m.pts[cv.x];
+            B = m.pts[cv.y];
+            C = m.pts[cv.z];
+            r = classify(A, B, C, P);
+            c = c0 + j;
+        }
+    }
+    if (r < 0) {
+        at_or(s.err, r == -2 ? MERR_DUPLICATE : MERR_LOCATE);
+        s.loc[p] = -1;
+        return 0;
+    }
+    *l = c * 4 + r;
+    *close = ins_close(s, A, B, C, P, p, r);
+    return 1;
 }
 
 // ------------------------------------------------------------------ flips
@@ -508,12 +579,8 @@ __host__ __device__ inline void rec_store(FRec* p, const int3& v, const int3& a,
     q[3] = make_int4(meta, stamp, (int)(unsigned)claim, (int)(unsigned)(claim >> 32));
 }
 
-// coordinate k of a record by selects over values (a runtime index into the
-// local copy, or selects through a reference, would put it on the stack)
-__host__ __device__ inline int2 sel_pt(int2 p0, int2 p1, int2 p2, int k)
-{
-    return make_int2(k == 0 ? p0.x : (k == 1 ? p1.x : p2.x), k == 0 ? p0.y : (k == 1 ? p1.y : p2.y));
-}
+// by selects over values (a runtime index into the local copy, or selects
+// through a reference, would put it on the stack)
 #define rec_pt(r, k) sel_pt((r).p[0], (r).p[1], (r).p[2], (k))
 
 struct FlipP {

@@ -248,6 +248,14 @@ inline void __hip_atomic_store(T* p, V v, int, int)
 {
     *p = (T)v;
 }
+template <class T, class V>
+inline T __hip_atomic_fetch_max(T* p, V v, int, int)
+{
+    ::emu::atomic_point();
+    T o = *p;
+    if ((T)v > o) *p = (T)v;
+    return o;
+}
 inline void __threadfence() {}
 inline void __threadfence_block() {}
 
