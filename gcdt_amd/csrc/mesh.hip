@@ -1652,11 +1652,12 @@ __device__ inline void claim_combined_w(unsigned long long* claim, int t, int t2
     *f2 = t2 >= 0 && claim_first(atomicMax(&claim[t2], key), epoch);
 }
 
-// Claims of `epoch` for up to IT points per thread (p < 0: none), appending
-// first-claimed triangles to wl.  Block-uniform: every thread of the block
-// calls it.
+// Claims of `epoch` for up to IT points per thread (l: their places, < 0 none;
+// close: their closeness there), appending first-claimed triangles to wl.
+// Block-uniform: every thread of the block calls it.
 template <int IT>
-__device__ inline void claim_items(const Ins& s, const int (&pp)[IT], unsigned epoch, Staged<STAGE_CAP>& sw)
+__device__ inline void claim_items(const Ins& s, const int (&p)[IT], const int (&l)[IT], const unsigned (&close)[IT],
+                                   unsigned epoch, Staged<STAGE_CAP>& sw)
 {
     int wt[2 * IT];
     int nq = 0;
@@ -1664,7 +1665,12 @@ __device__ inline void claim_items(const Ins& s, const int (&pp)[IT], unsigned e
     for (int j = 0; j < IT; j++) {
         int t = -1, t2 = -1;
         unsigned long long key = 0;
-        if (pp[j] >= 0) t = ins_key_round(s, pp[j], epoch, &key, &t2);
+        if (l[j] >= 0) {
+            const int k = l[j] & 3;
+            t = l[j] >> 2;
+            key = ins_key(p[j], k < 3, close[j], epoch);
+            if (k < 3) t2 = ins_edge_neighbour(s, t, k);
+        }
         bool f1, f2;
         claim_combined_w(s.claim, t, t2, key, epoch, &f1, &f2);
         wt[2 * j] = f1 ? t : -1;
@@ -1677,6 +1683,19 @@ __device__ inline void claim_items(const Ins& s, const int (&pp)[IT], unsigned e
         if (wt[j] >= 0) sw.buf[b++] = wt[j];
 }
 
+// The first tile's entries of a list, read beside its length (which a launch
+// otherwise waits for alone): entries past the length are read and not used.
+template <int IT>
+__device__ inline void first_tile(const int* list, long long cap, int (&v)[IT])
+{
+#pragma unroll
+    for (int j = 0; j < IT; j++) {
+        const long long i = (long long)blockIdx.x * kBlock * IT + j * kBlock + threadIdx.x;
+        v[j] = list && i < cap ? list[i] : 0;
+    }
+}
+#define TILE_ITEM(list, first, base, i, j, IT) ((base) == (long long)blockIdx.x * kBlock * (IT) ? (first)[j] : (list)[i])
+
 // First claims of a run of rounds (later rounds claim inside k_ins_reloc).
 __global__ __launch_bounds__(kBlock) void k_ins_claim_w(Ins s, const int* list, const int* cnt, unsigned epoch, int* wl,
                                                         int* nw, int wcap)
@@ -1688,8 +1707,17 @@ __global__ __launch_bounds__(kBlock) void k_ins_claim_w(Ins s, const int* list, 
     TILE_LOOP(base, n, kBlock)
     {
         long long i = base + threadIdx.x;
-        int pp[1] = {i < n ? list[i] : -1};
-        claim_items<1>(s, pp, epoch, sw);
+        int p[1] = {-1}, l[1] = {-1};
+        unsigned close[1] = {0};
+        if (i < n) {
+            p[0] = list[i];
+            l[0] = s.loc[p[0]];
+            if (l[0] >= 0) {
+                const int3 tv = s.m.tri[l[0] >> 2];
+                close[0] = ins_close(s, s.m.pts[tv.x], s.m.pts[tv.y], s.m.pts[tv.z], s.m.pts[p[0]], p[0], l[0] & 3);
+            }
+        }
+        claim_items<1>(s, p, l, close, epoch, sw);
     }
     sw.flush();
 }
@@ -1708,15 +1736,17 @@ void with_items(int v, F&& f)
 // winning point; an on-edge winner splits from its own triangle (loc), not
 // from the second one it claimed.
 template <int INS_ITEMS>
-__global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, const int* cnt, int lcap, unsigned epoch,
-                                                      int* set, RoundSnap snap)
+__global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, const int* cnt, int lcap, int* set,
+                                                      RoundSnap snap)
 {
     round_snap_store(snap);
+    int pre[INS_ITEMS];
+    first_tile(list, lcap, pre);
     int n = min(*cnt, lcap);  // an overfull list has flagged MERR_CAPACITY
     const int first = set[R_BASE];
     TILE_LOOP(base, n, kBlock * INS_ITEMS)
     {
-        int pp[INS_ITEMS], need[INS_ITEMS];
+        int pp[INS_ITEMS], ll[INS_ITEMS], need[INS_ITEMS];
         int tot = 0;
 #pragma unroll
         for (int j = 0; j < INS_ITEMS; j++) {
@@ -1724,12 +1754,15 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
             pp[j] = -1;
             need[j] = 0;
             if (i < n) {
-                int t = list[i];
-                int p = (int)(unsigned)s.claim[t];
-                int l = s.loc[p];
+                const int t = TILE_ITEM(list, pre, base, i, j, INS_ITEMS);
+                const unsigned long long w = s.claim[t];
+                const int p = (int)(unsigned)w;
+                const int l = s.loc[p];
                 if (l >= 0 && (l >> 2) == t) {
+                    const int k = l & 3;
                     pp[j] = p;
-                    need[j] = ins_need<false>(s, p, epoch);
+                    ll[j] = l;
+                    need[j] = k == 3 ? 3 : (s.claim[A3(s.m, t, k)] == w ? 4 : 0);
                 }
             }
             tot += need[j];
@@ -1739,7 +1772,7 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
         for (int j = 0; j < INS_ITEMS; j++) {
             if (need[j]) {
                 if (b + need[j] > s.cap) atomicOr(s.err, MERR_CAPACITY);
-                else ins_split(s, pp[j], b);
+                else ins_split_at(s, pp[j], ll[j], b);
                 b += need[j];
             }
         }
@@ -1753,13 +1786,15 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
 // launch has not settled yet (ins_edge_neighbour).  The slots of the next round
 // begin where this round's end.
 template <int INS_ITEMS>
-__global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, const int* cnt, int* list2,
+__global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, const int* cnt, int lcap, int* list2,
                                                       unsigned next_ep, int* wl, int wcap, int* set, int* next_set)
 {
     __shared__ int s_buf[STAGE_CAP], s_buf2[STAGE_CAP];
     __shared__ int s_base, s_base2;
     Staged<STAGE_CAP> sl(s_buf, &s_base, list2, &set[R_NEXT]),
         sw(s_buf2, &s_base2, wl, &set[R_NW], wcap, s.err, MERR_CAPACITY);
+    int pre[INS_ITEMS];
+    first_tile(list, lcap, pre);
     const int tb = set[R_BASE], te = tb + set[R_NEW];
     if (blockIdx.x == 0 && threadIdx.x == 0) next_set[R_BASE] = te;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x + tb; i < min(te, s.cap);
@@ -1768,23 +1803,29 @@ __global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, co
     int n = *cnt;
     TILE_LOOP(base, n, kBlock * INS_ITEMS)
     {
-        int keep[INS_ITEMS];
+        int p[INS_ITEMS], l[INS_ITEMS];
+        unsigned close[INS_ITEMS];
         int tot = 0;
 #pragma unroll
         for (int j = 0; j < INS_ITEMS; j++) {
             long long i = base + (long long)j * kBlock + threadIdx.x;
-            keep[j] = -1;
+            l[j] = -1;
             if (i < n) {
-                int p = list[i];
-                if (ins_relocate(s, p)) keep[j] = p;
+                p[j] = TILE_ITEM(list, pre, base, i, j, INS_ITEMS);
+                const int at = s.loc[p[j]];
+                int to = at;
+                if (at >= 0 && ins_relocate_at<CLAIM_LAUNCH, true>(s, p[j], &to, &close[j])) {
+                    if (to != at) s.loc[p[j]] = to;
+                    l[j] = to;
+                }
             }
-            tot += keep[j] >= 0;
+            tot += l[j] >= 0;
         }
         int b = sl.reserve(tot);
 #pragma unroll
         for (int j = 0; j < INS_ITEMS; j++)
-            if (keep[j] >= 0) s_buf[b++] = keep[j];
-        claim_items<INS_ITEMS>(s, keep, next_ep, sw);
+            if (l[j] >= 0) s_buf[b++] = p[j];
+        claim_items<INS_ITEMS>(s, p, l, close, next_ep, sw);
     }
     sl.flush();
     sw.flush();
@@ -1908,7 +1949,7 @@ __device__ inline int ins_short_rounds(const Ins& s, const int* P, int n, InsLis
                 l = in.l[i];
                 close = in.close[i];
             }
-            const bool keep = l >= 0 && ins_relocate_at(s, p, &l, &close);
+            const bool keep = l >= 0 && ins_relocate_at<CLAIM_WG, false>(s, p, &l, &close);
             const int b = wave_alloc(keep ? 1 : 0, &s_np[q]);
             if (keep) {
                 out.p[b] = p;
@@ -2047,15 +2088,14 @@ int insert_rounds(Ctx& c, const Ins& s_in, DBuf<int>& pend, DBuf<int>& pend2, in
         with_items(c.ins_items, [&](auto it) {
             constexpr int IT = decltype(it)::value;
             ProfScope ps("ins_split", c.st, 0);
-            k_ins_split<IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(s, W, in + R_NW, (int)wcap, ep, set,
-                                                                                 snap);
+            k_ins_split<IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(s, W, in + R_NW, (int)wcap, set, snap);
             GCDT_LAUNCH_CHECK();
         });
         with_items(c.ins_items, [&](auto it) {
             constexpr int IT = decltype(it)::value;
             ProfScope ps("ins_reloc", c.st, 0);
             k_ins_reloc<IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
-                s, P, in + R_NEXT, P2, ep + 1, W2, (int)wcap, set, c.round_set(r + 1));
+                s, P, in + R_NEXT, npend, P2, ep + 1, W2, (int)wcap, set, c.round_set(r + 1));
             GCDT_LAUNCH_CHECK();
         });
         std::swap(P, P2);
@@ -2230,6 +2270,8 @@ __global__ __launch_bounds__(kBlock) void k_flip_test(E e, const int* list, cons
     // a triangle proposes at most once per round, so `prop` (cap entries)
     // cannot overflow; a miscount flags MERR_CAPACITY instead of writing past it
     Staged<STAGE_CAP> sp(s_buf, &s_base, prop, nprop, cap, eflag, MERR_CAPACITY);
+    int pre[FT_ITEMS];
+    first_tile(list, lcap, pre);
     int n = min(*cnt, lcap);
     TILE_LOOP(base, n, kBlock * FT_ITEMS)
     {
@@ -2240,7 +2282,7 @@ __global__ __launch_bounds__(kBlock) void k_flip_test(E e, const int* list, cons
             q[j] = -1;
             long long i = base + (long long)j * kBlock + threadIdx.x;
             if (i < n) {
-                q[j] = e.propose(list ? list[i] : (int)i, epoch, list == nullptr, single != 0);
+                q[j] = e.propose(list ? TILE_ITEM(list, pre, base, i, j, FT_ITEMS) : (int)i, epoch, list == nullptr, single != 0);
             }
             nq += q[j] >= 0;
         }
@@ -2256,13 +2298,18 @@ template <class E, int FA_ITEMS>
 __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, const int* cnt, unsigned epoch, int* list2,
                                                        int* cnt2, int* flipped, int* nflip, int cap, int* eflag)
 {
-    __shared__ int s_buf[STAGE_CAP], s_buf2[STAGE_CAP];
+    __shared__ int s_buf[STAGE_CAP], s_buf2[E::kFused ? 1 : STAGE_CAP];
     __shared__ int s_base, s_base2;
     // each triangle enters the next list at most once per round (a lost
     // proposer that keeps its own claim is flipped by no one), so both lists
     // hold at most cap entries; a miscount flags MERR_CAPACITY
     Staged<STAGE_CAP> sq(s_buf, &s_base, list2, cnt2, cap, eflag, MERR_CAPACITY),
         sf(s_buf2, &s_base2, flipped, nflip, cap, eflag, MERR_CAPACITY);
+    __shared__ int s_nf;  // fused engines need only the number of flipped triangles
+    if (E::kFused && threadIdx.x == 0) s_nf = 0;
+    int flips = 0;
+    int pre[FA_ITEMS];
+    first_tile(list, cap, pre);
     int n = min(*cnt, cap);
     TILE_LOOP(base, n, kBlock * FA_ITEMS)
     {
@@ -2275,7 +2322,7 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
             long long i = base + (long long)j * kBlock + threadIdx.x;
             if (i < n) {
                 int t, nn = -1;
-                int res = e.apply_round(list[i], epoch, &t, &nn);
+                int res = e.apply_round(TILE_ITEM(list, pre, base, i, j, FA_ITEMS), epoch, &t, &nn);
                 if (res == 1) e.set_mark(t, (int)epoch + 1);
                 if (res == 1 || res == 2) qa[j] = t;
                 if (res == 2) qb[j] = nn;
@@ -2284,19 +2331,28 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
             nf += (qb[j] >= 0) ? 2 : 0;
         }
         int b = sq.reserve(nq);
-        int fb = sf.reserve(nf);
+        int fb = E::kFused ? 0 : sf.reserve(nf);
+        flips += nf;
 #pragma unroll
         for (int j = 0; j < FA_ITEMS; j++) {
             if (qa[j] >= 0) s_buf[b++] = qa[j];
             if (qb[j] >= 0) {
                 s_buf[b++] = qb[j];
-                s_buf2[fb++] = qa[j];
-                s_buf2[fb++] = qb[j];
+                if (!E::kFused) {
+                    s_buf2[fb++] = qa[j];
+                    s_buf2[fb++] = qb[j];
+                }
             }
         }
     }
     sq.flush();
-    sf.flush();
+    if (E::kFused) {  // after the barrier in flush
+        wave_alloc(flips, &s_nf);
+        __syncthreads();
+        if (threadIdx.x == 0 && s_nf) atomicAdd(nflip, s_nf);
+    } else {
+        sf.flush();
+    }
 }
 
 template <class E>
@@ -2660,15 +2716,9 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
     if (r >= 1) {
         c.round_snapshot(r);
         check_round(c.round_wait(r));
-        // the last round's flips are settled by the tail (or the fix below)
+        // the last round's flips are settled by the tail: flipped triangles are
+        // in the next list, so a round with flips is never the last
         if (E::kFused) prof_add_items("flip_test_fix", settled - n_flip);
-        if (E::kFused && done && n_flip > 0) {
-            // settle the last round's flips (no test follows; the tail's first
-            // test settles them when the tail runs)
-            ProfScope ps("flip_fix", c.st, n_flip);
-            k_flip_fix<E><<<grid_for(n_flip), kBlock, 0, c.st>>>(e, lf.p, c.round_set(r) + R_FLIP, T, c.epoch);
-            GCDT_LAUNCH_CHECK();
-        }
     }
     if (!done) {
         // the rest in one persistent workgroup

@@ -54,6 +54,14 @@ __host__ __device__ inline unsigned long long ld_claim(const unsigned long long*
     if (COH) return ld_u64(p);
     return *p;
 }
+// who made the claims that a round reads: an earlier launch, this workgroup at
+// device scope, this workgroup in its own L2
+enum { CLAIM_LAUNCH = 0, CLAIM_DEVICE = 1, CLAIM_WG = 2 };
+template <int FROM>
+__host__ __device__ inline unsigned long long ld_claim_from(const unsigned long long* p)
+{
+    return FROM == CLAIM_DEVICE ? ld_u64(p) : (FROM == CLAIM_WG ? ld_u64_wg(p) : *p);
+}
 
 enum : int {
     MERR_CAPACITY = 1,     // triangle slots exhausted
@@ -90,7 +98,7 @@ struct Ins {
     Mesh m;
     int* loc;
     unsigned long long* claim;
-    unsigned long long* pkey;  // per point: its claim key of the current round
+    unsigned long long* pkey;  // per point: its claim key of the current round (ins_claim, ins_need)
     int cap;
     int pivot;                 // 0: random among the triangle's points, 1: central ones first
     int* err;
@@ -201,16 +209,15 @@ __host__ __device__ inline void ins_claim(const Ins& s, int p, unsigned epoch)
 }
 
 // slots needed by p if it won every triangle it claimed (3 interior, 4 edge)
-template <bool COH = true>
 __host__ __device__ inline int ins_need(const Ins& s, int p, unsigned epoch)
 {
     int l = s.loc[p];
     if (l < 0) return 0;
     int t = l >> 2, k = l & 3;
     unsigned long long key = s.pkey[p];
-    if (ld_claim<COH>(&s.claim[t]) != key) return 0;
+    if (ld_claim<true>(&s.claim[t]) != key) return 0;
     if (k == 3) return 3;
-    return ld_claim<COH>(&s.claim[A3(s.m, t, k)]) == key ? 4 : 0;
+    return ld_claim<true>(&s.claim[A3(s.m, t, k)]) == key ? 4 : 0;
 }
 
 // Split the triangle(s) of winner p (at l = loc[p]) into new slots
@@ -308,71 +315,53 @@ __host__ __device__ inline int classify(int2 A, int2 B, int2 C, int2 P)
     return o0 == 0 ? 0 : (o1 == 0 ? 1 : 2);
 }
 
-// After the splits: move a still-pending point into the child of its split
-// triangle that contains it.  Returns 1 if p stays pending.
-// Reference: scatterPoints/scatterPoint, rawMesh.cu:338-463.
-__host__ __device__ inline int ins_relocate(const Ins& s, int p)
-{
-    const Mesh& m = s.m;
-    int l = s.loc[p];
-    if (l < 0) return 0;
-    int t = l >> 2;
-    int sn = m.sons[t];
-    if (sn == -1) return 1;  // untouched (an on-edge point keeps its edge: see ins_fix)
-    int c0 = sn > 0 ? sn : -sn, nc = sn > 0 ? 3 : 2;
-    int2 P = m.pts[p];
-    for (int c = c0; c < c0 + nc; c++) {
-        int3 tv = m.tri[c];
-        int r = classify(m.pts[tv.x], m.pts[tv.y], m.pts[tv.z], P);
-        if (r >= 0) {
-            s.loc[p] = c * 4 + r;
-            return 1;
-        }
-        if (r == -2) {
-            at_or(s.err, MERR_DUPLICATE);
-            s.loc[p] = -1;
-            return 0;
-        }
-    }
-    at_or(s.err, MERR_LOCATE);
-    s.loc[p] = -1;
-    return 0;
-}
-
-// The same for the tail's short lists, where the claim words still name the
-// point that split a triangle: the children of an interior split follow from
-// the parent's vertices and that point, so the two reads of a level go out
-// together.  *l becomes the point's new place, *close its closeness there.
+// After the splits: move a still-pending point (at *l) into the child of its
+// split triangle that contains it; *l becomes its new place and *close its
+// closeness there, which an untouched point keeps (RANK: computed for it too).
 // Returns 1 if p stays pending.
+// Reference: scatterPoints/scatterPoint, rawMesh.cu:338-463.
+//
+// The claim word of a split triangle still names the point q that split it --
+// the next round claims only its children -- so the children (q,y,z), (q,z,x),
+// (q,x,y) of an interior split follow from the parent's vertices: the parent,
+// its sons and its claim are read together and then the four points, where
+// reading the children would put one more trip in between.  With P in the closed triangle
+// (on the edge opposite slot k < 3 of it, as recorded), its sides of qx, qy
+// and qz give the child and the edge of it.
+template <int FROM, bool RANK>
 __host__ __device__ inline int ins_relocate_at(const Ins& s, int p, int* l, unsigned* close)
 {
     const Mesh& m = s.m;
-    const int t = *l >> 2;
+    const int t = *l >> 2, k = *l & 3;
     const int sn = m.sons[t];
-    const int q = (int)(unsigned)s.claim[t];
+    const int q = (int)(unsigned)ld_claim_from<FROM>(&s.claim[t]);
     const int3 tv = m.tri[t];
     const int2 P = m.pts[p];
-    if (sn == -1) return 1;
-    const int c0 = sn > 0 ? sn : -sn, nc = sn > 0 ? 3 : 2;
-    int r = -1, c = c0;
+    if (sn == -1) {  // untouched (an on-edge point keeps its edge: see ins_fix)
+        if (RANK) *close = ins_close(s, m.pts[tv.x], m.pts[tv.y], m.pts[tv.z], P, p, k);
+        return 1;
+    }
+    int r = -1, c = 0;
     int2 A, B, C;
     if (sn > 0) {
-        const int2 Q = m.pts[q], X = m.pts[tv.x], Y = m.pts[tv.y], Z = m.pts[tv.z];
-        for (int j = 0; j < 3 && r == -1; j++) {
-            A = Q;
-            B = sel_pt(Y, Z, X, j);
-            C = sel_pt(Z, X, Y, j);
-            r = classify(A, B, C, P);
-            c = c0 + j;
-        }
+        const int2 X = m.pts[tv.x], Y = m.pts[tv.y], Z = m.pts[tv.z];
+        A = m.pts[q];
+        const int sx = orient2d(A, X, P), sy = orient2d(A, Y, P), sz = orient2d(A, Z, P);
+        const int j = sy >= 0 && sz <= 0 ? 0 : (sz >= 0 && sx <= 0 ? 1 : (sx >= 0 && sy <= 0 ? 2 : 3));
+        B = sel_pt(Y, Z, X, j);
+        C = sel_pt(Z, X, Y, j);
+        const bool on0 = k == j, on1 = (j == 0 ? sz : (j == 1 ? sx : sy)) == 0,
+                   on2 = (j == 0 ? sy : (j == 1 ? sz : sx)) == 0;
+        if (j < 3) r = on0 + on1 + on2 > 1 ? -2 : (on0 ? 0 : (on1 ? 1 : (on2 ? 2 : 3)));
+        c = sn + j;
     } else {
-        for (int j = 0; j < nc && r == -1; j++) {
-            const int3 cv = m.tri[c0 + j];
+        for (int j = 0; j < 2 && r == -1; j++) {
+            const int3 cv = m.tri[j - sn];
             A = m.pts[cv.x];
             B = m.pts[cv.y];
             C = m.pts[cv.z];
             r = classify(A, B, C, P);
-            c = c0 + j;
+            c = j - sn;
         }
     }
     if (r < 0) {
@@ -382,6 +371,15 @@ __host__ __device__ inline int ins_relocate_at(const Ins& s, int p, int* l, unsi
     }
     *l = c * 4 + r;
     *close = ins_close(s, A, B, C, P, p, r);
+    return 1;
+}
+
+__host__ __device__ inline int ins_relocate(const Ins& s, int p)
+{
+    int l = s.loc[p];
+    unsigned close;
+    if (l < 0 || !ins_relocate_at<CLAIM_DEVICE, false>(s, p, &l, &close)) return 0;
+    s.loc[p] = l;
     return 1;
 }
 
