@@ -326,18 +326,20 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     int ntA = insert_rounds(c, ia, pend, pend2, S, 2, &rs);
     long long capB = 4LL * N + 8;
     DBuf<int3> tB(capB), aB(capB);
-    int Ts = filter_leaves_morton(c, pts, tA.p, aA.p, sA.p, ntA, tB.p, aB.p, 2LL * S + 2);
+    DBuf<FRec> recS(2LL * S + 2);  // stay for the location
+    int Ts = filter_leaves_morton_rec(c, pts, tA.p, aA.p, sA.p, ntA, recS.p, 2LL * S + 2);
     tA.release();
     aA.release();
     sA.release();
     clA.release();
-    validate_mesh(c, "the sample mesh's insertion", Mesh{pts, tB.p, aB.p, nullptr, nullptr}, N + 4, Ts, false);
+    validate_records(c, "the sample mesh's insertion", recS.p, Mesh{pts, tB.p, aB.p, nullptr, nullptr}, N + 4, Ts, false);
     int fr = 0;
-    st.flips += flip_rounds(c, Mesh{pts, tB.p, aB.p, nullptr, nullptr}, Ts, nullptr, 0, &fr);
+    st.flips += flip_rounds_records(c, recS.p, Mesh{pts, tB.p, aB.p, nullptr, nullptr}, Ts, &fr);
     validate_mesh(c, "the sample mesh's flips", Mesh{pts, tB.p, aB.p, nullptr, nullptr}, N + 4, Ts, true);
     st.ms_sample = phase.lap();
     // ---- 2. locate the rest, each walking from its own cell's sample
-    int np = locate_walk(c, pts, N, tB.p, aB.p, Ts, sid.p, soff.p, loc.p, pend.p);
+    int np = locate_walk(c, pts, N, tB.p, recS.p, Ts, sid.p, soff.p, loc.p, pend.p);
+    recS.release();
     sid.release();
     soff.release();
     // ---- 3. insert them
@@ -873,19 +875,21 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     long long capB = 2LL * K + 2LL * S + 4LL * (NP - S) + 8;
     if (capB > (1LL << 31) - 1) throw Error(GCDT_ERR_INVALID, "batch too large");
     DBuf<int3> tB(capB), aB(capB);
-    int Ts = filter_leaves_inst(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, ncells, NP, tA.p, aA.p, sA.p, ntA, tB.p,
-                                aB.p, 2LL * S + 2LL * K);
+    DBuf<FRec> recS(2LL * S + 2LL * K);  // stay for the location
+    int Ts = filter_leaves_inst_rec(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, ncells, NP, tA.p, aA.p, sA.p, ntA, recS.p,
+                                    2LL * S + 2LL * K);
     tA.release();
     aA.release();
     sA.release();
     clA.release();
-    validate_mesh(c, "the sample meshes' insertion", Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, nv, Ts, false);
+    validate_records(c, "the sample meshes' insertion", recS.p, Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, nv, Ts, false);
     int fr = 0;
-    bs.flips += flip_rounds(c, Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, Ts, nullptr, 0, &fr);
+    bs.flips += flip_rounds_records(c, recS.p, Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, Ts, &fr);
     validate_mesh(c, "the sample meshes' flips", Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, nv, Ts, true);
     // ---- 2. locate the other points, each walking from its own cell's sample,
     //         then insert them
-    int np = locate_walk_batch(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, cell_end.p, NP, K, tB.p, aB.p, Ts, loc.p, pend.p);
+    int np = locate_walk_batch(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, cell_end.p, NP, K, tB.p, recS.p, Ts, loc.p, pend.p);
+    recS.release();
     cell_end.release();
     DBuf<int> sB(capB);
     DBuf<unsigned long long> clB(capB);

@@ -1543,11 +1543,12 @@ struct CellSampleInst {
 // point strictly outside, to the triangle whose closed region holds it (on a
 // Delaunay mesh such a walk ends).  Which of an edge's two triangles a point
 // on it is recorded in does not matter (closeness_rank_edge).  Bound by the
-// chain of loads: two per triangle, mostly in L2 (the sample mesh has at most
-// 131k triangles).
+// chain of loads, so it reads the sample mesh's flip records: one 64-byte line
+// a triangle, where triangle and neighbours and then the three vertices were
+// two loads in a row.
 template <class S>
-__global__ __launch_bounds__(kBlock) void k_locate_walk(S smp, const int2* pts, int n, const int3* tri, const int3* adj,
-                                                        int T, const int* vt, int* loc, int* pend, int* npend, int* err)
+__global__ __launch_bounds__(kBlock) void k_locate_walk(S smp, const int2* pts, int n, const FRec* rec, int T,
+                                                        const int* vt, int* loc, int* pend, int* npend, int* err)
 {
     __shared__ int s_buf[STAGE_CAP];
     __shared__ int s_base;
@@ -1563,15 +1564,15 @@ __global__ __launch_bounds__(kBlock) void k_locate_walk(S smp, const int2* pts, 
             int r = -1, t = vt[v];
             if (v != p) {
                 for (int g = 0; g < T && t >= 0; g++) {
-                    const int3 tv = tri[t], ta = adj[t];
-                    const int2 A = pts[tv.x], B = pts[tv.y], C = pts[tv.z];
+                    const FRec x = rec_load(&rec[t]);
+                    const int2 A = x.p[0], B = x.p[1], C = x.p[2];
                     const int o0 = orient2d(B, C, P), o1 = orient2d(C, A, P), o2 = orient2d(A, B, P);
                     if (o0 >= 0 && o1 >= 0 && o2 >= 0) {
                         const int z = (o0 == 0) + (o1 == 0) + (o2 == 0);
                         r = z == 0 ? 3 : (z > 1 ? -2 : (o0 == 0 ? 0 : (o1 == 0 ? 1 : 2)));
                         break;
                     }
-                    t = o0 < 0 ? ta.x : (o1 < 0 ? ta.y : ta.z);
+                    t = o0 < 0 ? x.a.x : (o1 < 0 ? x.a.y : x.a.z);
                 }
                 want = r >= 0;
                 if (!want) atomicOr(err, r == -2 ? MERR_DUPLICATE : MERR_LOCATE);
@@ -1585,7 +1586,7 @@ __global__ __launch_bounds__(kBlock) void k_locate_walk(S smp, const int2* pts, 
 }
 
 template <class S>
-static int locate_walk_s(Ctx& c, const S& smp, const int2* pts, int n, long long nv, const int3* tri, const int3* adj,
+static int locate_walk_s(Ctx& c, const S& smp, const int2* pts, int n, long long nv, const int3* tri, const FRec* rec,
                          int T, int* loc, int* pend)
 {
     if (n <= 0) return 0;
@@ -1594,7 +1595,7 @@ static int locate_walk_s(Ctx& c, const S& smp, const int2* pts, int n, long long
     GCDT_LAUNCH_CHECK();
     {
         ProfScope ps("locate_walk", c.st, n);
-        k_locate_walk<S><<<grid_for(n), kBlock, 0, c.st>>>(smp, pts, n, tri, adj, T, vt.p, loc, pend, c.dcnt.p + C_NPEND,
+        k_locate_walk<S><<<grid_for(n), kBlock, 0, c.st>>>(smp, pts, n, rec, T, vt.p, loc, pend, c.dcnt.p + C_NPEND,
                                                            c.dcnt.p + C_ERR);
         GCDT_LAUNCH_CHECK();
     }
@@ -1603,16 +1604,16 @@ static int locate_walk_s(Ctx& c, const S& smp, const int2* pts, int n, long long
     return c.hcnt[C_NPEND];
 }
 
-int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const int3* adj, int T, const int* ids,
+int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const FRec* rec, int T, const int* ids,
                 const int* offs, int* loc, int* pend)
 {
-    return locate_walk_s(c, CellSampleOne{ids, offs}, pts, n, (long long)n + 4, tri, adj, T, loc, pend);
+    return locate_walk_s(c, CellSampleOne{ids, offs}, pts, n, (long long)n + 4, tri, rec, T, loc, pend);
 }
 
 int locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
-                      long long NP, int K, const int3* tri, const int3* adj, int T, int* loc, int* pend)
+                      long long NP, int K, const int3* tri, const FRec* rec, int T, int* loc, int* pend)
 {
-    return locate_walk_s(c, CellSampleInst{vinst, cbase, lvl, cell_end}, pts, (int)NP, NP + 4LL * K, tri, adj, T, loc,
+    return locate_walk_s(c, CellSampleInst{vinst, cbase, lvl, cell_end}, pts, (int)NP, NP + 4LL * K, tri, rec, T, loc,
                          pend);
 }
 
@@ -3155,6 +3156,14 @@ void validate_mesh(Ctx& c, const char* phase, const Mesh& m, long long nv, int T
                                        std::to_string(first));
 }
 
+void validate_records(Ctx& c, const char* phase, const FRec* rec, const Mesh& m, long long nv, int T, bool delaunay)
+{
+    if (!Tunables::get().validate || T <= 0) return;
+    k_unpack_faces<<<grid_for(T), kBlock, 0, c.st>>>(rec, T, m.tri, m.adj, m.cflag);
+    GCDT_LAUNCH_CHECK();
+    validate_mesh(c, phase, m, nv, T, delaunay);
+}
+
 // ================================================================== leaves
 
 __global__ __launch_bounds__(kBlock) void k_leaf_flags(const int* sons, int T, int* flags)
@@ -3285,33 +3294,12 @@ __global__ __launch_bounds__(kBlock) void k_leaf_dest(const int* sons, const int
     }
 }
 
-// Where the moved leaves go: plain tri/adj arrays, or straight into the
-// packed flip records (coordinates gathered here, so the flips need no
-// separate pack pass over a freshly written mesh).
-struct LeafToArrays {
-    int3* tri2;
-    int3* adj2;
-    __device__ void put(long long o, int3 v, int3 a) const
-    {
-        tri2[o] = v;
-        adj2[o] = a;
-    }
-};
-
-struct LeafToRecords {
-    FRec* rec;
-    const int2* pts;
-    __device__ void put(long long o, int3 v, int3 a) const
-    {
-        rec_store(&rec[o], v, a, pts[v.x], pts[v.y], pts[v.z], FREC_NOCAND | FREC_NOPARTNER, 0, 0ull);
-    }
-};
-
-// Walks the destinations in order and gathers each one's leaf, so the
-// (64-byte record) writes are contiguous and the reads do the scattering.
-template <class OUT>
+// Leaves into packed flip records (the coordinates gathered here, so the flips
+// need no pack pass over a freshly written mesh).  Walks the destinations in
+// order and gathers each one's leaf, so the 64-byte writes are contiguous and
+// the reads do the scattering.
 __global__ __launch_bounds__(kBlock) void k_leaf_move(const int3* tri, const int3* adj, const int* dest,
-                                                      const int* src, int n, OUT out)
+                                                      const int* src, int n, const int2* pts, FRec* rec)
 {
     for (long long o = (long long)blockIdx.x * blockDim.x + threadIdx.x; o < n; o += (long long)gridDim.x * blockDim.x) {
         int i = src[o];
@@ -3319,14 +3307,15 @@ __global__ __launch_bounds__(kBlock) void k_leaf_move(const int3* tri, const int
         a.x = a.x >= 0 ? dest[a.x] : -1;
         a.y = a.y >= 0 ? dest[a.y] : -1;
         a.z = a.z >= 0 ? dest[a.z] : -1;
-        out.put(o, tri[i], a);
+        const int3 v = tri[i];
+        rec_store(&rec[o], v, a, pts[v.x], pts[v.y], pts[v.z], FREC_NOCAND | FREC_NOPARTNER, 0, 0ull);
     }
 }
 
 // CK: the order inside a cell
-template <class CK, class KEY, class OUT>
+template <class CK, class KEY>
 static int filter_leaves_sorted(Ctx& c, CK ck, const KEY& kf, long long ncells, const int2* pts, const int3* tri,
-                                const int3* adj, const int* sons, int T, const OUT& out, long long nleaf)
+                                const int3* adj, const int* sons, int T, FRec* rec, long long nleaf)
 {
     DBuf<int> cnt((size_t)ncells + 1), cellof(T > 0 ? T : 1), dest(T > 0 ? T : 1);
     FillJobs f;
@@ -3357,35 +3346,22 @@ static int filter_leaves_sorted(Ctx& c, CK ck, const KEY& kf, long long ncells, 
     }
     if (n > 0) {
         ProfScope ps("leaf_move", c.st, n);
-        k_leaf_move<OUT><<<grid_for(n), kBlock, 0, c.st>>>(tri, adj, dest.p, src.p, n, out);
+        k_leaf_move<<<grid_for(n), kBlock, 0, c.st>>>(tri, adj, dest.p, src.p, n, pts, rec);
         GCDT_LAUNCH_CHECK();
     }
     return n;
 }
 
-template <class OUT>
-static int filter_leaves_one(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
-                             const OUT& out, long long nleaf)
+int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
+                             FRec* rec, long long nleaf)
 {
     const int b = leaf_bits(nleaf);
     const LeafKeyOne key{2 * (LEAF_CELL_BITS - b)};
     if (b == LEAF_CELL_BITS)
-        return filter_leaves_sorted(c, CellKeyTri{}, key, LEAF_CELLS, pts, tri, adj, sons, T, out, nleaf);
+        return filter_leaves_sorted(c, CellKeyTri{}, key, LEAF_CELLS, pts, tri, adj, sons, T, rec, nleaf);
     CellKeyTriFine ck{};
     ck.pts = pts;
-    return filter_leaves_sorted(c, ck, key, 1LL << (2 * b), pts, tri, adj, sons, T, out, nleaf);
-}
-
-int filter_leaves_morton(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2,
-                         int3* adj2, long long nleaf)
-{
-    return filter_leaves_one(c, pts, tri, adj, sons, T, LeafToArrays{tri2, adj2}, nleaf);
-}
-
-int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
-                             FRec* rec, long long nleaf)
-{
-    return filter_leaves_one(c, pts, tri, adj, sons, T, LeafToRecords{rec, pts}, nleaf);
+    return filter_leaves_sorted(c, ck, key, 1LL << (2 * b), pts, tri, adj, sons, T, rec, nleaf);
 }
 
 // Batch meshes: instance-major, then the Morton order of the centroid's cell
@@ -3403,20 +3379,12 @@ struct LeafKeyInst {
     }
 };
 
-int filter_leaves_inst(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, long long ncells,
-                       long long NP, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2, int3* adj2,
-                       long long nleaf)
-{
-    return filter_leaves_sorted(c, CellKeyTri{}, LeafKeyInst{vinst, cbase, lvl, NP}, ncells, pts, tri, adj, sons, T,
-                                LeafToArrays{tri2, adj2}, nleaf);
-}
-
 int filter_leaves_inst_rec(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl,
                            long long ncells, long long NP, const int3* tri, const int3* adj, const int* sons, int T,
                            FRec* rec, long long nleaf)
 {
     return filter_leaves_sorted(c, CellKeyTri{}, LeafKeyInst{vinst, cbase, lvl, NP}, ncells, pts, tri, adj, sons, T,
-                                LeafToRecords{rec, pts}, nleaf);
+                                rec, nleaf);
 }
 
 int filter_leaves(Ctx& c, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2, int3* adj2,

@@ -317,6 +317,8 @@ void validate_mesh(Ctx& c, const char* phase, const Mesh& m, long long nv, int T
 // lowest failing triangle (-1 if none).
 void check_mesh(Ctx& c, const int2* pts, long long nv, const int3* tri, const int3* adj, const int* cflag, int T,
                 bool delaunay, int* failed, int* first);
+// The same for T packed records, unpacked into m.tri / m.adj for it.
+void validate_records(Ctx& c, const char* phase, const FRec* rec, const Mesh& m, long long nv, int T, bool delaunay);
 // whole-mesh flip rounds on records already packed (filter_leaves_*_rec);
 // the result is unpacked into m.tri / m.adj (and m.cflag when set)
 long long flip_rounds_records(Ctx& c, FRec* rec, const Mesh& m, int T, int* rounds);
@@ -356,17 +358,10 @@ int flags_to_list(Ctx& c, const int* flags, int n, int* list);
 // leaves of a DAG -> compact arrays (adjacency remapped); returns count
 int filter_leaves(Ctx& c, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2, int3* adj2,
                   long long cap);
-// same, with the leaves placed in Morton order of their centroid cell
-int filter_leaves_morton(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2,
-                         int3* adj2, long long nleaf);
-// batch meshes: leaves sorted by (instance, centroid cell in the instance's
-// grid of 4^L cells: cbase/lvl/ncells as for the batched point order)
-int filter_leaves_inst(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, long long ncells,
-                       long long NP, const int3* tri, const int3* adj, const int* sons, int T, int3* tri2, int3* adj2,
-                       long long nleaf);
-// the same two orders, written straight into packed flip records
-// (filter_leaves_morton, _inst and these fail with GCDT_ERR_INTERNAL unless the
-// mesh has nleaf leaves)
+// same into packed flip records, the leaves placed in Morton order of their
+// centroid cell (batch meshes: by instance, then centroid cell in the
+// instance's grid of 4^L cells: cbase/lvl/ncells as for the batched point
+// order); GCDT_ERR_INTERNAL unless the mesh has nleaf leaves
 int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
                              FRec* rec, long long nleaf);
 int filter_leaves_inst_rec(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl,
@@ -380,13 +375,14 @@ int locate_bitmap(Ctx& c, const int2* pts, int n, const int3* tri, int T, const 
                   int* loc, int* isv, int* pend);
 // Location without a bitmap: every point of [0,n) that is no sample walks through
 // the sample Delaunay mesh from its own cell's sample; fills loc and pend,
-// returns npend.  ids / offs as sample_points_morton gives them.  (The bitmap's
+// returns npend.  tri and rec: the sample mesh and its flip records; ids / offs
+// as sample_points_morton gives them.  (The bitmap's
 // build alone costs 190 us with its launches and waits; the walk also wins at
 // 10M points, 27.68 -> 27.48 ms of kernels.)
-int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const int3* adj, int T, const int* ids,
+int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const FRec* rec, int T, const int* ids,
                 const int* offs, int* loc, int* pend);
 int locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
-                      long long NP, int K, const int3* tri, const int3* adj, int T, int* loc, int* pend);
+                      long long NP, int K, const int3* tri, const FRec* rec, int T, int* loc, int* pend);
 // locate all points of [0,n) in the two corner triangles 0/1
 int locate_two(Ctx& c, const int2* pts, int n, int* loc, int* pend);
 // adjacency of a plain triangle list (edges matched through vertex buckets)
