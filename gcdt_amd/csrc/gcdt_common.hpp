@@ -188,12 +188,19 @@ struct Staged {
         if (staged == 0) return;
         if (threadIdx.x == 0) *base = atomicAdd(counter, staged);
         __syncthreads();
+        write();
+        __syncthreads();  // buf is free again
+        staged = 0;
+    }
+
+    // the staged entries to *base on
+    __device__ void write()
+    {
+        if (staged == 0) return;
         long long b = *base;
         if (b + staged > cap && threadIdx.x == 0 && err) atomicOr(err, capbit);
         for (int i = threadIdx.x; i < staged; i += blockDim.x)
             if (b + i < cap) out[b + i] = buf[i];
-        __syncthreads();  // buf is free again
-        staged = 0;
     }
 
     // This thread's first position in buf for its k entries (k * blockDim.x
@@ -208,6 +215,21 @@ struct Staged {
         return p;
     }
 };
+
+// flush of two lists, their counters' trips at the same time
+template <int CAP>
+__device__ inline void flush_both(Staged<CAP>& a, Staged<CAP>& b)
+{
+    __syncthreads();  // the staged entries are written
+    if (threadIdx.x == 0 && a.staged) *a.base = atomicAdd(a.counter, a.staged);
+    if (threadIdx.x == 64 && b.staged) *b.base = atomicAdd(b.counter, b.staged);
+    __syncthreads();
+    a.write();
+    b.write();
+    __syncthreads();  // the buffers are free again
+    a.staged = 0;
+    b.staged = 0;
+}
 
 // LDS staging capacity of a list append (ints per list per block): at least
 // the most entries one tile can append (256 threads x 4 items x 2 entries).

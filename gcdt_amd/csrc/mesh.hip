@@ -1687,15 +1687,16 @@ __device__ inline void claim_items(const Ins& s, const int (&p)[IT], const int (
 // The first tile's entries of a list, read beside its length (which a launch
 // otherwise waits for alone): entries past the length are read and not used.
 template <int IT>
-__device__ inline void first_tile(const int* list, long long cap, int (&v)[IT])
+__device__ inline void first_tile(const int* list, long long cap, long long bid, int (&v)[IT])
 {
 #pragma unroll
     for (int j = 0; j < IT; j++) {
-        const long long i = (long long)blockIdx.x * kBlock * IT + j * kBlock + threadIdx.x;
+        const long long i = bid * kBlock * IT + j * kBlock + threadIdx.x;
         v[j] = list && i < cap ? list[i] : 0;
     }
 }
-#define TILE_ITEM(list, first, base, i, j, IT) ((base) == (long long)blockIdx.x * kBlock * (IT) ? (first)[j] : (list)[i])
+#define TILE_ITEM(list, first, base, bid, i, j, IT) \
+    ((base) == (long long)(bid)*kBlock * (IT) ? (first)[j] : (list)[i])
 
 // First claims of a run of rounds (later rounds claim inside k_ins_reloc).
 __global__ __launch_bounds__(kBlock) void k_ins_claim_w(Ins s, const int* list, const int* cnt, unsigned epoch, int* wl,
@@ -1742,7 +1743,7 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
 {
     round_snap_store(snap);
     int pre[INS_ITEMS];
-    first_tile(list, lcap, pre);
+    first_tile(list, lcap, blockIdx.x, pre);
     int n = min(*cnt, lcap);  // an overfull list has flagged MERR_CAPACITY
     const int first = set[R_BASE];
     TILE_LOOP(base, n, kBlock * INS_ITEMS)
@@ -1755,7 +1756,7 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
             pp[j] = -1;
             need[j] = 0;
             if (i < n) {
-                const int t = TILE_ITEM(list, pre, base, i, j, INS_ITEMS);
+                const int t = TILE_ITEM(list, pre, base, blockIdx.x, i, j, INS_ITEMS);
                 const unsigned long long w = s.claim[t];
                 const int p = (int)(unsigned)w;
                 const int l = s.loc[p];
@@ -1780,30 +1781,43 @@ __global__ __launch_bounds__(kBlock) void k_ins_split(Ins s, const int* list, co
     }
 }
 
+// rounds of at most this many points settle and relocate in workgroups of their
+// own: both halves are then on the chip at once
+#ifndef GCDT_INS_SPLIT_MAX
+#define GCDT_INS_SPLIT_MAX 131072
+#endif
+constexpr int INS_SPLIT_MAX = GCDT_INS_SPLIT_MAX;
+
 // Outer adjacency of the round's new triangles (their slots follow from the
 // round's counters), then the relocation of the pending points, fused with the
 // next round's claims (epoch next_ep) and its claimed-triangle list.  Only the
 // claims of on-edge points read adjacency, and they resolve entries that this
 // launch has not settled yet (ins_edge_neighbour).  The slots of the next round
 // begin where this round's end.
+//
+// split: even workgroups relocate, odd ones settle.  Both are chains of three to
+// five trips to memory, which a small round is made of (12 rounds of 20,000
+// points 124 -> 105 us); a large one is better off settling first, while the
+// lines that the splits wrote are near (10M points 2.70 ms, split 3.14).
 template <int INS_ITEMS>
-__global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, const int* cnt, int lcap, int* list2,
+__global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, const int* cnt, int lcap, int split, int* list2,
                                                       unsigned next_ep, int* wl, int wcap, int* set, int* next_set)
 {
     __shared__ int s_buf[STAGE_CAP], s_buf2[STAGE_CAP];
     __shared__ int s_base, s_base2;
     Staged<STAGE_CAP> sl(s_buf, &s_base, list2, &set[R_NEXT]),
         sw(s_buf2, &s_base2, wl, &set[R_NW], wcap, s.err, MERR_CAPACITY);
+    const long long bid = split ? blockIdx.x >> 1 : blockIdx.x, nblk = split ? gridDim.x >> 1 : gridDim.x;
     int pre[INS_ITEMS];
-    first_tile(list, lcap, pre);
-    const int tb = set[R_BASE], te = tb + set[R_NEW];
-    if (blockIdx.x == 0 && threadIdx.x == 0) next_set[R_BASE] = te;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x + tb; i < min(te, s.cap);
-         i += (long long)gridDim.x * blockDim.x)
-        ins_fix(s, (int)i);
+    first_tile(list, lcap, bid, pre);
+    if (!split || (blockIdx.x & 1)) {
+        const int tb = set[R_BASE], te = tb + set[R_NEW];
+        if (bid == 0 && threadIdx.x == 0) next_set[R_BASE] = te;
+        for (long long i = bid * kBlock + threadIdx.x + tb; i < min(te, s.cap); i += nblk * kBlock) ins_fix(s, (int)i);
+        if (split) return;
+    }
     int n = *cnt;
-    TILE_LOOP(base, n, kBlock * INS_ITEMS)
-    {
+    for (long long base = bid * kBlock * INS_ITEMS; base < n; base += nblk * kBlock * INS_ITEMS) {
         int p[INS_ITEMS], l[INS_ITEMS];
         unsigned close[INS_ITEMS];
         int tot = 0;
@@ -1812,7 +1826,7 @@ __global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, co
             long long i = base + (long long)j * kBlock + threadIdx.x;
             l[j] = -1;
             if (i < n) {
-                p[j] = TILE_ITEM(list, pre, base, i, j, INS_ITEMS);
+                p[j] = TILE_ITEM(list, pre, base, bid, i, j, INS_ITEMS);
                 const int at = s.loc[p[j]];
                 int to = at;
                 if (at >= 0 && ins_relocate_at<CLAIM_LAUNCH, true>(s, p[j], &to, &close[j])) {
@@ -1828,8 +1842,7 @@ __global__ __launch_bounds__(kBlock) void k_ins_reloc(Ins s, const int* list, co
             if (l[j] >= 0) s_buf[b++] = p[j];
         claim_items<INS_ITEMS>(s, p, l, close, next_ep, sw);
     }
-    sl.flush();
-    sw.flush();
+    flush_both(sl, sw);
 }
 
 // ---- persistent single-workgroup tail: all remaining insertion rounds in one
@@ -2095,8 +2108,9 @@ int insert_rounds(Ctx& c, const Ins& s_in, DBuf<int>& pend, DBuf<int>& pend2, in
         with_items(c.ins_items, [&](auto it) {
             constexpr int IT = decltype(it)::value;
             ProfScope ps("ins_reloc", c.st, 0);
-            k_ins_reloc<IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
-                s, P, in + R_NEXT, npend, P2, ep + 1, W2, (int)wcap, set, c.round_set(r + 1));
+            const int split = est <= INS_SPLIT_MAX;
+            k_ins_reloc<IT><<<grid_for((est + IT - 1) / IT) << split, kBlock, 0, c.st>>>(
+                s, P, in + R_NEXT, npend, split, P2, ep + 1, W2, (int)wcap, set, c.round_set(r + 1));
             GCDT_LAUNCH_CHECK();
         });
         std::swap(P, P2);
@@ -2272,7 +2286,7 @@ __global__ __launch_bounds__(kBlock) void k_flip_test(E e, const int* list, cons
     // cannot overflow; a miscount flags MERR_CAPACITY instead of writing past it
     Staged<STAGE_CAP> sp(s_buf, &s_base, prop, nprop, cap, eflag, MERR_CAPACITY);
     int pre[FT_ITEMS];
-    first_tile(list, lcap, pre);
+    first_tile(list, lcap, blockIdx.x, pre);
     int n = min(*cnt, lcap);
     TILE_LOOP(base, n, kBlock * FT_ITEMS)
     {
@@ -2283,7 +2297,7 @@ __global__ __launch_bounds__(kBlock) void k_flip_test(E e, const int* list, cons
             q[j] = -1;
             long long i = base + (long long)j * kBlock + threadIdx.x;
             if (i < n) {
-                q[j] = e.propose(list ? TILE_ITEM(list, pre, base, i, j, FT_ITEMS) : (int)i, epoch, list == nullptr, single != 0);
+                q[j] = e.propose(list ? TILE_ITEM(list, pre, base, blockIdx.x, i, j, FT_ITEMS) : (int)i, epoch, list == nullptr, single != 0);
             }
             nq += q[j] >= 0;
         }
@@ -2310,7 +2324,7 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
     if (E::kFused && threadIdx.x == 0) s_nf = 0;
     int flips = 0;
     int pre[FA_ITEMS];
-    first_tile(list, cap, pre);
+    first_tile(list, cap, blockIdx.x, pre);
     int n = min(*cnt, cap);
     TILE_LOOP(base, n, kBlock * FA_ITEMS)
     {
@@ -2323,7 +2337,7 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
             long long i = base + (long long)j * kBlock + threadIdx.x;
             if (i < n) {
                 int t, nn = -1;
-                int res = e.apply_round(TILE_ITEM(list, pre, base, i, j, FA_ITEMS), epoch, &t, &nn);
+                int res = e.apply_round(TILE_ITEM(list, pre, base, blockIdx.x, i, j, FA_ITEMS), epoch, &t, &nn);
                 if (res == 1) e.set_mark(t, (int)epoch + 1);
                 if (res == 1 || res == 2) qa[j] = t;
                 if (res == 2) qb[j] = nn;

@@ -830,14 +830,15 @@ __host__ __device__ inline int flip_apply_peer(const FlipP& f, int e, unsigned e
     const int t = (int)((unsigned)e / 3u), k = e - 3 * t;
     const unsigned long long key = ((unsigned long long)epoch << 32) | (unsigned)e;
     const FRec r = rec_load(&f.r[t]);
-    if (r.claim > key) {
-        // r.claim is t2's; it wins (and flips t) unless t2 is claimed above it
-        const int t2 = (int)((r.claim & 0xffffffffu) / 3);
-        return ld_claim<false>(&f.r[t2].claim) <= r.claim ? 3 : 1;
-    }
-    const int n = get3(r.a, k);
+    // the record that decides: n's, or, where t is claimed above its key, the
+    // claimant's (a wave waits for both kinds at once)
+    const bool lost = r.claim > key;
+    const int n = lost ? (int)((r.claim & 0xffffffffu) / 3) : get3(r.a, k);
+    const bool above = !lost && n > t && cl.prop[n] == cl.tag;  // n's own proposal
     const FRec rn = rec_load(&f.r[n]);
-    if (rn.claim != key || (n > t && cl.prop[n] == cl.tag)) return 1;
+    // t's claimant wins (and flips t) unless it is claimed above itself
+    if (lost) return rn.claim <= r.claim ? 3 : 1;
+    if (rn.claim != key || above) return 1;
     flip_records(&f.r[t], &f.r[n], t, r, k, n, rn, epoch, key);
     *nout = n;
     return 2;
