@@ -2309,9 +2309,42 @@ __global__ __launch_bounds__(kBlock) void k_flip_test(E e, const int* list, cons
     sp.flush();
 }
 
+// The same for short lists of packed records, whose time is the chain of trips
+// to memory: four lanes share a triangle, one an edge, and the proposal (or -1)
+// of entry i goes to prop[i], so that no list is appended to.
+__global__ __launch_bounds__(kBlock) void k_flip_test_short(FlipP f, PeerClaims cl, const int* list, const int* cnt, int lcap,
+                                                            unsigned epoch, int single, int* prop, RoundSnap snap)
+{
+    round_snap_store(snap);
+    const int k = (int)threadIdx.x & 3, lead = (int)threadIdx.x & 60;
+    const long long i0 = (long long)blockIdx.x * (kBlock / 4) + (threadIdx.x >> 2);
+    const int pre = list && i0 < lcap ? list[i0] : 0;
+    const int n = min(*cnt, lcap);
+    TILE_LOOP(base, n, kBlock / 4)
+    {
+        const long long i = base + (threadIdx.x >> 2);
+        int t = -1, nn = -1;
+        bool hit = false;
+        if (i < n) {
+            t = list ? (i == i0 ? pre : list[i]) : (int)i;
+            const FRec r = rec_load(&f.r[t]);
+            FRec rn;
+            hit = k < 3 && flip_fixtest_edge(f, t, r, k, epoch, list == nullptr, single != 0, &nn, &rn);
+        }
+        const unsigned m = (unsigned)(__ballot(hit) >> lead) & 7u;
+        const int cand = m ? __ffsll((long long)m) - 1 : 3;
+        if (i < n && k == cand) {
+            if (cand < 3) cl.propose(f, t, nn, ((unsigned long long)epoch << 32) | (unsigned)(3 * t + cand));
+            prop[i] = cand < 3 ? 3 * t + cand : -1;
+        }
+    }
+}
+
+// holes: entries of the list are proposals or -1; their number goes to *nprop.
 template <class E, int FA_ITEMS>
-__global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, const int* cnt, unsigned epoch, int* list2,
-                                                       int* cnt2, int* flipped, int* nflip, int cap, int* eflag)
+__global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, const int* cnt, int holes, int* nprop,
+                                                       unsigned epoch, int* list2, int* cnt2, int* flipped, int* nflip,
+                                                       int cap, int* eflag)
 {
     __shared__ int s_buf[STAGE_CAP], s_buf2[E::kFused ? 1 : STAGE_CAP];
     __shared__ int s_base, s_base2;
@@ -2320,9 +2353,9 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
     // hold at most cap entries; a miscount flags MERR_CAPACITY
     Staged<STAGE_CAP> sq(s_buf, &s_base, list2, cnt2, cap, eflag, MERR_CAPACITY),
         sf(s_buf2, &s_base2, flipped, nflip, cap, eflag, MERR_CAPACITY);
-    __shared__ int s_nf;  // fused engines need only the number of flipped triangles
-    if (E::kFused && threadIdx.x == 0) s_nf = 0;
-    int flips = 0;
+    __shared__ int s_nf, s_np;  // fused engines need only the number of flipped triangles
+    if (E::kFused && threadIdx.x == 0) s_nf = s_np = 0;
+    int flips = 0, props = 0;
     int pre[FA_ITEMS];
     first_tile(list, cap, blockIdx.x, pre);
     int n = min(*cnt, cap);
@@ -2337,10 +2370,14 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
             long long i = base + (long long)j * kBlock + threadIdx.x;
             if (i < n) {
                 int t, nn = -1;
-                int res = e.apply_round(TILE_ITEM(list, pre, base, blockIdx.x, i, j, FA_ITEMS), epoch, &t, &nn);
-                if (res == 1) e.set_mark(t, (int)epoch + 1);
-                if (res == 1 || res == 2) qa[j] = t;
-                if (res == 2) qb[j] = nn;
+                const int q = TILE_ITEM(list, pre, base, blockIdx.x, i, j, FA_ITEMS);
+                if (q >= 0) {
+                    int res = e.apply_round(q, epoch, &t, &nn);
+                    if (res == 1) e.set_mark(t, (int)epoch + 1);
+                    if (res == 1 || res == 2) qa[j] = t;
+                    if (res == 2) qb[j] = nn;
+                    props++;
+                }
             }
             nq += (qa[j] >= 0) + (qb[j] >= 0);
             nf += (qb[j] >= 0) ? 2 : 0;
@@ -2363,8 +2400,10 @@ __global__ __launch_bounds__(kBlock) void k_flip_apply(E e, const int* list, con
     sq.flush();
     if (E::kFused) {  // after the barrier in flush
         wave_alloc(flips, &s_nf);
+        if (holes) wave_alloc(props, &s_np);
         __syncthreads();
         if (threadIdx.x == 0 && s_nf) atomicAdd(nflip, s_nf);
+        if (threadIdx.x == 0 && s_np) atomicAdd(nprop, s_np);
     } else {
         sf.flush();
     }
@@ -2405,7 +2444,7 @@ __device__ inline int short_round(const FlipP& f, int* list, FRec* rec, bool kep
         if (i < n && k < 3) {
             t = list[i];
             r = kept ? rec_load(&rec[i]) : rec_load(&f.r[t]);
-            hit = flip_fixtest_edge(f, t, r, k, ep, &nn, &rn);
+            hit = flip_fixtest_edge(f, t, r, k, ep, false, false, &nn, &rn);
         }
         const unsigned m = (unsigned)(__ballot(hit) >> lead) & 7u;
         cand = m ? __ffsll((long long)m) - 1 : 3;
@@ -2639,6 +2678,12 @@ namespace {
 #endif
 constexpr int FLIP_WG_LIST = GCDT_FLIP_WG_LIST;
 
+// rounds of at most this many triangles test by edges (k_flip_test_short)
+#ifndef GCDT_FLIP_SHORT_MAX
+#define GCDT_FLIP_SHORT_MAX 65536
+#endif
+constexpr int FLIP_SHORT_MAX = GCDT_FLIP_SHORT_MAX;
+
 // Rounds of test / apply / fix over a triangle list until no edge needs a
 // flip.  Round 1 reads `init` (or the implicit list of all T triangles); later
 // rounds alternate between two device lists whose lengths stay on the device
@@ -2702,7 +2747,16 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
             }
             with_items(c.flip_items, [&](auto it) {
                 constexpr int IT = decltype(it)::value;
-                {
+                bool holes = false;
+                if constexpr (E::kFused) holes = est <= FLIP_SHORT_MAX;
+                if (holes) {
+                    if constexpr (E::kFused) {
+                        ProfScope ps("flip_test", c.st, 0);
+                        k_flip_test_short<<<grid_for(4LL * est), kBlock, 0, c.st>>>(
+                            e.f, e.pc, act, in + R_NEXT, (init && act == init) ? ninit : T, ep, single, lp.p, snap);
+                        GCDT_LAUNCH_CHECK();
+                    }
+                } else {
                     ProfScope ps("flip_test", c.st, 0);
                     k_flip_test<E, IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
                         e, act, in + R_NEXT, (init && act == init) ? ninit : T, ep, single, lp.p, set + R_PROP, T,
@@ -2712,7 +2766,8 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
                 {
                     ProfScope ps("flip_apply", c.st, 0);
                     k_flip_apply<E, IT><<<grid_for((est + IT - 1) / IT), kBlock, 0, c.st>>>(
-                        e, lp.p, set + R_PROP, ep, nxt, set + R_NEXT, lf.p, set + R_FLIP, T, c.dcnt.p + C_ERR);
+                        e, lp.p, holes ? in + R_NEXT : set + R_PROP, holes, set + R_PROP, ep, nxt, set + R_NEXT, lf.p,
+                        set + R_FLIP, T, c.dcnt.p + C_ERR);
                     GCDT_LAUNCH_CHECK();
                 }
             });

@@ -754,12 +754,11 @@ __host__ __device__ inline bool flip_fixtest_p(const FlipP& f, int t, unsigned e
     return cand != 3;
 }
 
-// Edge k of triangle t (record r) in flip_fixtest_p, for rounds in which every
-// listed triangle tests: settles the slot if t flipped last round, and tests
-// the edge.  True if the edge needs a flip; *nout and *rn are then the
-// triangle across it and its record.
-__host__ __device__ inline bool flip_fixtest_edge(const FlipP& f, int t, const FRec& r, int k, unsigned epoch, int* nout,
-                                                  FRec* rn)
+// Edge k of triangle t (record r) in flip_fixtest_p: settles the slot if t
+// flipped last round, and tests the edge.  True if the edge needs a flip;
+// *nout and *rn are then the triangle across it and its record.
+__host__ __device__ inline bool flip_fixtest_edge(const FlipP& f, int t, const FRec& r, int k, unsigned epoch, bool all_active,
+                                                  bool single, int* nout, FRec* rn)
 {
     const int prev = (int)epoch - 1;
     const bool cons = (r.meta >> k) & 1;
@@ -787,6 +786,7 @@ __host__ __device__ inline bool flip_fixtest_edge(const FlipP& f, int t, const F
         if (get3(rn->a, j) != t) (&f.r[av].a.x)[j] = t;
     }
     if (cons || n == partner) return false;
+    if (single && n < t && (all_active || rec_marked(rn->meta, epoch))) return false;
     *nout = n;
     return incircle(r.p[0], r.p[1], r.p[2], rec_pt(*rn, slot_other(rn->v, u, v))) > 0;
 }
