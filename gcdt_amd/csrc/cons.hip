@@ -809,7 +809,7 @@ __global__ __launch_bounds__(kBlock) void k_cav_fix(Cons c, const Win* wins, con
             cav_fix_one(c, wins, scr, t, epoch, true);
             if (touched && !touched[t]) {
                 touched[t] = 1;
-                first = true;
+                first = tlist != nullptr;
             }
         }
         const int at = sl.reserve(first ? 1 : 0);
