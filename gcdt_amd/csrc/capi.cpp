@@ -284,6 +284,10 @@ int gcdt_prof_names(char* buf, int cap) { return prof_names(buf, cap); }
 namespace gcdt {
 
 // Full pipeline on device arrays; pts holds N+4 entries (corners written here).
+// bytes counted for the phases before the constraints beside those per point,
+// sample point and segment
+constexpr size_t NOALLOC_BASE = 21243136;
+
 void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, int3* tris_out, int3* adj_out,
                 SolveOut& out, int* cflag_out, const SteinerArgs* steiner)
 {
@@ -393,6 +397,13 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
         ConsDefer defer;
         DBuf<int> tl(T);
         ConsResult cr = insert_constraints(c, m, T, N + 4, N, cons, C, touched.p, tl.p, cell_end.p,
+        // The solve on a fixed array takes or refuses an input by a demand that
+        // follows from the input alone, whatever the phases before still hold.
+        DBuf<int> held;
+        if (g_arena) {
+            const size_t demand = NOALLOC_BASE + 172 * (size_t)N + 168 * (size_t)S + 8 * (size_t)C;
+            if (demand > g_arena->top) held.alloc((demand - g_arena->top) / sizeof(int));
+        }
                                            steiner ? &defer : nullptr);
         st.constraint_rounds = cr.rounds;
         st.segments = cr.pieces;

@@ -1057,13 +1057,57 @@ __global__ __launch_bounds__(kBlock) void k_seg_walk(Cons c, const int2* cons, c
 // *nq: true when the pieces that need a cavity have been queued (C_NQ was
 // cleared by the caller, and C_NREW, C_NQ2 as cursors)
 static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const int2* cons, int C, int nmax,
-                              DBuf<int2>& pieces, DBuf<int>& queue, bool* queued)
+                              DBuf<int2>& pieces, DBuf<int>& queue, bool* queued, DBuf<int>& pad)
 {
+// Cells that the closed segments can touch, column by column (a superset): what
+// the solve on a fixed array bounds its inputs by (demand_words).
+__global__ __launch_bounds__(64) void k_seg_demand(const int2* pts, const int2* cons, int C, int nmax, int* total)
+{
+    for (int i = blockIdx.x; i < C; i += gridDim.x) {
+        const int2 e = cons[i];
+        if (!seg_valid(e, nmax)) continue;
+        int2 A = pts[e.x], B = pts[e.y];
+        if (A.x > B.x) {
+            const int2 t = A;
+            A = B;
+            B = t;
+        }
+        const long long dx = (long long)B.x - A.x, dy = (long long)B.y - A.y;
+        int k = 0;
+        for (int cx = (A.x >> 20) + (int)threadIdx.x; cx <= B.x >> 20; cx += 64) {
+            int lo = min(A.y, B.y) >> 20, hi = max(A.y, B.y) >> 20;
+            if (dx > 0) {
+                const long long xl = max((long long)A.x, (long long)cx << 20),
+                                xr = min((long long)B.x, ((long long)(cx + 1) << 20) - 1);
+                const long long nl = A.y * dx + (xl - A.x) * dy, nr = A.y * dx + (xr - A.x) * dy;
+                // all within the square, so neither numerator is negative
+                lo = (int)((min(nl, nr) / dx) >> 20);
+                hi = (int)(((max(nl, nr) + dx - 1) / dx) >> 20);
+                hi = min(hi, 1023);
+            }
+            k += hi - lo + 1;
+        }
+        wave_alloc(k, total);
+    }
+}
+
+// Words that a split of C segments, nh vertices on them and `pairs` touched
+// cells counts for in the array of a solve without allocations, above what it
+// uses: that solve has always been bounded by them, and an input is taken or
+// refused (GCDT_ERR_SCRATCH) by the input alone.
+static long long demand_words(int C, long long nh, long long pairs) { return 6LL * C + 4 + nh + 2 * pairs; }
+
+// pad: the rest of that demand, held while the constraints are inserted
     const int2* pts = c.m.pts;
     int* cnt = cx.dcnt.p;
     DBuf<int> np((size_t)C + 1), hcnt(C), hpos(C), wlist(C), hits((size_t)2 * C + 1024);
     for (int tries = 0;; tries++) {
         const int hcap = (int)std::min<size_t>(hits.n, 1u << 30);
+    if (g_arena) {
+        cx.set(C_STUCK, 0);
+        k_seg_demand<<<std::min(C, 16384), 64, 0, cx.st>>>(pts, cons, C, nmax, cnt + C_STUCK);
+        GCDT_LAUNCH_CHECK();
+    }
         k_seg_find<<<std::min(C, 16384), 64, 0, cx.st>>>(pts, cell_end, cons, C, nmax, np.p, hcnt.p, hpos.p, hits.p, hcap,
                                                          cnt + C_NREW, wlist.p, cnt + C_NQ2, c.err);
         GCDT_LAUNCH_CHECK();
@@ -1083,6 +1127,11 @@ static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const
     if (nwalk > 0) {
         // segments with many vertices keep the walk: their counts, and the
         // offsets again (from the counts of the others)
+    if (g_arena) {
+        const long long held = (long long)(np.n + hcnt.n + hpos.n + wlist.n + hits.n);
+        const long long more = demand_words(C, cx.hcnt[C_NREW], cx.hcnt[C_STUCK]) - held;
+        if (more > 0) pad.alloc((size_t)more);
+    }
         DBuf<int> cnts((size_t)C + 1);
         k_seg_counts<<<grid_for(C), kBlock, 0, cx.st>>>(cons, C, nmax, hcnt.p, cnts.p);
         GCDT_LAUNCH_CHECK();
@@ -1175,7 +1224,8 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
     DBuf<int2> pieces;
     DBuf<int> qa;
     bool queued = false;
-    int np = cell_end ? split_pieces_cells(cx, c, cell_end, cons, C, nmax, pieces, qa, &queued)
+    DBuf<int> pad;
+    int np = cell_end ? split_pieces_cells(cx, c, cell_end, cons, C, nmax, pieces, qa, &queued, pad)
                       : split_pieces(cx, c, cons, C, nmax, pieces);
     res.pieces = np;
     DBuf<int> dflag;
@@ -1247,6 +1297,11 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
                                              cnt + C_NWIN, scr.p, cnt + C_SCR, (long long)scr.n);
         GCDT_LAUNCH_CHECK();
         // Few long pieces: the larger workgroup for all of them, in one launch (two
+        // the solve on a fixed array takes inputs up to a demand of 14 words per
+        // crossed triangle and 20 per piece here, whatever the round makes of them
+        const long long demand = std::min(13 * npath + 20LL * nq + 1024, 1LL << 30) + npath + 1,
+                        held = (long long)(paths.n + longq.n + longw.n + ppos.n + rew.n);
+        scr.ensure((size_t)std::max(cap, g_arena ? demand - held : 0LL));
         // in turn last as long as their longest cavities together: 1,000 rows over
         // 100,000 points 6.6 -> 5.9 ms).  Many: a wave each for the smaller ones,
         // as the larger workgroup's LDS admits two to a CU.

@@ -153,6 +153,8 @@ Ctx::Ctx(hipStream_t s, const HostSlot* fixed) : st(s)
     flip_items = Tunables::get().flip_items;
     ins_items = Tunables::get().ins_items;
     dcnt.alloc(C_NUM);
+    // on a fixed array below everything that is given back before it
+    if (g_arena) ring.ensure(ROUND_SETS * ROUND_INTS);
     HostSlot h = fixed ? *fixed : take_host_slot();
     fixed_slot = fixed != nullptr;
     hcnt = h.hcnt;

@@ -99,6 +99,7 @@ struct DBuf {
 // device counters (indices into Ctx::dcnt)
 enum : int {
     C_NPEND = 0,   // point location: pending points
+    C_STUCK = 1,   // constraint rounds: pieces left and none inserted (before them: k_seg_demand's total)
     C_NTRI = 2,    // insertion tail: triangles
     C_ERR = 4,
     C_NBIGW = 6,   // constraint rounds: winners above CAV_MID_K
