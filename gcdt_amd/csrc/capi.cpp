@@ -342,7 +342,8 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     validate_mesh(c, "the sample mesh's flips", Mesh{pts, tB.p, aB.p, nullptr, nullptr}, N + 4, Ts, true);
     st.ms_sample = phase.lap();
     // ---- 2. locate the rest, each walking from its own cell's sample
-    int np = locate_walk(c, pts, N, tB.p, recS.p, Ts, sid.p, soff.p, loc.p, pend.p);
+    const int np = N - S;
+    locate_walk(c, pts, N, tB.p, recS.p, Ts, sid.p, soff.p, loc.p, pend.p);
     recS.release();
     sid.release();
     soff.release();
@@ -396,7 +397,6 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
         Mesh m{pts, tris_out, adj_out, nullptr, cflag};
         ConsDefer defer;
         DBuf<int> tl(T);
-        ConsResult cr = insert_constraints(c, m, T, N + 4, N, cons, C, touched.p, tl.p, cell_end.p,
         // The solve on a fixed array takes or refuses an input by a demand that
         // follows from the input alone, whatever the phases before still hold.
         DBuf<int> held;
@@ -404,6 +404,7 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
             const size_t demand = NOALLOC_BASE + 172 * (size_t)N + 168 * (size_t)S + 8 * (size_t)C;
             if (demand > g_arena->top) held.alloc((demand - g_arena->top) / sizeof(int));
         }
+        ConsResult cr = insert_constraints(c, m, T, N + 4, N, cons, C, touched.p, tl.p, cell_end.p,
                                            steiner ? &defer : nullptr);
         st.constraint_rounds = cr.rounds;
         st.segments = cr.pieces;
@@ -899,7 +900,8 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     validate_mesh(c, "the sample meshes' flips", Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, nv, Ts, true);
     // ---- 2. locate the other points, each walking from its own cell's sample,
     //         then insert them
-    int np = locate_walk_batch(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, cell_end.p, NP, K, tB.p, recS.p, Ts, loc.p, pend.p);
+    const int np = (int)(NP - S);
+    locate_walk_batch(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, cell_end.p, NP, K, tB.p, recS.p, Ts, loc.p, pend.p);
     recS.release();
     cell_end.release();
     DBuf<int> sB(capB);

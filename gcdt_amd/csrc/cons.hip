@@ -821,7 +821,10 @@ __global__ __launch_bounds__(kBlock) void k_cav_fix(Cons c, const Win* wins, con
 // move: the pieces left by the round before are the queue
 __global__ void k_cav_begin(int* cnt, int move)
 {
-    if (move) cnt[C_NQ] = cnt[C_NQ2];
+    if (move) {
+        cnt[C_NQ] = cnt[C_NQ2];
+        cnt[C_STUCK] = cnt[C_NQ2] > 0 && cnt[C_NWIN] == 0;
+    }
     cnt[C_NQ2] = 0;
     cnt[C_NWIN] = 0;
     cnt[C_SCR] = 0;
@@ -1056,9 +1059,6 @@ __global__ __launch_bounds__(kBlock) void k_seg_walk(Cons c, const int2* cons, c
 
 // *nq: true when the pieces that need a cavity have been queued (C_NQ was
 // cleared by the caller, and C_NREW, C_NQ2 as cursors)
-static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const int2* cons, int C, int nmax,
-                              DBuf<int2>& pieces, DBuf<int>& queue, bool* queued, DBuf<int>& pad)
-{
 // Cells that the closed segments can touch, column by column (a superset): what
 // the solve on a fixed array bounds its inputs by (demand_words).
 __global__ __launch_bounds__(64) void k_seg_demand(const int2* pts, const int2* cons, int C, int nmax, int* total)
@@ -1098,16 +1098,19 @@ __global__ __launch_bounds__(64) void k_seg_demand(const int2* pts, const int2* 
 static long long demand_words(int C, long long nh, long long pairs) { return 6LL * C + 4 + nh + 2 * pairs; }
 
 // pad: the rest of that demand, held while the constraints are inserted
+static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const int2* cons, int C, int nmax,
+                              DBuf<int2>& pieces, DBuf<int>& queue, bool* queued, DBuf<int>& pad)
+{
     const int2* pts = c.m.pts;
     int* cnt = cx.dcnt.p;
-    DBuf<int> np((size_t)C + 1), hcnt(C), hpos(C), wlist(C), hits((size_t)2 * C + 1024);
-    for (int tries = 0;; tries++) {
-        const int hcap = (int)std::min<size_t>(hits.n, 1u << 30);
     if (g_arena) {
         cx.set(C_STUCK, 0);
         k_seg_demand<<<std::min(C, 16384), 64, 0, cx.st>>>(pts, cons, C, nmax, cnt + C_STUCK);
         GCDT_LAUNCH_CHECK();
     }
+    DBuf<int> np((size_t)C + 1), hcnt(C), hpos(C), wlist(C), hits((size_t)2 * C + 1024);
+    for (int tries = 0;; tries++) {
+        const int hcap = (int)std::min<size_t>(hits.n, 1u << 30);
         k_seg_find<<<std::min(C, 16384), 64, 0, cx.st>>>(pts, cell_end, cons, C, nmax, np.p, hcnt.p, hpos.p, hits.p, hcap,
                                                          cnt + C_NREW, wlist.p, cnt + C_NQ2, c.err);
         GCDT_LAUNCH_CHECK();
@@ -1124,14 +1127,14 @@ static long long demand_words(int C, long long nh, long long pairs) { return 6LL
     }
     int total = cx.hcnt[C_TOTAL];
     const int nwalk = cx.hcnt[C_NQ2];
-    if (nwalk > 0) {
-        // segments with many vertices keep the walk: their counts, and the
-        // offsets again (from the counts of the others)
     if (g_arena) {
         const long long held = (long long)(np.n + hcnt.n + hpos.n + wlist.n + hits.n);
         const long long more = demand_words(C, cx.hcnt[C_NREW], cx.hcnt[C_STUCK]) - held;
         if (more > 0) pad.alloc((size_t)more);
     }
+    if (nwalk > 0) {
+        // segments with many vertices keep the walk: their counts, and the
+        // offsets again (from the counts of the others)
         DBuf<int> cnts((size_t)C + 1);
         k_seg_counts<<<grid_for(C), kBlock, 0, cx.st>>>(cons, C, nmax, hcnt.p, cnts.p);
         GCDT_LAUNCH_CHECK();
@@ -1271,6 +1274,8 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
                                                                   ppos.p);
             GCDT_LAUNCH_CHECK();
             cx.read(0, C_NUM);
+            if (cx.hcnt[C_ERR]) cx.check_err();
+            if (r > 1 && cx.hcnt[C_STUCK]) throw Error(GCDT_ERR_INTERNAL, "constraint round without progress");
             nq = cx.hcnt[C_NQ];
             npath = cx.hcnt[C_PATH];
             if (npath < 0 || npath > (1LL << 30)) throw Error(GCDT_ERR_SCRATCH, "constraints cross too many triangles");
@@ -1280,8 +1285,8 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
             if (tries) throw Error(GCDT_ERR_INTERNAL, "constraint paths changed between two walks");
             paths.ensure((size_t)npath);
         }
-        if (nq == 0) {  // every piece was an edge already
-            if (cx.hcnt[C_ERR]) cx.check_err();
+        if (nq == 0) {  // every piece was an edge already, or the round before inserted the last
+            res.rewritten = cx.hcnt[C_NPIECE];
             r--;
             break;
         }
@@ -1291,17 +1296,16 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
         const long long npl = cx.hcnt[C_TOTAL];
         long long cap = (npath - npl) + 9 * npl + 16LL * nlong + 1024;
         if (cap > (1LL << 30)) cap = 1LL << 30;
-        scr.ensure((size_t)cap);
         rew.ensure((size_t)npl + 1);
-        k_cav_check<<<g, kBlock, 0, cx.st>>>(c, Q, cnt + C_NQ, ncross.p, paths.p, ppos.p, ep, Q2, cnt + C_NQ2, wins.p,
-                                             cnt + C_NWIN, scr.p, cnt + C_SCR, (long long)scr.n);
-        GCDT_LAUNCH_CHECK();
-        // Few long pieces: the larger workgroup for all of them, in one launch (two
         // the solve on a fixed array takes inputs up to a demand of 14 words per
         // crossed triangle and 20 per piece here, whatever the round makes of them
         const long long demand = std::min(13 * npath + 20LL * nq + 1024, 1LL << 30) + npath + 1,
                         held = (long long)(paths.n + longq.n + longw.n + ppos.n + rew.n);
         scr.ensure((size_t)std::max(cap, g_arena ? demand - held : 0LL));
+        k_cav_check<<<g, kBlock, 0, cx.st>>>(c, Q, cnt + C_NQ, ncross.p, paths.p, ppos.p, ep, Q2, cnt + C_NQ2, wins.p,
+                                             cnt + C_NWIN, scr.p, cnt + C_SCR, (long long)scr.n);
+        GCDT_LAUNCH_CHECK();
+        // Few long pieces: the larger workgroup for all of them, in one launch (two
         // in turn last as long as their longest cavities together: 1,000 rows over
         // 100,000 points 6.6 -> 5.9 ms).  Many: a wave each for the smaller ones,
         // as the larger workgroup's LDS admits two to a CU.
@@ -1330,12 +1334,18 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
         k_cav_fix<<<grid_for(std::max<long long>((long long)FIX_LANES * (nq - nlong), npl)), kBlock, 0, cx.st>>>(
             c, wins.p, cnt + C_NWIN, scr.p, rew.p, cnt + C_NREW, ep, touched, tlist, cnt + C_NPIECE, tlist ? T : 0);
         GCDT_LAUNCH_CHECK();
-        cx.read(0, C_NUM);
-        if (cx.hcnt[C_ERR]) cx.check_err();
-        nq = cx.hcnt[C_NQ2];
-        if (nq > 0 && cx.hcnt[C_NWIN] == 0) throw Error(GCDT_ERR_INTERNAL, "constraint round without progress");
-        res.rewritten = cx.hcnt[C_NPIECE];
         std::swap(Q, Q2);
+        // After the first round, which is often the only one, the host looks
+        // whether it was the last; a later one is followed by the next round's
+        // claims at once, whose counters tell (a wait is 10 us, and the claims of
+        // an empty queue as much).
+        if (r == 1) {
+            cx.read(0, C_NUM);
+            if (cx.hcnt[C_ERR]) cx.check_err();
+            nq = cx.hcnt[C_NQ2];
+            if (nq > 0 && cx.hcnt[C_NWIN] == 0) throw Error(GCDT_ERR_INTERNAL, "constraint round without progress");
+            res.rewritten = cx.hcnt[C_NPIECE];
+        }
     }
     res.rounds = r;
     if (defer) {

@@ -198,8 +198,6 @@ __device__ inline void round_snap_store(const RoundSnap& s)
     }
 }
 
-__global__ void k_round_snap(RoundSnap s) { round_snap_store(s); }
-
 __global__ __launch_bounds__(kBlock) void k_rounds_start(int* ring, int next, int base)
 {
     static_assert(ROUND_INTS == kBlock, "a workgroup per set");
@@ -287,12 +285,6 @@ RoundSnap Ctx::round_snap(int r)
     s.set = round_set(r);
     s.err = dcnt.p + C_ERR;
     return s;
-}
-
-void Ctx::round_snapshot(int r)
-{
-    k_round_snap<<<1, C_NUM, 0, st>>>(round_snap(r));
-    GCDT_LAUNCH_CHECK();
 }
 
 // through the mapped ring and a poll: a copy and a stream synchronisation cost
@@ -1576,10 +1568,10 @@ __global__ __launch_bounds__(kBlock) void k_locate_walk(S smp, const int2* pts, 
                     }
                     t = o0 < 0 ? x.a.x : (o1 < 0 ? x.a.y : x.a.z);
                 }
-                want = r >= 0;
-                if (!want) atomicOr(err, r == -2 ? MERR_DUPLICATE : MERR_LOCATE);
+                want = true;  // also when not found: the list's length is known to the host
+                if (r < 0) atomicOr(err, r == -2 ? MERR_DUPLICATE : MERR_LOCATE);
             }
-            loc[p] = want ? t * 4 + r : -1;
+            loc[p] = r >= 0 ? t * 4 + r : -1;
         }
         const int slot = sp.reserve(want ? 1 : 0);
         if (want) s_buf[slot] = (int)i;
@@ -1588,35 +1580,29 @@ __global__ __launch_bounds__(kBlock) void k_locate_walk(S smp, const int2* pts, 
 }
 
 template <class S>
-static int locate_walk_s(Ctx& c, const S& smp, const int2* pts, int n, long long nv, const int3* tri, const FRec* rec,
-                         int T, int* loc, int* pend)
+static void locate_walk_s(Ctx& c, const S& smp, const int2* pts, int n, long long nv, const int3* tri, const FRec* rec,
+                          int T, int* loc, int* pend)
 {
-    if (n <= 0) return 0;
+    if (n <= 0) return;
     DBuf<int> vt((size_t)nv);
     k_vertex_tri<<<grid_for(T), kBlock, 0, c.st>>>(tri, T, vt.p);
     GCDT_LAUNCH_CHECK();
-    {
-        ProfScope ps("locate_walk", c.st, n);
-        k_locate_walk<S><<<grid_for(n), kBlock, 0, c.st>>>(smp, pts, n, rec, T, vt.p, loc, pend, c.dcnt.p + C_NPEND,
-                                                           c.dcnt.p + C_ERR);
-        GCDT_LAUNCH_CHECK();
-    }
-    c.read(0, C_NUM);
-    if (c.hcnt[C_ERR]) c.check_err();
-    return c.hcnt[C_NPEND];
+    ProfScope ps("locate_walk", c.st, n);
+    k_locate_walk<S><<<grid_for(n), kBlock, 0, c.st>>>(smp, pts, n, rec, T, vt.p, loc, pend, c.dcnt.p + C_NPEND,
+                                                       c.dcnt.p + C_ERR);
+    GCDT_LAUNCH_CHECK();
 }
 
-int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const FRec* rec, int T, const int* ids,
-                const int* offs, int* loc, int* pend)
+void locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const FRec* rec, int T, const int* ids,
+                 const int* offs, int* loc, int* pend)
 {
-    return locate_walk_s(c, CellSampleOne{ids, offs}, pts, n, (long long)n + 4, tri, rec, T, loc, pend);
+    locate_walk_s(c, CellSampleOne{ids, offs}, pts, n, (long long)n + 4, tri, rec, T, loc, pend);
 }
 
-int locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
-                      long long NP, int K, const int3* tri, const FRec* rec, int T, int* loc, int* pend)
+void locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
+                       long long NP, int K, const int3* tri, const FRec* rec, int T, int* loc, int* pend)
 {
-    return locate_walk_s(c, CellSampleInst{vinst, cbase, lvl, cell_end}, pts, (int)NP, NP + 4LL * K, tri, rec, T, loc,
-                         pend);
+    locate_walk_s(c, CellSampleInst{vinst, cbase, lvl, cell_end}, pts, (int)NP, NP + 4LL * K, tri, rec, T, loc, pend);
 }
 
 // ================================================================== insertion rounds
@@ -1853,11 +1839,11 @@ constexpr int TAIL_BS = 1024;
 
 // What a persistent tail hands to the host ring in place of the counters: one
 // word per thread, the others 0.
-__device__ inline void tail_snap(const RoundSnap& snap, int n, int r, int err, int ntri, int flips)
+__device__ inline void tail_snap(const RoundSnap& snap, int n, int r, int err, int ntri, int flips, int props)
 {
     const int j = threadIdx.x;
     if (j >= C_NUM) return;
-    int v = j == C_TAIL_N ? n : j == C_TAIL_R ? r : j == C_TAIL_ERR ? err : j == C_NTRI ? ntri : j == C_TAIL_F ? flips : 0;
+    int v = j == C_TAIL_N ? n : j == C_TAIL_R ? r : j == C_TAIL_ERR ? err : j == C_NTRI ? ntri : j == C_TAIL_F ? flips : j == C_TAIL_P ? props : 0;
     if (j == C_ERR) v = __hip_atomic_load(snap.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     snap_store(&snap.dst[j], snap.seq, v);
 }
@@ -1988,9 +1974,15 @@ __device__ inline int ins_short_rounds(const Ins& s, const int* P, int n, InsLis
     return n;
 }
 
-__global__ __launch_bounds__(TAIL_BS) void k_ins_tail(Ins s, int* P, int* P2, int n, int ntri, unsigned epoch0,
-                                                      int max_rounds, RoundSnap snap)
+// set: the counters of the launched round that made the list P (the host has
+// not waited for them), or null: n points and ntri triangles
+__global__ __launch_bounds__(TAIL_BS) void k_ins_tail(Ins s, int* P, int* P2, int n, int ntri, const int* set,
+                                                      unsigned epoch0, int max_rounds, RoundSnap snap)
 {
+    if (set) {
+        n = set[R_NEXT];
+        ntri = set[R_BASE] + set[R_NEW];
+    }
     __shared__ int s_np, s_nt, s_tb, s_np2[2];
     __shared__ InsList s_list[2];
     unsigned ep = epoch0;
@@ -2044,7 +2036,7 @@ __global__ __launch_bounds__(TAIL_BS) void k_ins_tail(Ins s, int* P, int* P2, in
         __syncthreads();
     }
     __syncthreads();
-    tail_snap(snap, n, r, err, s_nt, 0);
+    tail_snap(snap, n, r, err, s_nt, 0, 0);
 }
 
 int insert_rounds(Ctx& c, const Ins& s_in, DBuf<int>& pend, DBuf<int>& pend2, int npend, int ntri, int* rounds)
@@ -2118,17 +2110,16 @@ int insert_rounds(Ctx& c, const Ins& s_in, DBuf<int>& pend, DBuf<int>& pend2, in
         std::swap(P, P2);
         if (r >= 2) check_round(c.round_wait(r - 1));  // round r is queued
     }
-    if (r >= 1) {
-        c.round_snapshot(r);
-        check_round(c.round_wait(r));
-    }
     if (!done) {
-        // finish in one persistent workgroup
+        // finish in one persistent workgroup, which reads the last launched
+        // round's counters itself (a wait here idles the GPU for 10 us)
+        prof_add_items("ins_split", r ? nw_in : 0);
+        prof_add_items("ins_reloc", r ? n_in : 0);
         unsigned ep0 = c.epoch + 1;
         RoundSnap snap = c.round_snap(0);
         {
             ProfScope ps("ins_tail", c.st, est);
-            k_ins_tail<<<1, TAIL_BS, 0, c.st>>>(s, P, P2, est, nt, ep0, 1 << 20, snap);
+            k_ins_tail<<<1, TAIL_BS, 0, c.st>>>(s, P, P2, est, nt, r ? c.round_set(r) : nullptr, ep0, 1 << 20, snap);
             GCDT_LAUNCH_CHECK();
         }
         const int* h = c.round_wait(0);
@@ -2497,9 +2488,10 @@ __device__ inline int short_round(const FlipP& f, int* list, FRec* rec, bool kep
 }
 
 // Persistent single-workgroup tail of the flip rounds.
+// set: the counters of the launched round that made the list A, or null: n.
 template <class E>
-__global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int* lf, int n, int cap, unsigned epoch0,
-                                                       int max_rounds, int* eflag, RoundSnap snap)
+__global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int* lf, int n, const int* set, int cap,
+                                                       unsigned epoch0, int max_rounds, int* eflag, RoundSnap snap)
 {
     // round counters double-buffered by round parity: a round's pair is reset
     // after the round's first barrier, which every thread passes only after
@@ -2513,7 +2505,17 @@ __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int*
     __shared__ int s_list[E::kFused ? 2 * SHORT_MAX : 1];
     __shared__ int4 s_rec[E::kFused ? SHORT_MAX * (sizeof(FRec) / sizeof(int4)) : 1];
     unsigned ep = epoch0;  // A, B and lf hold cap entries each, n <= cap
-    int r = 0, err = 0, flips = 0;
+    int r = 0, err = 0, flips = 0, props = 0;
+    if (set) {
+        n = min(set[R_NEXT], cap);
+        flips = set[R_FLIP] / 2;
+        props = set[R_PROP];
+        // the highest-keyed proposal always wins both of its triangles
+        if (n > 0 && flips == 0) {
+            err = 1;
+            max_rounds = 0;
+        }
+    }
     int nf = 0;
     if (threadIdx.x == 0) {
         s_n2[0] = 0;
@@ -2625,7 +2627,7 @@ __global__ __launch_bounds__(TAIL_BS) void k_flip_tail(E e, int* A, int* B, int*
         __syncthreads();
     }
     __syncthreads();
-    tail_snap(snap, n, r, err, 0, flips);
+    tail_snap(snap, n, r, err, 0, flips, props);
 }
 
 template <class E>
@@ -2785,15 +2787,13 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
     };
     launch_rounds(c.tail_threshold, c.single_tester);
     launch_rounds(FLIP_WG_LIST, 0);
-    if (r >= 1) {
-        c.round_snapshot(r);
-        check_round(c.round_wait(r));
-        // the last round's flips are settled by the tail: flipped triangles are
-        // in the next list, so a round with flips is never the last
-        if (E::kFused) prof_add_items("flip_test_fix", settled - n_flip);
-    }
+    // the last round's flips are settled by the tail: flipped triangles are in
+    // the next list, so a round with flips is never the last
+    if (E::kFused && r) prof_add_items("flip_test_fix", settled);
     if (!done) {
-        // the rest in one persistent workgroup
+        // the rest in one persistent workgroup, which reads the last launched
+        // round's counters itself
+        const int last = r;
         unsigned ep0 = c.epoch + 1;
         if (!act) {  // small mesh: materialise the implicit list
             k_iota<<<grid_for(est), kBlock, 0, c.st>>>(lb.p, est);
@@ -2810,8 +2810,8 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
         RoundSnap snap = c.round_snap(0);
         {
             ProfScope ps("flip_tail", c.st, est);
-            k_flip_tail<E><<<1, TAIL_BS, 0, c.st>>>(e, (int*)act, nxt, lf.p, est, T, ep0, 1 << 20, c.dcnt.p + C_ERR,
-                                                    snap);
+            k_flip_tail<E><<<1, TAIL_BS, 0, c.st>>>(e, (int*)act, nxt, lf.p, est, last ? c.round_set(last) : nullptr, T,
+                                                    ep0, 1 << 20, c.dcnt.p + C_ERR, snap);
             GCDT_LAUNCH_CHECK();
         }
         const int* h = c.round_wait(0);
@@ -2820,6 +2820,11 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
         r += h[C_TAIL_R];
         c.epoch += (unsigned)h[C_TAIL_R];
         flips += h[C_TAIL_F];
+        if (last) {
+            prof_add_items("flip_test", n_in);
+            prof_add_items("flip_apply", h[C_TAIL_P]);
+            if (!E::kFused) prof_add_items("flip_fix", 2LL * h[C_TAIL_F]);
+        }
         if (h[C_TAIL_N] != 0) throw Error(GCDT_ERR_NOT_CONVERGED, "flip tail did not converge");
     }
     if (rounds) *rounds = r;

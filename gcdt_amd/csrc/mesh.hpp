@@ -114,6 +114,7 @@ enum : int {
     C_TAIL_R = 17,    // rounds done
     C_TAIL_ERR = 18,  // 1 = a round without progress
     C_TAIL_F = 20,    // flips done
+    C_TAIL_P = 21,    // proposals of the launched round before the tail
     C_STN_T = 24,     // crossing pass: triangles in use
     C_STN_S = 25,     // crossing pass: crossing vertices
     C_HUGE = 26,      // count passes: cells of more elements than one workgroup sorts
@@ -242,7 +243,6 @@ struct Ctx {
     void rounds_turn(int r);  // before round r is queued: clears sets that come into use later
     RoundSnap round_snap(int r);
     const int* round_wait(int r) { return wait_snapshot(r & 1); }
-    void round_snapshot(int r);  // a launch of its own, after the last round
     void check_err();  // throws on a device error flag
     // deferred pool releases of a solve on a non-null stream
     std::vector<PendingFree> deferred;
@@ -375,15 +375,16 @@ void build_bitmap(Ctx& c, const int2* pts, const int3* tri, int T, int** offsets
 int locate_bitmap(Ctx& c, const int2* pts, int n, const int3* tri, int T, const int* bm_off, const int* bm_tri,
                   int* loc, int* isv, int* pend);
 // Location without a bitmap: every point of [0,n) that is no sample walks through
-// the sample Delaunay mesh from its own cell's sample; fills loc and pend,
-// returns npend.  tri and rec: the sample mesh and its flip records; ids / offs
+// the sample Delaunay mesh from its own cell's sample; fills loc and pend (all
+// but the samples; a point that is not found gets loc -1 and an error bit, which
+// the next check of the counters meets).  tri and rec: the sample mesh and its flip records; ids / offs
 // as sample_points_morton gives them.  (The bitmap's
 // build alone costs 190 us with its launches and waits; the walk also wins at
 // 10M points, 27.68 -> 27.48 ms of kernels.)
-int locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const FRec* rec, int T, const int* ids,
-                const int* offs, int* loc, int* pend);
-int locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
-                      long long NP, int K, const int3* tri, const FRec* rec, int T, int* loc, int* pend);
+void locate_walk(Ctx& c, const int2* pts, int n, const int3* tri, const FRec* rec, int T, const int* ids,
+                 const int* offs, int* loc, int* pend);
+void locate_walk_batch(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl, const int* cell_end,
+                       long long NP, int K, const int3* tri, const FRec* rec, int T, int* loc, int* pend);
 // locate all points of [0,n) in the two corner triangles 0/1
 int locate_two(Ctx& c, const int2* pts, int n, int* loc, int* pend);
 // adjacency of a plain triangle list (edges matched through vertex buckets)
