@@ -284,9 +284,15 @@ int gcdt_prof_names(char* buf, int cap) { return prof_names(buf, cap); }
 namespace gcdt {
 
 // Full pipeline on device arrays; pts holds N+4 entries (corners written here).
-// bytes counted for the phases before the constraints beside those per point,
-// sample point and segment
-constexpr size_t NOALLOC_BASE = 21243136;
+// The solve on a fixed array takes or refuses an input by a demand that follows
+// from the input alone (N points, S of them in the sample, C segments) and from
+// what the caller holds, whatever the phases make of it: the peak before the
+// constraints, and what they start from.
+static size_t noalloc_demand_insert(size_t top, int N, int S) { return top + 38037504 + 324 * (size_t)N + 160 * (size_t)S; }
+static size_t noalloc_demand_cons(size_t top, int N, int S, int C)
+{
+    return top + 21242624 + 148 * (size_t)N + 168 * (size_t)S + 8 * (size_t)C;
+}
 
 void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, int3* tris_out, int3* adj_out,
                 SolveOut& out, int* cflag_out, const SteinerArgs* steiner)
@@ -294,6 +300,8 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     gcdt_stats& st = out.st;
     Timer total(c.st);
     // work in Morton order for locality; ids are mapped back at the end
+    // held by the caller; the context's own buffers are not counted
+    const size_t top0 = g_arena ? g_arena->top - sizeof(int) * (ROUND_SETS * ROUND_INTS + ARENA_SCAN_SUMS) : 0;
     DBuf<int2> pts_buf((size_t)N + 4);
     DBuf<int> perm(N > 0 ? N : 1), inv(N > 0 ? N : 1);
     DBuf<int2> cons_buf(C > 0 ? C : 1);
@@ -306,6 +314,7 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     PhaseClock phase;
     DBuf<int> sid(1 << 16), soff((1 << 16) + 1);
     int S = sample_points_morton(c, pts, cell_end.p, sid.p, soff.p);
+    if (g_arena) g_arena->require(noalloc_demand_insert(top0, N, S));
     // cell_end stays for the constraints' split pass
     DBuf<int> loc((size_t)N + 4), pend((size_t)(N > 1 ? N : 1)), pend2((size_t)(N > 1 ? N : 1));
     DBuf<unsigned long long> pkey((size_t)N + 4);
@@ -397,11 +406,9 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
         Mesh m{pts, tris_out, adj_out, nullptr, cflag};
         ConsDefer defer;
         DBuf<int> tl(T);
-        // The solve on a fixed array takes or refuses an input by a demand that
-        // follows from the input alone, whatever the phases before still hold.
         DBuf<int> held;
         if (g_arena) {
-            const size_t demand = NOALLOC_BASE + 172 * (size_t)N + 168 * (size_t)S + 8 * (size_t)C;
+            const size_t demand = noalloc_demand_cons(top0, N, S, C);
             if (demand > g_arena->top) held.alloc((demand - g_arena->top) / sizeof(int));
         }
         ConsResult cr = insert_constraints(c, m, T, N + 4, N, cons, C, touched.p, tl.p, cell_end.p,

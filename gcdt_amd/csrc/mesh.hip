@@ -61,12 +61,17 @@ int g_grid_cap = kMaxGrid;
 
 thread_local Arena* g_arena = nullptr;
 
+void Arena::require(size_t bytes) const
+{
+    if (bytes > cap)
+        throw Error(GCDT_ERR_SCRATCH, "the scratch array (" + std::to_string(cap) + " bytes) is too small for this "
+                                      "input: " + std::to_string(bytes) + " bytes needed so far");
+}
+
 void* Arena::take(size_t bytes)
 {
     size_t len = (bytes + 255) & ~(size_t)255;
-    if (len > cap - top)
-        throw Error(GCDT_ERR_SCRATCH, "the scratch array (" + std::to_string(cap) + " bytes) is too small for this "
-                                      "input: " + std::to_string(top + len) + " bytes needed so far");
+    require(top + len);
     void* p = base + top;
     top += len;
     if (top > high) high = top;
@@ -153,8 +158,11 @@ Ctx::Ctx(hipStream_t s, const HostSlot* fixed) : st(s)
     flip_items = Tunables::get().flip_items;
     ins_items = Tunables::get().ins_items;
     dcnt.alloc(C_NUM);
-    // on a fixed array below everything that is given back before it
-    if (g_arena) ring.ensure(ROUND_SETS * ROUND_INTS);
+    // on a fixed array below everything that is given back before them
+    if (g_arena) {
+        ring.ensure(ROUND_SETS * ROUND_INTS);
+        scan_sums.ensure(ARENA_SCAN_SUMS);
+    }
     HostSlot h = fixed ? *fixed : take_host_slot();
     fixed_slot = fixed != nullptr;
     hcnt = h.hcnt;
@@ -3431,7 +3439,9 @@ static int filter_leaves_sorted(Ctx& c, CK ck, const KEY& kf, long long ncells, 
 int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
                              FRec* rec, long long nleaf)
 {
-    const int b = leaf_bits(nleaf);
+    // on a fixed array, where the longer keys of a crowded coarse cell count, for
+    // the smallest meshes only
+    const int b = g_arena && nleaf > 65536 ? LEAF_CELL_BITS : leaf_bits(nleaf);
     const LeafKeyOne key{2 * (LEAF_CELL_BITS - b)};
     if (b == LEAF_CELL_BITS)
         return filter_leaves_sorted(c, CellKeyTri{}, key, LEAF_CELLS, pts, tri, adj, sons, T, rec, nleaf);

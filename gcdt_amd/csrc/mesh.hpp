@@ -40,6 +40,7 @@ struct Arena {
     bool owns(const void* p) const { return (const char*)p >= base && (const char*)p < base + cap; }
     void* take(size_t bytes);
     void give(void* p, size_t bytes);
+    void require(size_t bytes) const;  // GCDT_ERR_SCRATCH unless the region holds as much
 };
 extern thread_local Arena* g_arena;
 
@@ -183,6 +184,8 @@ struct HostSlot {
 };
 // a slot from the process-wide free list, or newly allocated pinned pages
 HostSlot take_host_slot();
+
+constexpr int ARENA_SCAN_SUMS = 4096 + 1;  // tiles of the largest scan on a fixed array, and more
 
 struct Ctx {
     hipStream_t st = nullptr;
