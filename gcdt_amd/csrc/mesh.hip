@@ -1863,7 +1863,10 @@ __device__ inline void tail_snap(const RoundSnap& snap, int n, int r, int err, i
 // vertices it was just located by, while the last waves settle the outer
 // adjacency of the round's new triangles (ins_edge_neighbour).
 // Returns the points left (0 unless the round limit or an error stops it).
-constexpr int INS_LIST = 4096;
+#ifndef GCDT_INS_LIST
+#define GCDT_INS_LIST 4096
+#endif
+constexpr int INS_LIST = GCDT_INS_LIST;
 
 struct InsList {
     int p[INS_LIST];
@@ -2429,7 +2432,11 @@ __global__ __launch_bounds__(kBlock) void k_flip_fix(E e, const int* list, const
 // Such a round is a chain of waits: list, record, neighbours, up to three
 // in-circle tests in a row (0.4 us each for a lone wave), claims, and in the
 // apply list, record, neighbour and stores again.
-constexpr int SHORT_MAX = TAIL_BS / 4;
+#ifndef GCDT_SHORT_MAX
+#define GCDT_SHORT_MAX (TAIL_BS / 4)
+#endif
+constexpr int SHORT_MAX = GCDT_SHORT_MAX;
+static_assert(4 * SHORT_MAX <= TAIL_BS, "four lanes a triangle");
 
 __device__ inline int short_round(const FlipP& f, int* list, FRec* rec, bool kept, int n, unsigned ep,
                                   const LdsClaims& cl, const LdsClaims& next, int* n2, int* nf, int q, int* lf)
