@@ -42,30 +42,30 @@ def _checker(args):
 
 # Algorithmic bytes per processed list item of the instrumented kernels.
 #   flip_test : tri 12 + adj 12 + cflag 4 + own 3 points 24
-#               + 3 x (neighbour tri 12 + opposite point 8) + cand 4 + 2 claims 16
-#   ins_reloc : loc 4 + sons 4 + list write 4 + 2 children tri 24 + 3 points 24 + loc write 4
-#               + next round's claim: key write 8 + claim atomic 8 + claimed-triangle append 4
+#               + 3 x (neighbour tri 12 + opposite point 8) + proposal 4 + tag 1 + claim 8
+#   ins_reloc : list 4 + loc 4 + sons 4 + claim 8 + parent tri 12 + 4 points 32 + list write 4
+#               + next round's claim: claim atomic 8 + claimed-triangle append 4
 #   ins_claim : loc 4 + point id 4 + 1.x claim atomics 8 (first round of a run only)
-#   ins_split : per claimed triangle: list 4 + claim 8 + winner loc 4 + key 8 + tri/adj 24
+#   ins_split : per claimed triangle: list 4 + claim 8 + winner loc 4 + tri/adj 24
 #               + 3 children x (tri 12 + adj 12) written + sons 4 + loc 4
-#   flip_apply: per proposal meta 4 + own claim 8; a winning proposal (92.2% of them on
+#   flip_apply: per proposal list 4 + own claim 8; a winning proposal (92.2% of them on
 #               the 10M workload) adds its own vertices, neighbours and coordinates 48,
-#               the neighbour record's 60, both records rewritten 2 x 56 and 4 list
-#               entries 16; a losing one the winner's claim 8, its mark 4 and a list
-#               entry 4: 12 + 0.922 x 236 + 0.078 x 16 = 231
-#   locate_bitmap: point 8 + isv 4 + 2 offsets 8 + ~1.5 x (tri id 4 + tri 12 + 3 points 24) + loc 4 + list 4
+#               the neighbour record's 60 and tag 1, both records rewritten 2 x 56 and
+#               2 list entries 8; a losing one the winner's claim 8, its mark 4 and a
+#               list entry 4: 12 + 0.922 x 229 + 0.078 x 16 = 224
+#   locate_walk: point 8 + sample 8 + its triangle 4 + ~3 records x 48 + loc 4 + list 4
 # With the packed records, each flip_test launch also settles the previous
 # round's flips (listed as flip_test_fix items): per settled triangle, 2 x
 # (neighbour adj 12 + stamp 4 + meta 4) read + 2 own slots and 2 back-pointers
 # written (16); its other reads are the test's own.
 BYTES_PER_FIX_IN_TEST = 56
 BYTES_PER_ITEM = {
-    "flip_test": 132,
-    "ins_reloc": 84,
+    "flip_test": 125,
+    "ins_reloc": 80,
     "ins_claim": 16,
-    "flip_apply": 231,
-    "locate_bitmap": 88,
-    "ins_split": 128,
+    "flip_apply": 224,
+    "locate_walk": 172,
+    "ins_split": 120,
 }
 
 

@@ -85,7 +85,7 @@ size_t gcdt_scratch_bytes(int64_t n);
 
 /* Live kernel timing: while enabled, launches of the instrumented kernels
  * (ins_claim, ins_split, ins_fix, ins_reloc, flip_test, flip_apply,
- * flip_fix, locate_bitmap) are bracketed by hipEvents on their stream.
+ * flip_fix, locate_walk) are bracketed by hipEvents on their stream.
  * gcdt_prof_read returns the summed milliseconds, launch count and items
  * processed (list entries) of one kernel; gcdt_prof_names writes the
  * ';'-separated names seen so far and returns the full length. */
@@ -176,7 +176,7 @@ int gcdt_add_constraints(void* tmp, size_t tmpBytes, const gcdt_int2* points, gc
 typedef struct {
     double ms_total;       /* GPU time of the whole solve */
     double ms_sample;      /* sampling + sample mesh + sample flips */
-    double ms_bitmap;
+    double ms_bitmap;      /* 0: points are located by walks, counted in ms_insert */
     double ms_insert;      /* location + insertion rounds */
     double ms_flip;        /* Delaunay flips of the full mesh */
     double ms_constraints; /* constraint recovery + constrained flips */
