@@ -37,10 +37,15 @@ __device__ inline unsigned long long ld_u64(const unsigned long long* p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // The same for words that only one workgroup touches while it runs: performed
-// in its own L2 (a device-scope atomic goes to memory and back).
+// in its own L2 (a device-scope atomic goes to memory and back).  A compiler
+// without the scoped builtin takes the device-scope one, which serves as well.
 __device__ inline unsigned long long at_max_wg(unsigned long long* p, unsigned long long v)
 {
+#if __has_builtin(__hip_atomic_fetch_max)
     return __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#else
+    return atomicMax(p, v);
+#endif
 }
 __device__ inline unsigned long long ld_u64_wg(const unsigned long long* p)
 {
