@@ -1204,14 +1204,13 @@ static void cell_reorder_huge(Ctx& c, const KF& kf, const int* end, const typena
     GCDT_LAUNCH_CHECK();
 }
 
-// What the count passes leave in C_HUGE: buckets of more than CELL_RANK_MAX
-// elements, plus CELL_HUGE for each of more than CELL_BLOCK_MAX (so many of the
-// former that they reach CELL_HUGE only cost the larger path an empty scan).
-constexpr int CELL_HUGE = 1 << 20;
+// What the count passes leave in C_HUGE: CELL_LARGE when a bucket holds more than
+// CELL_RANK_MAX elements, CELL_HUGE when one holds more than CELL_BLOCK_MAX.
+enum : int { CELL_LARGE = 1, CELL_HUGE = 2 };
 __device__ inline void count_large(int r, int* huge)
 {
-    if (r == CELL_RANK_MAX) atomicAdd(huge, 1);
-    if (r == CELL_BLOCK_MAX) atomicAdd(huge, CELL_HUGE);
+    if (r == CELL_RANK_MAX) atomicOr(huge, CELL_LARGE);
+    if (r == CELL_BLOCK_MAX) atomicOr(huge, CELL_HUGE);
 }
 
 // eb[0..n): (element, bucket, ...), grouped by bucket.  Each element is
@@ -1221,16 +1220,15 @@ template <class KF>
 static void cell_reorder(Ctx& c, const KF& kf, const int* end, const typename KF::Slot* eb, long long n, int large)
 {
     if (n <= 0) return;
-    const bool huge = large >= CELL_HUGE;
     // a list entry per bucket above the rank cap: at most n / (cap + 1)
     DBuf<int> big((size_t)(n / (CELL_RANK_MAX + 1) + 1));
     k_cell_rank<KF><<<grid_for(n), kBlock, 0, c.st>>>(kf, end, eb, n, big.p, c.dcnt.p + C_NQ);
     GCDT_LAUNCH_CHECK();
-    if (large) {
+    if (large & CELL_LARGE) {
         k_cell_sort_block<KF><<<1024, kBlock, 0, c.st>>>(kf, end, big.p, c.dcnt.p + C_NQ, eb);
         GCDT_LAUNCH_CHECK();
     }
-    if (huge) cell_reorder_huge(c, kf, end, eb, n);
+    if (large & CELL_HUGE) cell_reorder_huge(c, kf, end, eb, n);
 }
 
 // Counting sort of points by 20-bit Morton cell: the count pass keeps the

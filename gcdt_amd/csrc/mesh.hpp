@@ -118,7 +118,7 @@ enum : int {
     C_TAIL_P = 21,    // proposals of the launched round before the tail
     C_STN_T = 24,     // crossing pass: triangles in use
     C_STN_S = 25,     // crossing pass: crossing vertices
-    C_HUGE = 26,      // count passes: cells of more elements than one workgroup sorts
+    C_HUGE = 26,      // count passes: CELL_LARGE / CELL_HUGE (mesh.hip)
     C_VAL = 27,       // mesh check: failed checks (VAL_* bits)
     C_VAL_FIRST = 28, // mesh check: first failing triangle
     C_NLONG = 29,  // constraint rounds: pieces that cross many triangles
