@@ -894,8 +894,8 @@ struct SegStrips {
 
 __device__ inline bool seg_valid(int2 e, int nmax) { return e.x >= 0 && e.y >= 0 && e.x < nmax && e.y < nmax && e.x != e.y; }
 
-// Vertices strictly inside each segment, one wave per segment: its lanes take
-// strips in turn, test the points of every cell and collect the vertices on
+// Vertices strictly inside each segment, one wave per segment: its lanes share
+// the strips, test the points of every cell and collect the vertices on
 // the segment in LDS, where they are sorted along it.  They leave at hpos[i]
 // of hits[] (room permitting: the cursor counts on and the caller repeats the
 // launch with more), np[i] = pieces of the segment.  A segment with more than
@@ -903,6 +903,12 @@ __device__ inline bool seg_valid(int2 e, int nmax) { return e.x >= 0 && e.y >= 0
 // Bound by the latency of a strip's chain (cell ends, points); the passes of
 // one thread per segment and strip that this replaces took 155 + 186 us for
 // 12 segments over 300 points and 864 + 1,024 us for 1,000 rows over 100,000.
+// A segment of up to 32 strips has several lanes to a strip, which stride over
+// the points of its cells: a short segment lies in one or two cells, and with
+// a lane to a strip 20,000 of them in one cell of 200,000 points took 222 ms
+// (the two passes before 56; so 4.8), 20,000 of them in 100 cells 2.7 ms (1.2;
+// so 0.4).  Constraint recovery of 100,000 segments among 1M points all over
+// the square takes 0.6 ms either way.
 __global__ __launch_bounds__(64) void k_seg_find(const int2* pts, const int* cell_end, const int2* cons, int C, int nmax,
                                                  int* np, int* hcnt, int* hpos, int* hits, int hcap, int* hcur,
                                                  int* walk_list, int* nwalk, int* err)
@@ -926,13 +932,17 @@ __global__ __launch_bounds__(64) void k_seg_find(const int2* pts, const int* cel
         const int2 A = pts[e.x], B = pts[e.y];
         const long long dx = (long long)B.x - A.x, dy = (long long)B.y - A.y;
         const SegStrips g(A, B);
-        for (int st = g.first() + lane; st <= g.last(); st += 64) {
+        const int first = g.first(), last = g.last();
+        int per = 1;  // lanes to a strip
+        while (2 * per * (last - first + 1) <= 64) per <<= 1;
+        const int sub = lane & (per - 1);
+        for (int st = first + lane / per; st <= last; st += 64 / per) {
             int lo, hi;
             g.cells(st, lo, hi);
             for (int v = lo; v <= hi; v++) {
                 const unsigned cell = g.rows ? cell_morton((unsigned)v, (unsigned)st) : cell_morton((unsigned)st, (unsigned)v);
                 const int p1 = cell_end[cell];
-                for (int p = cell ? cell_end[cell - 1] : 0; p < p1; p++) {
+                for (int p = (cell ? cell_end[cell - 1] : 0) + sub; p < p1; p += per) {
                     if (p == e.x || p == e.y) continue;
                     const int2 P = pts[p];
                     if (orient2d(A, B, P) != 0 || !strictly_between(A, B, P)) continue;
