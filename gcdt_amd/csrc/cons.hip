@@ -490,10 +490,14 @@ struct DvWave {
 #ifndef GCDT_CAV_MID_K
 #define GCDT_CAV_MID_K 128
 #endif
+#ifndef GCDT_CAV_FEW
+#define GCDT_CAV_FEW 1024  // long pieces of a round
+#endif
 #ifndef GCDT_CAV_LDS_K
 #define GCDT_CAV_LDS_K 2048
 #endif
 constexpr int CAV_MID_K = GCDT_CAV_MID_K;
+constexpr int CAV_FEW = GCDT_CAV_FEW;
 constexpr int CAV_LDS_K = GCDT_CAV_LDS_K;
 // nodes of up to this many candidates are scanned by as many lanes, several
 // nodes at once; larger ones by a wave each
@@ -1315,11 +1319,20 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
         k_cav_check<<<g, kBlock, 0, cx.st>>>(c, Q, cnt + C_NQ, ncross.p, paths.p, ppos.p, ep, Q2, cnt + C_NQ2, wins.p,
                                              cnt + C_NWIN, scr.p, cnt + C_SCR, (long long)scr.n);
         GCDT_LAUNCH_CHECK();
-        // Few long pieces: the larger workgroup for all of them, in one launch (two
-        // in turn last as long as their longest cavities together: 1,000 rows over
-        // 100,000 points 6.6 -> 5.9 ms).  Many: a wave each for the smaller ones,
-        // as the larger workgroup's LDS admits two to a CU.
-        const int mid_k = nlong <= 1024 ? CAV_WAVE_K : CAV_MID_K;
+        // Few long pieces, or very long ones: the larger workgroup for all of them, in
+        // one launch (two in turn last as long as their longest cavities
+        // together).  Many of up to CAV_MID_K triangles on average: a wave each for
+        // those below it, as the larger workgroup's LDS admits two to a CU.  Solves
+        // with c segments that cross k triangles each, one workgroup size / both:
+        //   n 100,000  c 1,000  k 350        4.36 / 5.27 ms
+        //   n 100,000  c 4,000  k 300        7.72 / 9.24
+        //   n 1M       c 4,000  k 1,000     13.03 / 14.20
+        //   n 1M       c 8,000  k 200        7.10 / 7.87
+        //   n 1M       c 2,000  k 80         3.74 / 3.70
+        //   n 1M       c 8,000  k 80         5.44 / 5.12
+        //   n 4M       c 32,000  k 80       14.25 / 12.52
+        const bool many = nlong > CAV_FEW && npl <= (long long)CAV_MID_K * nlong;
+        const int mid_k = many ? CAV_MID_K : CAV_WAVE_K;
         if (nlong > 0) {
             k_cav_check_long<<<grid_for(64LL * nlong), kBlock, 0, cx.st>>>(
                 c, Q, longq.p, cnt + C_NLONG, ncross.p, paths.p, ppos.p, ep, Q2, cnt + C_NQ2, wins.p, cnt + C_NWIN,
@@ -1331,7 +1344,7 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
                                                                                            cnt + C_NWIN, ep);
             GCDT_LAUNCH_CHECK();
         }
-        if (nlong > 0 && mid_k == CAV_MID_K) {
+        if (nlong > 0 && many) {
             k_cav_retri_block<64, CAV_MID_K, false><<<std::min(nlong, 8192), 64, 0, cx.st>>>(
                 c, pieces.p, wins.p, longw.p, cnt + C_NMID, cnt + C_NLONG, scr.p, ep, rew.p, cnt + C_NREW);
             GCDT_LAUNCH_CHECK();
