@@ -274,7 +274,8 @@ int prof_names(char* buf, int cap);
 // primitives
 void fill_i32(Ctx& c, int* p, int v, long long n);
 void fill_u64(Ctx& c, unsigned long long* p, unsigned long long v, long long n);
-// several fills in one launch; each repeats a 32-bit word
+// several fills in one launch; each repeats a 32-bit word (p null: an output
+// that the caller did not ask for, nothing to fill)
 struct FillJobs {
     static constexpr int kMax = 6;
     struct Job {
@@ -285,7 +286,9 @@ struct FillJobs {
     int njobs = 0;
     void add(void* p, int v, long long n)
     {
-        if (n > 0) job[njobs++] = Job{(int*)p, n, v};
+        if (n <= 0 || !p) return;
+        if (njobs == kMax) throw Error(GCDT_ERR_INTERNAL, "more fills in one launch than it takes");
+        job[njobs++] = Job{(int*)p, n, v};
     }
 };
 void fill_jobs(Ctx& c, const FillJobs& f);
