@@ -283,25 +283,41 @@ int gcdt_prof_names(char* buf, int cap) { return prof_names(buf, cap); }
 
 namespace gcdt {
 
-// Full pipeline on device arrays; pts holds N+4 entries (corners written here).
-// The solve on a fixed array takes or refuses an input by a demand that follows
-// from the input alone (N points, S of them in the sample, C segments) and from
-// what the caller holds, whatever the phases make of it: the peak before the
-// constraints, and what they start from.
-static size_t noalloc_demand_insert(size_t top, int N, int S) { return top + 38037504 + 324 * (size_t)N + 160 * (size_t)S; }
-static size_t noalloc_demand_cons(size_t top, int N, int S, int C)
+// The solve on a fixed array takes an input or refuses it (GCDT_ERR_SCRATCH) by
+// the buffers below, in this order, and by those of the phases that follow
+// them; a buffer released below another one stays counted.  Phases that make
+// do with less hold the rest meanwhile, so that the limit is a matter of the
+// input alone and does not move with their layout.  These are the bytes in use
+// once the sample's mesh is there: `top` held by the caller, N points, C
+// segments, S points in the sample and nA triangle slots in its insertion.
+static size_t array_limit(size_t top, size_t N, size_t C, size_t S, size_t nA)
 {
-    return top + 21242624 + 148 * (size_t)N + 168 * (size_t)S + 8 * (size_t)C;
+    constexpr size_t cells = 1 << 20, leaf_cells = 1 << 22;  // of the points' sort and the leaves'
+    const size_t n1 = std::max<size_t>(N, 1), a = 4 * S + 8, b = 4 * N + 8;
+    const size_t bytes[] = {
+        8 * (N + 4), 4 * n1, 4 * n1, 8 * std::max<size_t>(C, 1),  // points, their order and its inverse, segments
+        4 * (cells + 1), 4 * (size_t)scan_scratch_ints(cells),    // cell ends, totals of their scan
+        4 << 16, 4 * (N + 4), 4 * n1, 4 * n1, 8 * (N + 4),        // sample, locations, two lists, claim keys
+        12 * a, 12 * a, 4 * a, 8 * a,                             // the sample mesh's insertion
+        12 * b, 12 * b,                                           // triangles and neighbours of the whole
+        4 * (leaf_cells + 1), 4 * nA, 4 * nA,                     // sample leaves: counts, cells, places
+        4 * (size_t)scan_scratch_ints(leaf_cells),                // totals of the counts' scan
+    };
+    for (size_t n : bytes) top += Arena::size(n);
+    return top;
 }
 
+// Full pipeline on device arrays; pts holds N+4 entries (corners written here).
 void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, int3* tris_out, int3* adj_out,
                 SolveOut& out, int* cflag_out, const SteinerArgs* steiner)
 {
     gcdt_stats& st = out.st;
     Timer total(c.st);
     // work in Morton order for locality; ids are mapped back at the end
-    // held by the caller; the context's own buffers are not counted
-    const size_t top0 = g_arena ? g_arena->top - sizeof(int) * (ROUND_SETS * ROUND_INTS + ARENA_SCAN_SUMS) : 0;
+    // on a fixed array: the bytes held by the caller, without the context's counters
+    const size_t top0 = g_arena ? g_arena->top - Arena::size(sizeof(int) * ROUND_SETS * ROUND_INTS) -
+                                      Arena::size(sizeof(int) * ARENA_SCAN_SUMS)
+                                : 0;
     DBuf<int2> pts_buf((size_t)N + 4);
     DBuf<int> perm(N > 0 ? N : 1), inv(N > 0 ? N : 1);
     DBuf<int2> cons_buf(C > 0 ? C : 1);
@@ -314,7 +330,6 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     PhaseClock phase;
     DBuf<int> sid(1 << 16), soff((1 << 16) + 1);
     int S = sample_points_morton(c, pts, cell_end.p, sid.p, soff.p);
-    if (g_arena) g_arena->require(noalloc_demand_insert(top0, N, S));
     // cell_end stays for the constraints' split pass
     DBuf<int> loc((size_t)N + 4), pend((size_t)(N > 1 ? N : 1)), pend2((size_t)(N > 1 ? N : 1));
     DBuf<unsigned long long> pkey((size_t)N + 4);
@@ -351,6 +366,8 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     validate_mesh(c, "the sample mesh's flips", Mesh{pts, tB.p, aB.p, nullptr, nullptr}, N + 4, Ts, true);
     st.ms_sample = phase.lap();
     // ---- 2. locate the rest, each walking from its own cell's sample
+    const size_t limit = g_arena ? array_limit(top0, N, C, S, ntA) : 0;
+    require_bitmap(c, pts, tB.p, Ts, limit, Arena::size(sizeof(int) * (size_t)std::max(N, 1)));
     const int np = N - S;
     locate_walk(c, pts, N, tB.p, recS.p, Ts, sid.p, soff.p, loc.p, pend.p);
     recS.release();
@@ -379,8 +396,11 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     pend.release();
     pend2.release();
     // leaves in Morton order, written straight into the packed flip records
+    DBuf<int> held;
+    hold_to(held, limit + Arena::size(sizeof(int) * (size_t)capB));
     DBuf<FRec> rec(2LL * N + 2);
     int T = filter_leaves_morton_rec(c, pts, tB.p, aB.p, sB.p, ntB, rec.p, 2LL * N + 2);
+    held.release();
     tB.release();
     aB.release();
     sB.release();
@@ -406,11 +426,7 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
         Mesh m{pts, tris_out, adj_out, nullptr, cflag};
         ConsDefer defer;
         DBuf<int> tl(T);
-        DBuf<int> held;
-        if (g_arena) {
-            const size_t demand = noalloc_demand_cons(top0, N, S, C);
-            if (demand > g_arena->top) held.alloc((demand - g_arena->top) / sizeof(int));
-        }
+        hold_to(held, limit + 2 * Arena::size(sizeof(int) * (size_t)T));  // touched, cflag
         ConsResult cr = insert_constraints(c, m, T, N + 4, N, cons, C, touched.p, tl.p, cell_end.p,
                                            steiner ? &defer : nullptr);
         st.constraint_rounds = cr.rounds;

@@ -1071,10 +1071,8 @@ __global__ __launch_bounds__(kBlock) void k_seg_walk(Cons c, const int2* cons, c
     }
 }
 
-// *nq: true when the pieces that need a cavity have been queued (C_NQ was
-// cleared by the caller, and C_NREW, C_NQ2 as cursors)
 // Cells that the closed segments can touch, column by column (a superset): what
-// the solve on a fixed array bounds its inputs by (demand_words).
+// the solve on a fixed array bounds its inputs by (split_limit).
 __global__ __launch_bounds__(64) void k_seg_demand(const int2* pts, const int2* cons, int C, int nmax, int* total)
 {
     for (int i = blockIdx.x; i < C; i += gridDim.x) {
@@ -1105,18 +1103,26 @@ __global__ __launch_bounds__(64) void k_seg_demand(const int2* pts, const int2* 
     }
 }
 
-// Words that a split of C segments, nh vertices on them and `pairs` touched
-// cells counts for in the array of a solve without allocations, above what it
-// uses: that solve has always been bounded by them, and an input is taken or
-// refused (GCDT_ERR_SCRATCH) by the input alone.
-static long long demand_words(int C, long long nh, long long pairs) { return 6LL * C + 4 + nh + 2 * pairs; }
+// Bytes that the solve on a fixed array counts for a split of C segments with
+// nh vertices on them and `pairs` touched cells, whatever it takes: offsets,
+// counts, positions and pieces by segment, two lists of segments, the
+// vertices, and each touched cell with its segment.
+static size_t split_limit(size_t C, size_t nh, size_t pairs)
+{
+    return 4 * Arena::size(4 * (C + 1)) + 2 * Arena::size(4 * C) + Arena::size(4 * std::max<size_t>(nh, 1)) +
+           2 * Arena::size(4 * std::max<size_t>(pairs, 1));
+}
 
-// pad: the rest of that demand, held while the constraints are inserted
+// Pieces of the segments, from the points' cells; *queued: those that need a
+// cavity are in queue already (C_NQ, C_NREW and C_NQ2 were cleared by the
+// caller).  pad: the rest of split_limit, held while the constraints are
+// inserted.
 static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const int2* cons, int C, int nmax,
                               DBuf<int2>& pieces, DBuf<int>& queue, bool* queued, DBuf<int>& pad)
 {
     const int2* pts = c.m.pts;
     int* cnt = cx.dcnt.p;
+    const size_t top0 = g_arena ? g_arena->top : 0;
     if (g_arena) {
         cx.set(C_STUCK, 0);
         k_seg_demand<<<std::min(C, 16384), 64, 0, cx.st>>>(pts, cons, C, nmax, cnt + C_STUCK);
@@ -1141,15 +1147,12 @@ static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const
     }
     int total = cx.hcnt[C_TOTAL];
     const int nwalk = cx.hcnt[C_NQ2];
-    if (g_arena) {
-        const long long held = (long long)(np.n + hcnt.n + hpos.n + wlist.n + hits.n);
-        const long long more = demand_words(C, cx.hcnt[C_NREW], cx.hcnt[C_STUCK]) - held;
-        if (more > 0) pad.alloc((size_t)more);
-    }
+    DBuf<int> cnts;
+    if (nwalk > 0) cnts.alloc((size_t)C + 1);
+    if (g_arena) hold_to(pad, top0 + split_limit(C, cx.hcnt[C_NREW], cx.hcnt[C_STUCK]));
     if (nwalk > 0) {
         // segments with many vertices keep the walk: their counts, and the
         // offsets again (from the counts of the others)
-        DBuf<int> cnts((size_t)C + 1);
         k_seg_counts<<<grid_for(C), kBlock, 0, cx.st>>>(cons, C, nmax, hcnt.p, cnts.p);
         GCDT_LAUNCH_CHECK();
         k_seg_walk<<<grid_for(nwalk), kBlock, 0, cx.st>>>(c, cons, wlist.p, cnt + C_NQ2, cnts.p, nullptr, nullptr);
@@ -1264,7 +1267,8 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
     int* Q = qa.p;
     int* Q2 = qb.p;
     DBuf<int> scr, rew;
-    DBuf<int> longq, longw, ppos, paths;
+    DBuf<int> longq, longw, ppos, paths, round_pad;
+    const size_t round_top = g_arena ? g_arena->top : 0;
     int r = 0;
     int* cnt = cx.dcnt.p;
     while (nq > 0) {
@@ -1311,11 +1315,12 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
         long long cap = (npath - npl) + 9 * npl + 16LL * nlong + 1024;
         if (cap > (1LL << 30)) cap = 1LL << 30;
         rew.ensure((size_t)npl + 1);
-        // the solve on a fixed array takes inputs up to a demand of 14 words per
-        // crossed triangle and 20 per piece here, whatever the round makes of them
-        const long long demand = std::min(13 * npath + 20LL * nq + 1024, 1LL << 30) + npath + 1,
-                        held = (long long)(paths.n + longq.n + longw.n + ppos.n + rew.n);
-        scr.ensure((size_t)std::max(cap, g_arena ? demand - held : 0LL));
+        scr.ensure((size_t)cap);
+        // a fixed array counts 13 words per crossed triangle and 20 per piece here,
+        // and a word per triangle for the list of them, whatever the round takes
+        if (r == 1 && g_arena)
+            hold_to(round_pad, round_top + Arena::size(sizeof(int) * (size_t)std::min(13 * npath + 20LL * nq + 1024, 1LL << 30)) +
+                                   Arena::size(sizeof(int) * (size_t)(npath + 1)));
         k_cav_check<<<g, kBlock, 0, cx.st>>>(c, Q, cnt + C_NQ, ncross.p, paths.p, ppos.p, ep, Q2, cnt + C_NQ2, wins.p,
                                              cnt + C_NWIN, scr.p, cnt + C_SCR, (long long)scr.n);
         GCDT_LAUNCH_CHECK();

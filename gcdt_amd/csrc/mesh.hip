@@ -70,7 +70,7 @@ void Arena::require(size_t bytes) const
 
 void* Arena::take(size_t bytes)
 {
-    size_t len = (bytes + 255) & ~(size_t)255;
+    const size_t len = size(bytes);
     require(top + len);
     void* p = base + top;
     top += len;
@@ -80,7 +80,7 @@ void* Arena::take(size_t bytes)
 
 void Arena::give(void* p, size_t bytes)
 {
-    size_t off = (size_t)((char*)p - base), end = off + ((bytes + 255) & ~(size_t)255);
+    size_t off = (size_t)((char*)p - base), end = off + size(bytes);
     if (end != top) {
         if (nfreed < kFreed) {
             freed_off[nfreed] = off;
@@ -101,6 +101,11 @@ void Arena::give(void* p, size_t bytes)
                 break;
             }
     }
+}
+
+void hold_to(DBuf<int>& pad, size_t top)
+{
+    if (g_arena && g_arena->top < top) pad.alloc((top - g_arena->top) / sizeof(int));
 }
 
 void* dev_take(size_t bytes)
@@ -3621,6 +3626,48 @@ static void build_bitmap_g(Ctx& c, const G& g, long long ncells, const int2* pts
 void build_bitmap(Ctx& c, const int2* pts, const int3* tri, int T, int** offsets, int** tris, int* ntris)
 {
     build_bitmap_g(c, GridOne{}, BITMAP_CELLS, pts, tri, T, offsets, tris, ntris);
+}
+
+template <class G>
+__global__ __launch_bounds__(kBlock) void k_bm_pairs(G, const int2* pts, const int3* tri, int T, unsigned long long* total)
+{
+    unsigned long long n = 0;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < T; i += (long long)gridDim.x * blockDim.x) {
+        const int3 t = tri[i];
+        int x0, y0, x1, y1;
+        tri_cells<G::LOG>(pts[t.x], pts[t.y], pts[t.z], x0, y0, x1, y1);
+        n += (unsigned long long)((x1 - x0 + 1) * (y1 - y0 + 1));
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) n += __shfl_down(n, d, 64);
+    if (__lane_id() == 0 && n) atomicAdd(total, n);
+}
+
+// By the buffers of build_bitmap: only where the triangles' cells fit and their
+// entries (no more than the pairs of triangle and cell) might not, the bitmap
+// itself tells.
+void require_bitmap(Ctx& c, const int2* pts, const int3* tri, int T, size_t top, size_t more)
+{
+    if (!g_arena) return;
+    static_assert(C_TOTAL % 2 == 0, "an aligned 64-bit word");
+    FillJobs f;
+    f.add(c.dcnt.p + C_TOTAL, 0, 2);
+    fill_jobs(c, f);
+    k_bm_pairs<GridOne><<<grid_for(T), kBlock, 0, c.st>>>(GridOne{}, pts, tri, T, (unsigned long long*)(c.dcnt.p + C_TOTAL));
+    GCDT_LAUNCH_CHECK();
+    c.read(C_TOTAL, 2);
+    const size_t npairs = ((size_t)(unsigned)c.hcnt[C_TOTAL + 1] << 32) | (unsigned)c.hcnt[C_TOTAL];
+    const size_t cells = top + Arena::size(sizeof(int) * ((size_t)T + 1)) + 2 * Arena::size(sizeof(int) * npairs) +
+                         Arena::size(sizeof(int) * (BITMAP_CELLS + 1));
+    g_arena->require(cells);
+    if (cells + Arena::size(sizeof(int) * npairs) + more <= g_arena->cap) return;
+    DBuf<int> pad;
+    hold_to(pad, top);
+    int *bo, *bt, nbt;
+    build_bitmap(c, pts, tri, T, &bo, &bt, &nbt);
+    g_arena->require(g_arena->top + more);
+    dev_give(bo, sizeof(int) * (BITMAP_CELLS + 1));
+    dev_give(bt, sizeof(int) * (size_t)(nbt > 0 ? nbt : 1));
 }
 
 // ================================================================== adjacency from a triangle list

@@ -41,6 +41,7 @@ struct Arena {
     void* take(size_t bytes);
     void give(void* p, size_t bytes);
     void require(size_t bytes) const;  // GCDT_ERR_SCRATCH unless the region holds as much
+    static size_t size(size_t bytes) { return (bytes + 255) & ~(size_t)255; }  // what a buffer takes of it
 };
 extern thread_local Arena* g_arena;
 
@@ -104,7 +105,7 @@ enum : int {
     C_NTRI = 2,    // insertion tail: triangles
     C_ERR = 4,
     C_NBIGW = 6,   // constraint rounds: winners above CAV_MID_K
-    C_TOTAL = 8,   // scan totals
+    C_TOTAL = 8,   // scan totals; with the next word, k_bm_pairs' 64-bit total
     C_NPIECE = 10,  // constraint rounds: triangles rewritten so far
     C_NQ = 11,
     C_NQ2 = 12,
@@ -374,6 +375,12 @@ int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int
 int filter_leaves_inst_rec(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl,
                            long long ncells, long long NP, const int3* tri, const int3* adj, const int* sons, int T,
                            FRec* rec, long long nleaf);
+// On a fixed array: pad takes the bytes in use up to `top`.  (Without one, or
+// with as many in use: nothing.)
+void hold_to(DBuf<int>& pad, size_t top);
+// On a fixed array: GCDT_ERR_SCRATCH unless a bitmap of these triangles and
+// `more` bytes fit above the first `top` bytes
+void require_bitmap(Ctx& c, const int2* pts, const int3* tri, int T, size_t top, size_t more);
 // bitmap CSR over 1024^2 cells; allocates offsets/tris from the pool
 void build_bitmap(Ctx& c, const int2* pts, const int3* tri, int T, int** offsets, int** tris, int* ntris);
 // mark vertices of tri[0..T) in isv (must be zeroed), then locate the other
