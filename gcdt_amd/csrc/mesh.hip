@@ -2813,7 +2813,10 @@ long long flip_driver(Ctx& c, E e, int T, const int* init, int ninit, int* round
         }
     };
     launch_rounds(c.tail_threshold, c.single_tester);
-    launch_rounds(FLIP_WG_LIST, 0);
+    if (!done) {
+        launch_rounds(FLIP_WG_LIST, 0);
+        if (done) r--;  // the round queued ahead had no input: the workgroup would not have run it
+    }
     // the last round's flips are settled by the tail: flipped triangles are in
     // the next list, so a round with flips is never the last
     if (E::kFused && r) prof_add_items("flip_test_fix", settled);
