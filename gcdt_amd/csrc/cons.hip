@@ -847,8 +847,8 @@ __global__ void k_cav_begin(int* cnt, int move)
 // about 190 each) is a long chain of dependent loads on a single thread.  When
 // the points are in Morton order of their 1024^2 cells (the single solve), the
 // vertices on a segment are found instead by testing the points of every cell
-// the segment touches, one (segment, cell) pair per thread; each segment's
-// vertices are then sorted along it in LDS, and each piece between two
+// the segment touches, a wave per segment; they are then sorted along it in
+// LDS, and each piece between two
 // consecutive ones is checked for being an existing edge on a thread of its
 // own.  The pieces are the same as the walk's: in order along the segment,
 // existing edges marked constrained and stored with a negative first vertex.

@@ -246,7 +246,7 @@ __host__ __device__ inline long long cav_block_ints(int K) { return 9LL * K + 16
 
 // owner[] of a triangle of such a cavity once it is rewritten: above every key
 // of a later round (keys fall with the epoch), the low word the place of one
-// of its boundary edges, for cav_fix_block.
+// of its boundary edges, for cav_new_owner.
 __host__ __device__ inline unsigned long long cav_place(int p) { return 0xFFFFFFFF00000000ull | (unsigned)p; }
 
 // The Delaunay vertex of base (A, B) among the polygon vertices lo..hi-1
@@ -271,11 +271,8 @@ struct DvScan {
 };
 
 // R3 body: collect winner wi's cavity and retriangulate it in place.
-// Returns false (and flags MERR_CAVITY) on an inconsistent cavity.  DV finds
-// each Delaunay vertex (DvScan, or a wave-wide search whose lanes all run this
-// body for the same cavity).  own: scratch of the caller's in place of
-// scr + w.off.
-template <class DV = DvScan>
+// Returns false (and flags MERR_CAVITY) on an inconsistent cavity.  own:
+// scratch of the caller's in place of scr + w.off.
 __host__ __device__ inline bool cav_retri_one(const Cons& c, const int2* pieces, const Win* wins, int wi, int* scr,
                                               unsigned epoch, int* own = nullptr)
 {
@@ -393,7 +390,7 @@ __host__ __device__ inline bool cav_retri_one(const Cons& c, const int2* pieces,
                 auto bnd_t = [&](int i) -> int { return side == 0 ? Lb[i] : Rb[M - i]; };
                 auto bnd_c = [&](int i) -> int { return side == 0 ? Lc[i] : Rc[M - i]; };
                 int A = poly(lo - 1), B = poly(hi);
-                const int ci = DV::find(PX, PY, lo, hi, make_int2(PX[lo - 1], PY[lo - 1]), make_int2(PX[hi], PY[hi]));
+                const int ci = DvScan::find(PX, PY, lo, hi, make_int2(PX[lo - 1], PY[lo - 1]), make_int2(PX[hi], PY[hi]));
                 int C = poly(ci);
                 int T = slots[e++];
                 int3 nt = make_int3(A, B, C);

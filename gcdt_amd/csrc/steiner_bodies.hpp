@@ -54,8 +54,6 @@ struct Stn {
     int* err;
 };
 
-__host__ __device__ inline HPt stn_pt(const Stn& s, int v) { return v < s.nv0 ? hpt_grid(s.pts[v]) : s.hp[v - s.nv0]; }
-
 __host__ __device__ inline DPt stn_dpt(const Stn& s, int v) { return v < s.nv0 ? dpt(s.pts[v]) : dpt(s.hp[v - s.nv0]); }
 
 // The exact determinants, out of line: inlined at every use they made the pass

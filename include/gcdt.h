@@ -173,6 +173,9 @@ int gcdt_add_constraints(void* tmp, size_t tmpBytes, const gcdt_int2* points, gc
 
 /* -------------------------------------------------------------- one call */
 
+/* ms_total is taken with events on the solve's stream.  The phases' times are
+ * the host's clock, each up to the counters that end the phase: they include
+ * waits for other work on the card, as when several streams share it. */
 typedef struct {
     double ms_total;       /* GPU time of the whole solve */
     double ms_sample;      /* sampling + sample mesh + sample flips */
@@ -211,11 +214,16 @@ int gcdt_solve_flags(const gcdt_int2* points, int N, const gcdt_int2* cons, int 
  * until the process ends; gcdt_pool_init() must have run once on the device
  * first (it looks up the array's device address and reserves pinned counter
  * pages), else GCDT_ERR_INVALID.  Arguments, outputs and status codes are
- * those of gcdt_solve.  The array holds about 40 MB plus 260 bytes per point,
- * plus about 48 bytes per triangle that a constraint segment crosses: inputs
- * above GCDT_NOALLOC_MAX_POINTS points or segments fail with
- * GCDT_ERR_SCRATCH at once, and an input whose constraints need more than the
- * array fails with GCDT_ERR_SCRATCH naming the bytes it needed.  All calls on
+ * those of gcdt_solve.  A solve counts about 38 MB and 324 bytes per point (24
+ * more without adj_out, 8 more where points lie on edges, as on a lattice, and
+ * about 110 more where they are packed into few of 1024 x 1024 cells) and 160
+ * per point of its sample, at most one in each of 256 x 256 cells; or, if that
+ * is more, 21 MB, 184 bytes per point and 56 per triangle that a constraint
+ * segment crosses.  Inputs above GCDT_NOALLOC_MAX_POINTS points or segments
+ * fail with GCDT_ERR_SCRATCH at once, and an input that counts more than the
+ * array fails with GCDT_ERR_SCRATCH naming the bytes.  So do a few hundred
+ * points on one line or circle, whose sample has triangles across much of the
+ * square, for the cells that these meet.  All calls on
  * a device share its array: they are serialised, each returning after its
  * stream has drained.  stats->ms_* come from the host clock. */
 #define GCDT_NOALLOC_SCRATCH_BYTES (256ull << 20)
@@ -275,7 +283,7 @@ int gcdt_check_mesh(const gcdt_int2* points, long long nv, const gcdt_int3* tris
 
 /* ------------------------------------------------------------ batches */
 
-typedef struct {
+typedef struct {           /* times as in gcdt_stats */
     double ms_total;
     double ms_insert;      /* location + insertion rounds of all instances */
     double ms_flip;
@@ -300,8 +308,8 @@ typedef struct {
  * N_i..N_i+3).  Every round of every phase runs for all instances at once,
  * so a batch costs about as many rounds as its largest instance.  Like
  * gcdt_solve, each instance first triangulates a sample (one point per cell
- * of its own 16x16 grid), makes it Delaunay and locates the other points
- * through a per-instance bitmap of it.  K <= 262144.
+ * of its own 16x16 grid), makes it Delaunay and locates the other points by
+ * walks on it.  K <= 262144.
  * inst_status (optional, HOST array of K ints): with it, an instance whose
  * own input makes the solve fail (bad ids or coordinates, duplicate points,
  * crossing constraints) fails alone: the batch is split in halves down to

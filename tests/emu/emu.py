@@ -31,7 +31,7 @@ LIB = os.path.join(HERE, "_build", "libgcdt_emu.so")
 # the per-cell reorder ranks buckets of up to 3 elements lane by lane, sorts
 # 4-8 in a workgroup and merge-sorts larger ones (the defaults are 256 and
 # 2048), and cavities of more than 4 crossed triangles are retriangulated by a
-# whole wave (the default is 64)
+# workgroup (the default is 12)
 CELLCAP = (("GCDT_CELL_RANK_MAX=3", "GCDT_CELL_BLOCK_MAX=8", "GCDT_CAV_WAVE_K=4"),
           os.path.join(HERE, "_build", "libgcdt_emu_cellcap.so"))
 _lib = None
