@@ -354,11 +354,10 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     int ntA = insert_rounds(c, ia, pend, pend2, S, 2, &rs);
     long long capB = 4LL * N + 8;
     DBuf<int3> tB(capB), aB(capB);
-    DBuf<FRec> recS(2LL * S + 2);  // stay for the location
-    int Ts = filter_leaves_morton_rec(c, pts, tA.p, aA.p, sA.p, ntA, recS.p, 2LL * S + 2);
+    DBuf<FRec> recS;  // stay for the location
+    int Ts = filter_leaves_morton_rec(c, pts, tA.p, aA.p, sA, ntA, recS, 2LL * S + 2);
     tA.release();
     aA.release();
-    sA.release();
     clA.release();
     validate_records(c, "the sample mesh's insertion", recS.p, Mesh{pts, tB.p, aB.p, nullptr, nullptr}, N + 4, Ts, false);
     int fr = 0;
@@ -398,12 +397,11 @@ void solve_impl(Ctx& c, const int2* pts_in, int N, const int2* cons_in, int C, i
     // leaves in Morton order, written straight into the packed flip records
     DBuf<int> held;
     hold_to(held, limit + Arena::size(sizeof(int) * (size_t)capB));
-    DBuf<FRec> rec(2LL * N + 2);
-    int T = filter_leaves_morton_rec(c, pts, tB.p, aB.p, sB.p, ntB, rec.p, 2LL * N + 2);
+    DBuf<FRec> rec;
+    int T = filter_leaves_morton_rec(c, pts, tB.p, aB.p, sB, ntB, rec, 2LL * N + 2);
     held.release();
     tB.release();
     aB.release();
-    sB.release();
     st.ms_insert = phase.lap();
     // ---- 4. Delaunay flips (unpacked into tris_out / adj_out)
     int f2 = 0;
@@ -909,14 +907,13 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     int ntA = insert_rounds(c, s, pend, pend2, S, 2 * K, &ri);
     long long capB = 2LL * K + 2LL * S + 4LL * (NP - S) + 8;
     if (capB > (1LL << 31) - 1) throw Error(GCDT_ERR_INVALID, "batch too large");
-    DBuf<int3> tB(capB), aB(capB);
-    DBuf<FRec> recS(2LL * S + 2LL * K);  // stay for the location
-    int Ts = filter_leaves_inst_rec(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, ncells, NP, tA.p, aA.p, sA.p, ntA, recS.p,
+    clA.release();
+    DBuf<FRec> recS;  // stay for the location
+    int Ts = filter_leaves_inst_rec(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, ncells, NP, tA.p, aA.p, sA, ntA, recS,
                                     2LL * S + 2LL * K);
     tA.release();
     aA.release();
-    sA.release();
-    clA.release();
+    DBuf<int3> tB(capB), aB(capB);  // after the samples' insertion is gone: a lower peak
     validate_records(c, "the sample meshes' insertion", recS.p, Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, nv, Ts, false);
     int fr = 0;
     bs.flips += flip_rounds_records(c, recS.p, Mesh{pts.p, tB.p, aB.p, nullptr, nullptr}, Ts, &fr);
@@ -948,12 +945,10 @@ void batch_impl(const gcdt_int2* points, const std::vector<long long>& poff, con
     pend.release();
     pend2.release();
     long long Tn = 2 * NP + 2LL * K;
-    DBuf<FRec> rec(Tn);
-    int T = filter_leaves_inst_rec(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, ncells, NP, tB.p, aB.p, sB.p, nt, rec.p,
-                                   Tn);
+    DBuf<FRec> rec;
+    int T = filter_leaves_inst_rec(c, pts.p, vinst.p, d_cbase.p, d_lvl.p, ncells, NP, tB.p, aB.p, sB, nt, rec, Tn);
     tB.release();
     aB.release();
-    sB.release();
     DBuf<int3> tri(Tn), adj(Tn);  // after the insertion DAG is gone: a lower peak
     bs.ms_insert = phase.lap();
     bs.insert_rounds = ri + ri2;

@@ -3418,18 +3418,22 @@ __global__ __launch_bounds__(kBlock) void k_leaf_move(const int3* tri, const int
     }
 }
 
-// CK: the order inside a cell
+// CK: the order inside a cell.  The records are allocated last, when what the
+// sort needs is gone: a batch of many small instances, nearly all of whose
+// points are in its samples, would peak here otherwise.  (A fixed array counts
+// them all.)
 template <class CK, class KEY>
 static int filter_leaves_sorted(Ctx& c, CK ck, const KEY& kf, long long ncells, const int2* pts, const int3* tri,
-                                const int3* adj, const int* sons, int T, FRec* rec, long long nleaf)
+                                const int3* adj, DBuf<int>& sons, int T, DBuf<FRec>& rec, long long nleaf)
 {
+    if (g_arena) rec.alloc((size_t)nleaf);
     DBuf<int> cnt((size_t)ncells + 1), cellof(T > 0 ? T : 1), dest(T > 0 ? T : 1);
     FillJobs f;
     f.add(cnt.p, 0, ncells + 1);
     f.add(c.dcnt.p + C_HUGE, 0, 1);
     f.add(c.dcnt.p + C_NQ, 0, 1);
     fill_jobs(c, f);
-    k_leaf_cells<KEY><<<grid_for(T), kBlock, 0, c.st>>>(kf, pts, tri, sons, T, cnt.p, cellof.p, dest.p,
+    k_leaf_cells<KEY><<<grid_for(T), kBlock, 0, c.st>>>(kf, pts, tri, sons.p, T, cnt.p, cellof.p, dest.p,
                                                         c.dcnt.p + C_HUGE);
     GCDT_LAUNCH_CHECK();
     scan_excl_total(c, cnt.p, cnt.p, ncells);
@@ -3440,9 +3444,10 @@ static int filter_leaves_sorted(Ctx& c, CK ck, const KEY& kf, long long ncells, 
     DBuf<int> src(n > 0 ? n : 1);
     {
         DBuf<int2> eb(n > 0 ? n : 1);
-        k_leaf_dest<<<grid_for(T), kBlock, 0, c.st>>>(sons, cellof.p, T, cnt.p, dest.p, eb.p, nleaf);
+        k_leaf_dest<<<grid_for(T), kBlock, 0, c.st>>>(sons.p, cellof.p, T, cnt.p, dest.p, eb.p, nleaf);
         GCDT_LAUNCH_CHECK();
         cellof.release();
+        sons.release();
         // each cell's leaves by their vertex ids (the count pass placed them
         // in arrival order); cnt holds the cells' starts, cnt[c + 1] their ends
         ck.tri = tri;
@@ -3450,16 +3455,18 @@ static int filter_leaves_sorted(Ctx& c, CK ck, const KEY& kf, long long ncells, 
         ck.dest = dest.p;
         cell_reorder(c, ck, cnt.p + 1, eb.p, n, large);
     }
+    cnt.release();
+    rec.ensure((size_t)nleaf);
     if (n > 0) {
         ProfScope ps("leaf_move", c.st, n);
-        k_leaf_move<<<grid_for(n), kBlock, 0, c.st>>>(tri, adj, dest.p, src.p, n, pts, rec);
+        k_leaf_move<<<grid_for(n), kBlock, 0, c.st>>>(tri, adj, dest.p, src.p, n, pts, rec.p);
         GCDT_LAUNCH_CHECK();
     }
     return n;
 }
 
-int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
-                             FRec* rec, long long nleaf)
+int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, DBuf<int>& sons, int T,
+                             DBuf<FRec>& rec, long long nleaf)
 {
     // on a fixed array, where the longer keys of a crowded coarse cell count, for
     // the smallest meshes only
@@ -3488,8 +3495,8 @@ struct LeafKeyInst {
 };
 
 int filter_leaves_inst_rec(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl,
-                           long long ncells, long long NP, const int3* tri, const int3* adj, const int* sons, int T,
-                           FRec* rec, long long nleaf)
+                           long long ncells, long long NP, const int3* tri, const int3* adj, DBuf<int>& sons, int T,
+                           DBuf<FRec>& rec, long long nleaf)
 {
     return filter_leaves_sorted(c, CellKeyTri{}, LeafKeyInst{vinst, cbase, lvl, NP}, ncells, pts, tri, adj, sons, T,
                                 rec, nleaf);

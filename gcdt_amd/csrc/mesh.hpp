@@ -369,12 +369,13 @@ int filter_leaves(Ctx& c, const int3* tri, const int3* adj, const int* sons, int
 // same into packed flip records, the leaves placed in Morton order of their
 // centroid cell (batch meshes: by instance, then centroid cell in the
 // instance's grid of 4^L cells: cbase/lvl/ncells as for the batched point
-// order); GCDT_ERR_INTERNAL unless the mesh has nleaf leaves
-int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, const int* sons, int T,
-                             FRec* rec, long long nleaf);
+// order); GCDT_ERR_INTERNAL unless the mesh has nleaf leaves.
+// sons is released when it has been read, rec allocated.
+int filter_leaves_morton_rec(Ctx& c, const int2* pts, const int3* tri, const int3* adj, DBuf<int>& sons, int T,
+                             DBuf<FRec>& rec, long long nleaf);
 int filter_leaves_inst_rec(Ctx& c, const int2* pts, const int* vinst, const int* cbase, const int* lvl,
-                           long long ncells, long long NP, const int3* tri, const int3* adj, const int* sons, int T,
-                           FRec* rec, long long nleaf);
+                           long long ncells, long long NP, const int3* tri, const int3* adj, DBuf<int>& sons, int T,
+                           DBuf<FRec>& rec, long long nleaf);
 // On a fixed array: pad takes the bytes in use up to `top`.  (Without one, or
 // with as many in use: nothing.)
 void hold_to(DBuf<int>& pad, size_t top);
