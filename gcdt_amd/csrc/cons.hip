@@ -87,6 +87,17 @@ __device__ inline unsigned cell_morton(unsigned x, unsigned y)
     return x | (y << 1);
 }
 
+// wave_alloc on a 64-bit counter: the triangles that all pieces cross may be
+// more than an int counts
+__device__ inline long long wave_alloc_64(int k, unsigned long long* counter)
+{
+    int total;
+    const int ex = wave_excl_scan(k, total);
+    unsigned long long base = 0;
+    if (__lane_id() == 0 && total > 0) base = atomicAdd(counter, (unsigned long long)total);
+    return (long long)__shfl(base, 0, 64) + ex;
+}
+
 // R1: claim crossed triangles; pieces that became edges are retired.  One
 // thread per piece: a walk that collects the crossed triangles in LDS, then
 // the claims and the path for the later steps (paths[] at ppos[i], room
@@ -94,8 +105,8 @@ __device__ inline unsigned cell_morton(unsigned x, unsigned y)
 // larger buffer).  A piece that crosses more than CAV_WAVE_K triangles goes
 // to the long list.
 __global__ __launch_bounds__(kBlock) void k_cav_claim(Cons c, const int2* pieces, const int* q, const int* nq,
-                                                      unsigned epoch, int* ncross, int* paths, int pcap, int* pcur,
-                                                      int* ppos, int* longq, int* nlong)
+                                                      unsigned epoch, int* ncross, int* paths, int pcap,
+                                                      unsigned long long* pcur, int* ppos, int* longq, int* nlong)
 {
     constexpr int KEEP = CAV_WAVE_K | 1;  // odd stride: no bank conflicts
     __shared__ int s_keep[kBlock * KEEP];
@@ -120,9 +131,9 @@ __global__ __launch_bounds__(kBlock) void k_cav_claim(Cons c, const int2* pieces
             const unsigned long long key = cav_key(epoch, pi);
             for (int j = 0; j < k; j++) atomicMin(&c.owner[mine[j]], key);
         }
-        const int off = wave_alloc(k, pcur);
-        if (k > 0) ppos[i] = off;
-        if (k > 0 && off >= 0 && k <= pcap - off)
+        const long long off = wave_alloc_64(k, pcur);
+        if (k > 0) ppos[i] = (int)off;
+        if (k > 0 && off + k <= pcap)
             for (int j = 0; j < k; j++) paths[off + j] = mine[j];
         const int l = wave_alloc(lng ? 1 : 0, nlong);
         if (lng) longq[l] = (int)i;
@@ -186,8 +197,8 @@ constexpr int WALK_KEEP = 32;  // triangles of a part kept in LDS (longer parts 
 
 __global__ __launch_bounds__(64) void k_cav_walk_long(Cons c, const int2* pieces, const int* q, const int* longq,
                                                       const int* nlong, const int* cell_end, unsigned epoch,
-                                                      int* ncross, int* total, int* paths, int pcap, int* pcur,
-                                                      int* ppos)
+                                                      int* ncross, int* total, int* paths, int pcap,
+                                                      unsigned long long* pcur, int* ppos)
 {
     __shared__ int s_tag[WALK_HASH], s_lane[WALK_HASH];
     __shared__ int s_next[64], s_sum[64], s_st[64], s_on[64];
@@ -313,11 +324,11 @@ __global__ __launch_bounds__(64) void k_cav_walk_long(Cons c, const int2* pieces
             if (bad) {
                 ncross[i] = 0;
             } else {
-                const int off = atomicAdd(pcur, K);
+                const long long off = (long long)atomicAdd(pcur, (unsigned long long)K);
                 ncross[i] = K;
-                ppos[i] = off;
+                ppos[i] = (int)off;
                 atomicAdd(total, K);
-                if (off >= 0 && K <= pcap - off) s_off = off;
+                if (off + K <= pcap) s_off = (int)off;
             }
         }
         __syncthreads();
@@ -836,6 +847,7 @@ __global__ void k_cav_begin(int* cnt, int move)
     cnt[C_TOTAL] = 0;
     cnt[C_NLONG] = 0;
     cnt[C_PATH] = 0;
+    cnt[C_PATH + 1] = 0;
     cnt[C_NMID] = 0;
     cnt[C_NBIGW] = 0;
 }
@@ -1130,7 +1142,7 @@ static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const
     }
     DBuf<int> np((size_t)C + 1), hcnt(C), hpos(C), wlist(C), hits((size_t)2 * C + 1024);
     for (int tries = 0;; tries++) {
-        const int hcap = (int)std::min<size_t>(hits.n, 1u << 30);
+        const int hcap = (int)std::min<size_t>(hits.n, INT_MAX);
         k_seg_find<<<std::min(C, 16384), 64, 0, cx.st>>>(pts, cell_end, cons, C, nmax, np.p, hcnt.p, hpos.p, hits.p, hcap,
                                                          cnt + C_NREW, wlist.p, cnt + C_NQ2, c.err);
         GCDT_LAUNCH_CHECK();
@@ -1138,7 +1150,7 @@ static int split_pieces_cells(Ctx& cx, const Cons& c, const int* cell_end, const
         cx.read(0, C_NUM);
         if (cx.hcnt[C_ERR]) cx.check_err();
         const long long nh = cx.hcnt[C_NREW];
-        if (nh < 0 || nh > (1LL << 30)) throw Error(GCDT_ERR_SCRATCH, "too many vertices on the constraints");
+        if (nh < 0) throw Error(GCDT_ERR_SCRATCH, "too many vertices on the constraints");
         if (nh <= (long long)hits.n) break;
         if (tries) throw Error(GCDT_ERR_INTERNAL, "constraint split changed between two passes");
         hits.ensure((size_t)nh);
@@ -1281,22 +1293,22 @@ ConsResult insert_constraints(Ctx& cx, const Mesh& m, int T, int nv, int nmax, c
         const int g = grid_for(nq);
         long long npath = 0;
         for (int tries = 0;; tries++) {
-            const int pcap = (int)std::min<size_t>(paths.n, 1u << 30);
+            const int pcap = (int)std::min<size_t>(paths.n, INT_MAX);
+            unsigned long long* pcur = (unsigned long long*)(cnt + C_PATH);
             k_cav_begin<<<1, 1, 0, cx.st>>>(cnt, r > 1 && tries == 0);
             GCDT_LAUNCH_CHECK();
-            k_cav_claim<<<g, kBlock, 0, cx.st>>>(c, pieces.p, Q, cnt + C_NQ, ep, ncross.p, paths.p, pcap, cnt + C_PATH,
-                                                 ppos.p, longq.p, cnt + C_NLONG);
+            k_cav_claim<<<g, kBlock, 0, cx.st>>>(c, pieces.p, Q, cnt + C_NQ, ep, ncross.p, paths.p, pcap, pcur, ppos.p,
+                                                 longq.p, cnt + C_NLONG);
             GCDT_LAUNCH_CHECK();
             k_cav_walk_long<<<std::min(nq, 2048), 64, 0, cx.st>>>(c, pieces.p, Q, longq.p, cnt + C_NLONG, cell_end, ep,
-                                                                  ncross.p, cnt + C_TOTAL, paths.p, pcap, cnt + C_PATH,
-                                                                  ppos.p);
+                                                                  ncross.p, cnt + C_TOTAL, paths.p, pcap, pcur, ppos.p);
             GCDT_LAUNCH_CHECK();
             cx.read(0, C_NUM);
             if (cx.hcnt[C_ERR]) cx.check_err();
             if (r > 1 && cx.hcnt[C_STUCK]) throw Error(GCDT_ERR_INTERNAL, "constraint round without progress");
             nq = cx.hcnt[C_NQ];
-            npath = cx.hcnt[C_PATH];
-            if (npath < 0 || npath > (1LL << 30)) throw Error(GCDT_ERR_SCRATCH, "constraints cross too many triangles");
+            npath = ((long long)cx.hcnt[C_PATH + 1] << 32) | (unsigned)cx.hcnt[C_PATH];
+            if (npath > INT_MAX) throw Error(GCDT_ERR_SCRATCH, "constraints cross too many triangles");
             if (npath <= (long long)paths.n) break;
             // the paths did not fit: a larger buffer, and the walks again (their
             // claims are the same)

@@ -117,13 +117,13 @@ enum : int {
     C_TAIL_ERR = 18,  // 1 = a round without progress
     C_TAIL_F = 20,    // flips done
     C_TAIL_P = 21,    // proposals of the launched round before the tail
+    C_PATH = 22,      // constraint rounds: crossed triangles, 64 bits
     C_STN_T = 24,     // crossing pass: triangles in use
     C_STN_S = 25,     // crossing pass: crossing vertices
     C_HUGE = 26,      // count passes: CELL_LARGE / CELL_HUGE (mesh.hip)
     C_VAL = 27,       // mesh check: failed checks (VAL_* bits)
     C_VAL_FIRST = 28, // mesh check: first failing triangle
     C_NLONG = 29,  // constraint rounds: pieces that cross many triangles
-    C_PATH = 30,   // constraint rounds: their crossed triangles
     C_NMID = 31,   // constraint rounds: the other long winners
     C_NUM = 32
 };
