@@ -1,23 +1,18 @@
 """Rounds with many long pieces: the smaller cavities by a wave each and the
 larger ones by a workgroup, or all of them by workgroups, as the pieces' number
 and average length say.  Every choice must give the same arrays."""
-import os
-
 import numpy as np
 import pytest
 
 from tests.emu import emu
+from tests.test_crowded_cells import TINY
 from tests.test_long_segments import check, emulated, segments
-
-# any number of long pieces is many: averages of up to 24 triangles are split
-BOTH = (("GCDT_CAV_WAVE_K=4", "GCDT_CAV_MID_K=24", "GCDT_CAV_LDS_K=30", "GCDT_CAV_FEW=0"),
-        os.path.join(os.path.dirname(emu.LIB), "libgcdt_emu_cavboth.so"))
 
 
 @pytest.mark.parametrize("case", [("rows", 300, 8), ("columns", 400, 8), ("steep", 500, 9), ("rows", 2000, 12)],
                          ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}")
 def test_both_sizes_give_the_default_arrays(case):
-    default, both = emu.build(), emu.build(BOTH)
+    default, both = emu.build(), emu.build(TINY)
     g, cons = segments(*case)
     tris, adj = emulated(default, case, 1)
     check(g, cons, tris)

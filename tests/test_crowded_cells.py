@@ -14,8 +14,12 @@ from tests.emu import emu
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 # a cell of more than two elements is sorted by a workgroup, of more than four
-# by the merge of all such cells
-TINY = (("GCDT_CELL_RANK_MAX=2", "GCDT_CELL_BLOCK_MAX=4"),
+# by the merge of all such cells; any number of long pieces is many, and those of
+# up to 24 triangles on average get a wave or a workgroup by their own size
+# (test_cavity_sizes.py); all flip rounds below the tail threshold run in one
+# workgroup (test_round_counts.py)
+TINY = (("GCDT_CELL_RANK_MAX=2", "GCDT_CELL_BLOCK_MAX=4", "GCDT_CAV_WAVE_K=4", "GCDT_CAV_MID_K=24", "GCDT_CAV_LDS_K=30",
+         "GCDT_CAV_FEW=0", "GCDT_FLIP_WG_LIST=4096"),
         os.path.join(os.path.dirname(emu.LIB), "libgcdt_emu_tinycap.so"))
 NONE = np.zeros((0, 2), np.int32)
 
@@ -40,8 +44,7 @@ def pieces(cells, each, seed=4):
 
 
 CASES = {
-    "points_2116": lambda: pieces(46, 6),    # cells of six points: 2,116 and 4,096 of them
-    "points_4096": lambda: pieces(64, 6),
+    "points": lambda: pieces(64, 6),          # 4,096 cells of six points
     "leaves": lambda: packed(30_000, 0.354),  # about 8,200 of 65,536 leaf cells hold 60,002 leaves
 }
 

@@ -7,10 +7,8 @@ import sys
 import pytest
 
 from tests.emu import emu
+from tests.test_crowded_cells import TINY
 from tests.test_round_routes import ROOT, SMALL
-
-# all rounds below the tail threshold in one workgroup
-WHOLE = (("GCDT_FLIP_WG_LIST=4096",), os.path.join(os.path.dirname(emu.LIB), "libgcdt_emu_wholetail.so"))
 
 
 def counts(lib, case, seed):
@@ -25,6 +23,6 @@ def counts(lib, case, seed):
 
 @pytest.mark.parametrize("case", [("rows", 3000, 25), ("columns", 1200, 10), ("steep", 5000, 40)], ids=lambda c: c[0])
 def test_counts_do_not_depend_on_the_route(case):
-    whole = counts(emu.build(WHOLE), case, 1)
+    whole = counts(emu.build(TINY), case, 1)
     assert counts(emu.build(), case, 2) == whole
     assert counts(emu.build(SMALL), case, 3) == whole
